@@ -38,6 +38,9 @@
 #include "ad_kernel.hpp"
 #include "gen/coef_mbpol_2b.inc"
 #include "gen/coef_mbpol_3b.inc"
+#define MBXG_SYM_SPACE static __device__
+#include "gen/sym_mbpol_2b.inc"
+#include "gen/sym_mbpol_3b.inc"
 #include "mbxg.h"
 #include "mbxg_device.hpp"
 #include "mbxg_kernels.hpp"
@@ -66,6 +69,24 @@ struct AdVar {
 
 constexpr int kNTheta = 10;
 
+// Slot q of the symmetry-adapted polynomial's coefficients (gen/sym_<name>.inc): the products with
+// the weights are exact, the sum is carried with its rounding errors, so slots at or past nrow get
+// what rounding left of slot low[q - nrow].
+__device__ __forceinline__ double ad_slot(const int* row, const unsigned short* k, const double* w,
+                                          const unsigned short* low, int nrow, int q,
+                                          const double* __restrict__ coef) {
+    const int r = q < nrow ? q : low[q - nrow];
+    double s = 0.0, err = 0.0;
+    for (int i = row[r]; i < row[r + 1]; ++i) {
+        const double p = coef[k[i]] * w[i];
+        const double t = s + p, z = t - s;
+        err += (s - (t - z)) + (p - z);
+        s = t;
+    }
+    const double b = s + err;
+    return q < nrow ? b : err - (b - s);
+}
+
 // Sites 0..5 = Oa Ha1 Ha2 Ob Hb1 Hb2, 6..9 = Xa1 Xa2 Xb1 Xb2 (x2b-v9x.cpp:1640-1675).
 struct Ad2b {
     static constexpr int kNV = 31, kNAt = 6, kNS = 10, kPairs = 1, kParts = kAdParts;
@@ -81,6 +102,10 @@ struct Ad2b {
         {0, 6, -1, 4.0, 0, 9}, {0, 6, -1, 4.0, 3, 6}, {0, 6, -1, 4.0, 3, 7}, {0, 7, -1, 4.0, 6, 8},
         {0, 7, -1, 4.0, 6, 9}, {0, 7, -1, 4.0, 7, 8}, {0, 7, -1, 4.0, 7, 9}};
     static constexpr int kPairA[3] = {0, 0, 0}, kPairB[3] = {3, 0, 0};
+    static constexpr int kNSlot = kNSlot_mbpol_2b;
+    static __device__ __forceinline__ double slot(int q, const double* __restrict__ coef) {
+        return ad_slot(kSymRow_mbpol_2b, kSymK_mbpol_2b, kSymW_mbpol_2b, kSymLow_mbpol_2b, kNRow_mbpol_2b, q, coef);
+    }
 };
 
 // Sites 0..8 = Oa Ha1 Ha2 Ob Hb1 Hb2 Oc Hc1 Hc2 (x3b-v2x.cpp:1548-1584); parameter set s uses
@@ -100,6 +125,10 @@ struct Ad3b {
         {2, 4, 9, 0, 3, 6}};
     // O-O pairs ab, ac, bc; the switch is s_ab s_ac + s_ab s_bc + s_ac s_bc (x3b-v2x.cpp:1614-1620)
     static constexpr int kPairA[3] = {0, 0, 3}, kPairB[3] = {3, 6, 6};
+    static constexpr int kNSlot = kNSlot_mbpol_3b;
+    static __device__ __forceinline__ double slot(int q, const double* __restrict__ coef) {
+        return ad_slot(kSymRow_mbpol_3b, kSymK_mbpol_3b, kSymW_mbpol_3b, kSymLow_mbpol_3b, kNRow_mbpol_3b, q, coef);
+    }
 };
 
 // f_switch (x2b-v9x.cpp:1349-1362, x3b-v2x.cpp:1275-1288) with its first and second derivatives.
@@ -254,13 +283,22 @@ __device__ __forceinline__ void ad_total_switch(const double* sv, const double* 
 }  // namespace
 
 // Stage 1: variables (and tangents) and the switch (and tangent).  Without TAN the tangent
-// outputs, when given, are written as zeros.
+// outputs, when given, are written as zeros.  The blocks past the n-mers' fill what the polynomial
+// kernels read: the adapted coefficients slots[kNSlot] and the n-mer count ndev.
 template <class F, bool TAN>
 __global__ void __launch_bounds__(64) k_ad_vars(const double* __restrict__ xyz, const double* __restrict__ u,
                                                 const double* __restrict__ theta, int n, int ld,
-                                                double* __restrict__ xs, double* __restrict__ xds,
-                                                double* __restrict__ sw_out, double* __restrict__ swd_out) {
+                                                const double* __restrict__ coef, double* __restrict__ xs,
+                                                double* __restrict__ xds, double* __restrict__ sw_out,
+                                                double* __restrict__ swd_out, double* __restrict__ slots,
+                                                int* __restrict__ ndev) {
     const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= ld) {
+        const int q = t - ld;
+        if (q < F::kNSlot) slots[q] = F::slot(q, coef);
+        if (q == 0) *ndev = n;
+        return;
+    }
     if (t >= n) return;
     double th[kNTheta];
 #pragma unroll
@@ -506,8 +544,6 @@ __global__ void __launch_bounds__(256) k_ad_sum_parts(double* __restrict__ gds, 
     gds[e] = s;
 }
 
-__global__ void k_ad_set_int(int* p, int v) { *p = v; }
-
 }  // namespace mbxg
 
 using namespace mbxg;
@@ -515,11 +551,13 @@ using namespace mbxg;
 namespace {
 
 struct AdLayout {
-    size_t xs, xds, sw, swd, gs, gds, ps, ndev, basis, theta, total;
+    size_t xs, xds, sw, swd, gs, gds, ps, ndev, slots, basis, theta, total;
 };
 
 constexpr size_t kAlign = 256;
 size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
+
+constexpr int kMaxSlots = kNSlot_mbpol_2b > kNSlot_mbpol_3b ? kNSlot_mbpol_2b : kNSlot_mbpol_3b;
 
 bool ad_shape(int family, int& nv, int& nat, int& ncoef) {
     if (family == MBXG_AD_MBPOL_2B) {
@@ -556,6 +594,7 @@ AdLayout ad_layout(int nv, int ncoef, int n) {
     L.gds = take(sizeof(double) * parts * nv * ld);
     L.ps = take(sizeof(double) * ld);
     L.ndev = take(sizeof(int));
+    L.slots = take(sizeof(double) * kMaxSlots);
     L.basis = take(sizeof(double) * nblk * ncoef);
     L.theta = take(sizeof(double) * nblk * 16);
     L.total = o;
@@ -629,22 +668,28 @@ extern "C" size_t mbxg_ad_workspace_bytes(int family, int n) {
 
 namespace {
 
-// The forward stages over stage buffers xs (nv x ld), sw (ld), gs (nv x ld), ps (ld) and the
+// Blocks of k_ad_vars: the n-mers, then the coefficient slots.
+template <class F>
+dim3 vars_grid(int nb) {
+    return dim3(nb + (F::kNSlot + 63) / 64);
+}
+
+// The forward stages over stage buffers xs (nv x ld), sw (ld), gs (nv x ld), ps (ld), slots and the
 // device n-mer count ndev, wherever they live (a caller's workspace or the library's scratch).
 int ad_forward_run(int family, int n, const double* xyz, const double* coef, const double* theta, double* energy,
-                   double* grad, double* xs, double* sw, double* gs, double* ps, int* ndev, hipStream_t st) {
+                   double* grad, double* xs, double* sw, double* gs, double* ps, int* ndev, double* slots,
+                   hipStream_t st) {
     const int ld = (n + 63) / 64 * 64, nb = ld / 64;
-    hipLaunchKernelGGL(k_ad_set_int, dim3(1), dim3(1), 0, st, ndev, n);
     if (family == MBXG_AD_MBPOL_2B) {
-        hipLaunchKernelGGL((k_ad_vars<Ad2b, false>), dim3(nb), dim3(64), 0, st, xyz, nullptr, theta, n, ld, xs,
-                           nullptr, sw, nullptr);
-        ADCHK(launch_poly_mbpol2b(xs, ndev, n, ld, coef, 1, gs, ps, 8, st));
+        hipLaunchKernelGGL((k_ad_vars<Ad2b, false>), vars_grid<Ad2b>(nb), dim3(64), 0, st, xyz, nullptr, theta, n, ld, coef,
+                           xs, nullptr, sw, nullptr, slots, ndev);
+        ADCHK(launch_poly_mbpol2b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
         hipLaunchKernelGGL((k_ad_chain<Ad2b, false>), dim3(nb), dim3(64), 0, st, xyz, nullptr, theta, nullptr, n, ld,
                            1, gs, nullptr, ps, nullptr, energy, grad, nullptr);
     } else {
-        hipLaunchKernelGGL((k_ad_vars<Ad3b, false>), dim3(nb), dim3(64), 0, st, xyz, nullptr, theta, n, ld, xs,
-                           nullptr, sw, nullptr);
-        ADCHK(launch_poly_mbpol3b(xs, ndev, n, ld, coef, 1, gs, ps, 8, st));
+        hipLaunchKernelGGL((k_ad_vars<Ad3b, false>), vars_grid<Ad3b>(nb), dim3(64), 0, st, xyz, nullptr, theta, n, ld, coef,
+                           xs, nullptr, sw, nullptr, slots, ndev);
+        ADCHK(launch_poly_mbpol3b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
         hipLaunchKernelGGL((k_ad_chain<Ad3b, false>), dim3(nb), dim3(64), 0, st, xyz, nullptr, theta, nullptr, n, ld,
                            1, gs, nullptr, ps, nullptr, energy, grad, nullptr);
     }
@@ -660,11 +705,12 @@ int ad_forward_run(int family, int n, const double* xyz, const double* coef, con
 // device (the array's name in host code is not a device address).
 constexpr int kNoAllocMaxNmers = 8192;
 constexpr size_t fwd_bytes(int nv, int n) {
-    // xs, sw, gs, ps and the count, each rounded up to kAlign bytes
+    // xs, sw, gs, ps, the count and the coefficient slots, each rounded up to kAlign bytes
     return ((sizeof(double) * nv * n + kAlign - 1) / kAlign * kAlign) * 2 +
-           ((sizeof(double) * n + kAlign - 1) / kAlign * kAlign) * 2 + kAlign;
+           ((sizeof(double) * n + kAlign - 1) / kAlign * kAlign) * 2 + kAlign +
+           (sizeof(double) * kMaxSlots + kAlign - 1) / kAlign * kAlign;
 }
-constexpr size_t kScratchBytes = fwd_bytes(36, kNoAllocMaxNmers);  // 4,849,920 bytes
+constexpr size_t kScratchBytes = fwd_bytes(36, kNoAllocMaxNmers);  // 4.6 MiB
 static_assert(fwd_bytes(31, kNoAllocMaxNmers) <= kScratchBytes, "the 2B forward fits the 3B scratch");
 
 }  // namespace
@@ -706,7 +752,8 @@ extern "C" int mbxg_ad_forward(int family, int n, const double* xyz, const doubl
     if (!xyz || !coef || !theta || !energy || !grad) return ad_err(MBXG_EINVAL, "mbxg_ad_forward: null pointer");
     char* w = (char*)workspace;
     return ad_forward_run(family, n, xyz, coef, theta, energy, grad, (double*)(w + L.xs), (double*)(w + L.sw),
-                          (double*)(w + L.gs), (double*)(w + L.ps), (int*)(w + L.ndev), (hipStream_t)stream);
+                          (double*)(w + L.gs), (double*)(w + L.ps), (int*)(w + L.ndev), (double*)(w + L.slots),
+                          (hipStream_t)stream);
 }
 
 extern "C" int mbxg_ad_forward_noalloc(int family, int n, const double* xyz, const double* coef,
@@ -722,7 +769,7 @@ extern "C" int mbxg_ad_forward_noalloc(int family, int n, const double* xyz, con
     void* base = nullptr;
     if (int e = scratch_on_current_device(&base)) return e;
     // the forward layout for this n inside the scratch; every stage writes its buffer before
-    // reading it (the count by k_ad_set_int), so nothing needs clearing between calls
+    // reading it (the count and the slots by k_ad_vars), so nothing needs clearing between calls
     const size_t ld = (size_t)(n + 63) / 64 * 64;
     char* w = (char*)base;
     size_t o = 0;
@@ -736,8 +783,9 @@ extern "C" int mbxg_ad_forward_noalloc(int family, int n, const double* xyz, con
     double* sw = (double*)take(sizeof(double) * ld);
     double* ps = (double*)take(sizeof(double) * ld);
     int* ndev = (int*)take(sizeof(int));
+    double* slots = (double*)take(sizeof(double) * kMaxSlots);
     if (o > kScratchBytes) return ad_err(MBXG_EINVAL, "mbxg_ad_forward_noalloc: layout exceeds the scratch");
-    return ad_forward_run(family, n, xyz, coef, theta, energy, grad, xs, sw, gs, ps, ndev, (hipStream_t)stream);
+    return ad_forward_run(family, n, xyz, coef, theta, energy, grad, xs, sw, gs, ps, ndev, slots, (hipStream_t)stream);
 }
 
 extern "C" int mbxg_ad_backward(int family, int n, const double* xyz, const double* coef, const double* theta,
@@ -765,25 +813,25 @@ extern "C" int mbxg_ad_backward(int family, int n, const double* xyz, const doub
     double* gds = (double*)(w + L.gds);
     double* ps = (double*)(w + L.ps);
     int* ndev = (int*)(w + L.ndev);
+    double* slots = (double*)(w + L.slots);
     double* basis = (double*)(w + L.basis);
     double* thp = (double*)(w + L.theta);
     const int ld = (n + 63) / 64 * 64, nb = ld / 64;
     // a null g_grad is the zero direction (an energy-only loss)
     const size_t rows = (size_t)nv * ld;
-    hipLaunchKernelGGL(k_ad_set_int, dim3(1), dim3(1), 0, st, ndev, n);
     if (family == MBXG_AD_MBPOL_2B) {
-        hipLaunchKernelGGL((k_ad_vars<Ad2b, true>), dim3(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, xs, xds, sw,
-                           swd);
-        if (!from_forward) ADCHK(launch_poly_mbpol2b(xs, ndev, n, ld, coef, 1, gs, ps, 8, st));
+        hipLaunchKernelGGL((k_ad_vars<Ad2b, true>), vars_grid<Ad2b>(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, coef, xs,
+                           xds, sw, swd, slots, ndev);
+        if (!from_forward) ADCHK(launch_poly_mbpol2b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
         ADCHK(launch_ad_tan_mbpol_2b(xs, xds, n, ld, coef, gds, st));
         ADCHK(launch_ad_basis_mbpol_2b(xs, xds, sw, swd, g_energy, n, ld, basis, st));
         hipLaunchKernelGGL(k_ad_sum_parts, dim3((rows + 255) / 256), dim3(256), 0, st, gds, rows, Ad2b::kParts);
         hipLaunchKernelGGL((k_ad_chain<Ad2b, true>), dim3(nb), dim3(64), 0, st, xyz, g_grad, theta, g_energy, n, ld, 1,
                            gs, gds, ps, xds, nullptr, d_xyz, thp);
     } else {
-        hipLaunchKernelGGL((k_ad_vars<Ad3b, true>), dim3(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, xs, xds, sw,
-                           swd);
-        if (!from_forward) ADCHK(launch_poly_mbpol3b(xs, ndev, n, ld, coef, 1, gs, ps, 8, st));
+        hipLaunchKernelGGL((k_ad_vars<Ad3b, true>), vars_grid<Ad3b>(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, coef, xs,
+                           xds, sw, swd, slots, ndev);
+        if (!from_forward) ADCHK(launch_poly_mbpol3b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
         ADCHK(launch_ad_tan_mbpol_3b(xs, xds, n, ld, coef, gds, st));
         ADCHK(launch_ad_basis_mbpol_3b(xs, xds, sw, swd, g_energy, n, ld, basis, st));
         hipLaunchKernelGGL(k_ad_sum_parts, dim3((rows + 255) / 256), dim3(256), 0, st, gds, rows, Ad3b::kParts);

@@ -37,6 +37,10 @@
 #include "gen/coef_ch4h2o_2b.inc"
 #include "gen/coef_mbpol_2b.inc"
 #include "gen/coef_mbpol_3b.inc"
+#define MBXG_SYM_SPACE static
+#include "gen/sym_ch4h2o2_3b.inc"
+#include "gen/sym_mbpol_2b.inc"
+#include "gen/sym_mbpol_3b.inc"
 #include "mbxg_kernels.hpp"
 #include "xfam.hpp"
 
@@ -66,6 +70,34 @@ int fail(int code, const char* fmt, ...) {
         if (e_ != hipSuccess) return fail(MBXG_EHIP, "%s: %s (%s:%d)", #expr, hipGetErrorString(e_), \
                                           __FILE__, __LINE__);                                      \
     } while (0)
+
+// The coefficients a kernel reads, from the fitted (or caller's) ones a: the polynomials in
+// symmetry-adapted coordinates take b = T a (gen/sym_<name>.inc), summed in extended precision and
+// rounded once, then the rests of the slots in `low`; the others take a itself.
+struct SymTable {
+    const int* row;
+    const unsigned short* k;
+    const double* w;
+    const unsigned short* low;
+    int nrow, nlow;
+};
+
+std::vector<double> kernel_coefficients(const SymTable* t, const double* a, int n) {
+    if (!t) return std::vector<double>(a, a + n);
+    std::vector<double> b(t->nrow + t->nlow);
+    auto sum = [&](int q) {
+        long double v = 0.0L;
+        for (int i = t->row[q]; i < t->row[q + 1]; ++i) v += (long double)a[t->k[i]] * t->w[i];
+        return v;
+    };
+    for (int q = 0; q < t->nrow; ++q) b[q] = (double)sum(q);
+    for (int j = 0; j < t->nlow; ++j) b[t->nrow + j] = (double)(sum(t->low[j]) - (long double)b[t->low[j]]);
+    return b;
+}
+
+#define MBXG_SYM(name) {kSymRow_##name, kSymK_##name, kSymW_##name, kSymLow_##name, kNRow_##name, kNLow_##name}
+const SymTable kSymMbpol2b = MBXG_SYM(mbpol_2b), kSymMbpol3b = MBXG_SYM(mbpol_3b), kSymCh4h2o2 = MBXG_SYM(ch4h2o2_3b);
+#undef MBXG_SYM
 
 template <class T>
 struct DBuf {
@@ -241,16 +273,20 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
         xfam_default_coef(f, &nx);
         xbad = xbad || c->d_xcoef[f].reserve(nx);
     }
-    if (xbad || c->d_xfam_tot.reserve(kXFam * kPartials) || c->d_coef2.reserve(kNCoef_mbpol_2b) ||
-        c->d_coef3.reserve(kNCoef_mbpol_3b) || c->d_totals.reserve(4 * kPartials) || c->d_coef1b.reserve(n1b) ||
+    if (xbad || c->d_xfam_tot.reserve(kXFam * kPartials) || c->d_coef2.reserve(kNSlot_mbpol_2b) ||
+        c->d_coef3.reserve(kNSlot_mbpol_3b) || c->d_totals.reserve(4 * kPartials) || c->d_coef1b.reserve(n1b) ||
         c->d_coef1b_co2.reserve(n1b_co2) ||
         c->d_box.reserve(1) || c->d_fam_tot.reserve(kFamilies * kPartials) ||
         c->d_coefn[FAM_CH4H2O_2B].reserve(kNCoef_ch4h2o_2b) || c->d_coefn[FAM_CH4CH4_2B].reserve(kNCoef_ch4ch4_2b) ||
-        c->d_coefn[FAM_CH4H2O2_3B].reserve(kNCoef_ch4h2o2_3b)) {
+        c->d_coefn[FAM_CH4H2O2_3B].reserve(kNSlot_ch4h2o2_3b)) {
         delete c;
         return fail(MBXG_ENOMEM, "mbxg_create: device allocation failed");
     }
-    HIPCHK(hipMemcpy(c->d_coef2.p, kFit_mbpol_2b, sizeof(double) * kNCoef_mbpol_2b, hipMemcpyHostToDevice));
+    auto upload = [](double* dst, const SymTable* t, const double* fit, int n) {
+        const std::vector<double> b = kernel_coefficients(t, fit, n);  // some 10 us a table
+        return hipMemcpy(dst, b.data(), sizeof(double) * b.size(), hipMemcpyHostToDevice);
+    };
+    HIPCHK(upload(c->d_coef2.p, &kSymMbpol2b, kFit_mbpol_2b, kNCoef_mbpol_2b));
     HIPCHK(hipMemcpy(c->d_coef1b.p, fit1b, sizeof(double) * n1b, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_coef1b_co2.p, fit1b_co2, sizeof(double) * n1b_co2, hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->d_totals.p, 0, sizeof(double) * 4 * kPartials));
@@ -259,13 +295,12 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
         const double* fit = xfam_default_coef(f, &nx);
         HIPCHK(hipMemcpy(c->d_xcoef[f].p, fit, sizeof(double) * nx, hipMemcpyHostToDevice));
     }
-    HIPCHK(hipMemcpy(c->d_coef3.p, kFit_mbpol_3b, sizeof(double) * kNCoef_mbpol_3b, hipMemcpyHostToDevice));
+    HIPCHK(upload(c->d_coef3.p, &kSymMbpol3b, kFit_mbpol_3b, kNCoef_mbpol_3b));
     HIPCHK(hipMemcpy(c->d_coefn[FAM_CH4H2O_2B].p, kFit_ch4h2o_2b, sizeof(double) * kNCoef_ch4h2o_2b,
                      hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_coefn[FAM_CH4CH4_2B].p, kFit_ch4ch4_2b, sizeof(double) * kNCoef_ch4ch4_2b,
                      hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_coefn[FAM_CH4H2O2_3B].p, kFit_ch4h2o2_3b, sizeof(double) * kNCoef_ch4h2o2_3b,
-                     hipMemcpyHostToDevice));
+    HIPCHK(upload(c->d_coefn[FAM_CH4H2O2_3B].p, &kSymCh4h2o2, kFit_ch4h2o2_3b, kNCoef_ch4h2o2_3b));
     c->box.periodic = 0;
     *out = c;
     return MBXG_OK;
@@ -608,12 +643,15 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
     std::string m(model);
     double* dst;
     const double* fit;
+    const SymTable* sym = nullptr;
     int need;
     if (m == "mbpol_2b") {
+        sym = &kSymMbpol2b;
         dst = c->d_coef2.p;
         fit = kFit_mbpol_2b;
         need = kNCoef_mbpol_2b;
     } else if (m == "mbpol_3b") {
+        sym = &kSymMbpol3b;
         dst = c->d_coef3.p;
         fit = kFit_mbpol_3b;
         need = kNCoef_mbpol_3b;
@@ -626,6 +664,7 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
         fit = kFit_ch4ch4_2b;
         need = kNCoef_ch4ch4_2b;
     } else if (m == "ch4h2o2_3b") {
+        sym = &kSymCh4h2o2;
         dst = c->d_coefn[FAM_CH4H2O2_3B].p;
         fit = kFit_ch4h2o2_3b;
         need = kNCoef_ch4h2o2_3b;
@@ -643,7 +682,8 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
         return fail(MBXG_EINVAL, "mbxg_set_coefficients: unknown model '%s'", model);
     }
     if (a && n != need) return fail(MBXG_EINVAL, "mbxg_set_coefficients: %s takes %d coefficients", model, need);
-    HIPCHK(hipMemcpyAsync(dst, a ? a : fit, sizeof(double) * need, hipMemcpyHostToDevice, c->stream));
+    const std::vector<double> b = kernel_coefficients(sym, a ? a : fit, need);
+    HIPCHK(hipMemcpyAsync(dst, b.data(), sizeof(double) * b.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->inputs_changed = true;
     return MBXG_OK;

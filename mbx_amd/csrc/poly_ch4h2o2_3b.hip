@@ -11,7 +11,7 @@ namespace mbxg {
 
 hipError_t launch_poly_ch4h2o2_3b(const double* xs, const int* n_dev, int cap, int ld, const double* coef,
                                   int do_grads, double* gs, double* ps, int P, hipStream_t st) {
-    return launch_poly<55, 8, poly_ch4h2o2_3b_parts, poly_ch4h2o2_3b_e_parts, 2>(xs, n_dev, cap, ld, coef, do_grads,
+    return launch_poly<55, 8, poly_ch4h2o2_3b_parts, poly_ch4h2o2_3b_e_parts, poly_ch4h2o2_3b_sym, 2>(xs, n_dev, cap, ld, coef, do_grads,
                                                                                    gs, ps, P, st);
 }
 

@@ -7,6 +7,16 @@
 // k_poly_eg_pair_chain3 (poly_mbpol_pair.hip), runs the 3B chain rule strictly after a block's
 // polynomial, behind a fence, so the two phases' registers are allocated one after the other.
 //
+// The polynomial is evaluated in symmetry-adapted coordinates (mbx_amd/gen/symmetry.py): sums and
+// differences of the variables that exchanges of like sites permute.  In them a fraction of the
+// monomials survives (MB-pol 3B 6,773 of 33,525: 17.1k FP64 operations a trimer for value and
+// gradient instead of 72.5k; 2B 6.5k instead of 27.5k; CH4-H2O-H2O 11.7k instead of 63.0k), which is
+// what bounds these kernels: at full occupancy they run at 95-99% of the FP64 issue slots, alone on
+// the chip at one wavefront's serial length.  The transform (SYM, in place on the registers, its own
+// transpose) costs one to three additions a variable each way.  Whole steps, before and after: 2048
+// waters 632 -> 354 us, 6859 waters 1592 -> 762 us, 32 beads of 57 CH4 + 513 H2O 4.24 -> 2.81 ms,
+// six waters 284 -> 206 us.
+//
 // Layout: xs and gs are variable-major ("SoA"), entry (j, t) at j*ld + t, so a wavefront's 64
 // lanes read and write 64 consecutive doubles per variable.
 #pragma once
@@ -20,6 +30,7 @@ namespace mbxg {
 
 typedef double (*poly_eg_part_fn)(int, int, mbxg_cptr, const double*, double*);
 typedef double (*poly_e_part_fn)(int, int, mbxg_cptr, const double*);
+typedef void (*poly_sym_fn)(double*);
 
 // The generated polynomial comes in Q pieces (linear: value and gradient are sums over the
 // pieces).  A block holds 64 n-mers and P = blockDim.x / 64 wavefronts (P divides Q); wavefront
@@ -32,7 +43,7 @@ constexpr int kRedChunk = 12;
 constexpr size_t poly_lds_bytes(int P) { return (size_t)(P - 1) * (kRedChunk + 1) * 64 * sizeof(double); }
 
 // One block's work: 64 n-mers of group `grp`, P = blockDim.x / 64 wavefronts.
-template <int NV, int Q, poly_eg_part_fn PART>
+template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM>
 __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict__ xs, const int* __restrict__ n_dev,
                                               int cap, int ld, uint64_t coef_addr, double* __restrict__ gs,
                                               double* __restrict__ ps, double* red) {
@@ -49,6 +60,7 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
         x[j] = active ? xs[(size_t)j * ld + t] : 0.0;
         g[j] = 0.0;
     }
+    SYM(x);
     double E = PART(wv, P, C, x, g);
     if (P > 1) {
 #pragma unroll
@@ -72,6 +84,7 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
         }
     }
     if (wv == 0 && active) {
+        SYM(g);
 #pragma unroll
         for (int j = 0; j < NV; ++j) gs[(size_t)j * ld + t] = g[j];
         ps[t] = E;
@@ -80,12 +93,12 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
 
 // Energy and gradient, WPE waves per SIMD: 3 for MB-pol (at most 168 VGPRs), 2 for the
 // 55-variable CH4-H2O-H2O polynomial (x and g alone take 220 VGPRs).
-template <int NV, int Q, poly_eg_part_fn PART, int WPE>
+template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM, int WPE>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_poly_eg(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap, int ld, uint64_t coef_addr,
               double* __restrict__ gs, double* __restrict__ ps) {
     extern __shared__ double red[];  // [P-1][kRedChunk+1][64]
-    poly_eg_group<NV, Q, PART>(blockIdx.x, xs, n_dev, cap, ld, coef_addr, gs, ps, red);
+    poly_eg_group<NV, Q, PART, SYM>(blockIdx.x, xs, n_dev, cap, ld, coef_addr, gs, ps, red);
 }
 
 // Two polynomials in one launch: blocks [0, nb_a) evaluate polynomial A (groups of 64 n-mers in
@@ -100,18 +113,18 @@ struct PolyJob {
     double* ps;
 };
 
-template <int NVA, int QA, poly_eg_part_fn PA, int NVB, int QB, poly_eg_part_fn PB>
+template <int NVA, int QA, poly_eg_part_fn PA, poly_sym_fn SA, int NVB, int QB, poly_eg_part_fn PB, poly_sym_fn SB>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 3)))
     k_poly_eg_pair(PolyJob A, PolyJob B, int nb_a) {
     extern __shared__ double red[];
     if ((int)blockIdx.x < nb_a)
-        poly_eg_group<NVA, QA, PA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
+        poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
     else
-        poly_eg_group<NVB, QB, PB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
+        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
 }
 
 // Energy only.
-template <int NV, int Q, poly_e_part_fn PART>
+template <int NV, int Q, poly_e_part_fn PART, poly_sym_fn SYM>
 __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap,
                                                 int ld, uint64_t coef_addr, double* __restrict__ ps) {
     extern __shared__ double red[];  // [P-1][64]
@@ -125,6 +138,7 @@ __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, c
     double x[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) x[j] = active ? xs[(size_t)j * ld + t] : 0.0;
+    SYM(x);
     double E = PART(wv, P, C, x);
     if (wv > 0) red[(wv - 1) * 64 + lane] = E;
     if (P > 1) __syncthreads();
@@ -135,7 +149,7 @@ __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, c
 }
 
 // Launch helper: P wavefronts per 64 n-mers (P in {1, 2, 4, 8}, dividing Q).
-template <int NV, int Q, poly_eg_part_fn PEG, poly_e_part_fn PE, int WPE = 3>
+template <int NV, int Q, poly_eg_part_fn PEG, poly_e_part_fn PE, poly_sym_fn SYM, int WPE = 3>
 hipError_t launch_poly(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads,
                        double* gs, double* ps, int P, hipStream_t st) {
     if (cap <= 0) return hipSuccess;
@@ -143,10 +157,10 @@ hipError_t launch_poly(const double* xs, const int* n_dev, int cap, int ld, cons
     const int nb = (cap + 63) / 64;
     const uint64_t ca = (uint64_t)(uintptr_t)coef;
     if (do_grads)
-        hipLaunchKernelGGL((k_poly_eg<NV, Q, PEG, WPE>), dim3(nb), dim3(64 * P), poly_lds_bytes(P), st, xs, n_dev, cap,
+        hipLaunchKernelGGL((k_poly_eg<NV, Q, PEG, SYM, WPE>), dim3(nb), dim3(64 * P), poly_lds_bytes(P), st, xs, n_dev, cap,
                            ld, ca, gs, ps);
     else
-        hipLaunchKernelGGL((k_poly_e<NV, Q, PE>), dim3(nb), dim3(64 * P), (size_t)(P - 1) * 64 * sizeof(double), st,
+        hipLaunchKernelGGL((k_poly_e<NV, Q, PE, SYM>), dim3(nb), dim3(64 * P), (size_t)(P - 1) * 64 * sizeof(double), st,
                            xs, n_dev, cap, ld, ca, ps);
     return hipGetLastError();
 }

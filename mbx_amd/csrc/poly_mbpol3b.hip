@@ -10,7 +10,7 @@ namespace mbxg {
 
 hipError_t launch_poly_mbpol3b(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads,
                                double* gs, double* ps, int P, hipStream_t st) {
-    return launch_poly<36, 8, poly_mbpol_3b_parts, poly_mbpol_3b_e_parts>(xs, n_dev, cap, ld, coef, do_grads, gs,
+    return launch_poly<36, 8, poly_mbpol_3b_parts, poly_mbpol_3b_e_parts, poly_mbpol_3b_sym>(xs, n_dev, cap, ld, coef, do_grads, gs,
                                                                                 ps, P, st);
 }
 

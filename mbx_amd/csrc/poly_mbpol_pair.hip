@@ -25,7 +25,8 @@ hipError_t launch_poly_mbpol_pair(double* ws3, const int* n3_dev, int cap3, cons
     const PolyJob B{ws2, n2_dev, cap2, ld2, (uint64_t)(uintptr_t)coef2, ws2 + (size_t)31 * ld2,
                     ws2 + (size_t)62 * ld2};
     const int nb3 = ld3 / 64, nb2 = ld2 / 64;
-    hipLaunchKernelGGL((k_poly_eg_pair<36, 8, poly_mbpol_3b_parts, 31, 8, poly_mbpol_2b_parts>), dim3(nb3 + nb2),
+    hipLaunchKernelGGL((k_poly_eg_pair<36, 8, poly_mbpol_3b_parts, poly_mbpol_3b_sym, 31, 8, poly_mbpol_2b_parts,
+                        poly_mbpol_2b_sym>), dim3(nb3 + nb2),
                        dim3(64 * split), poly_lds_bytes(split), st, A, B, nb3);
     return hipGetLastError();
 }
@@ -51,15 +52,15 @@ constexpr int kChainTable3 = 128;
 // other wavefronts end there, and their slots take further polynomial blocks.  The chain rule's
 // gathers and atomics so wait beside other wavefronts' polynomial arithmetic instead of in a
 // kernel of their own.  The 2B blocks are unchanged.
-template <int NVA, int QA, poly_eg_part_fn PA, int NVB, int QB, poly_eg_part_fn PB>
+template <int NVA, int QA, poly_eg_part_fn PA, poly_sym_fn SA, int NVB, int QB, poly_eg_part_fn PB, poly_sym_fn SB>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 3)))
     k_poly_eg_pair_chain3(PolyJob A, PolyJob B, int nb_a, NmerCtx N, Chain3Job C) {
     extern __shared__ double red[];
     if ((int)blockIdx.x >= nb_a) {
-        poly_eg_group<NVB, QB, PB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
+        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
         return;
     }
-    poly_eg_group<NVA, QA, PA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
+    poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
     const int n = min(*A.n_dev, A.cap);
     if ((threadIdx.x >> 6) != 0 || (int)blockIdx.x * 64 >= n) return;
     // this wavefront's gs / ps stores are complete before it loads them back
@@ -87,7 +88,8 @@ hipError_t launch_poly_mbpol_pair_chain3(double* ws3, const int* list3, const in
     const Chain3Job C{list3, ws3 + (size_t)73 * ld3, grad, e3_out, vir3_out, partials3};
     const int nb3 = ld3 / 64, nb2 = ld2 / 64;
     const size_t lds = std::max(poly_lds_bytes(split), sizeof(GradTable<kChainTable3, 9>));
-    hipLaunchKernelGGL((k_poly_eg_pair_chain3<36, 8, poly_mbpol_3b_parts, 31, 8, poly_mbpol_2b_parts>),
+    hipLaunchKernelGGL((k_poly_eg_pair_chain3<36, 8, poly_mbpol_3b_parts, poly_mbpol_3b_sym, 31, 8, poly_mbpol_2b_parts,
+                        poly_mbpol_2b_sym>),
                        dim3(nb3 + nb2), dim3(64 * split), lds, st, A, B, nb3, N, C);
     return hipGetLastError();
 }

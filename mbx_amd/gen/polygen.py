@@ -23,9 +23,10 @@ which keeps the number of level-3 nodes low.
 
 Output: a C++ include with
     __device__ __forceinline__ double <fn>(mbxg_cptr C, const double* x, double* g)
-where C is the derived coefficient table: C[q] = a[ck[q]] * cs[q] with the
-(ck, cs) map emitted alongside (the scale cs is 1 except for symmetry-reduced
-tables).  A second function <fn>_e evaluates E only.
+where C is the derived coefficient table.  The blocked polynomials are evaluated in
+symmetry-adapted coordinates (symmetry.py): x is transformed in place by <fn>_sym before the
+call, g by the same function after it, and C[q] = sum_i a[K[i]] W[i] with the (K, W) rows in
+gen/sym_<name>.inc.  A second function <fn>_e evaluates E only.
 
 Regions of the op stream are separated by MBXG_NODE_FENCE(C, v) (poly_support.hpp): a
 scheduling barrier plus an opaque redefinition of the coefficient pointer that consumes the
@@ -34,9 +35,12 @@ loads and temporaries local to the node, so the register allocator never sees te
 thousands of simultaneously live values, and keeps compile time linear in the code size.
 """
 import collections
+import functools
 import os
 import re
 import sys
+
+import symmetry
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
@@ -104,7 +108,7 @@ class Schedule:
         self.const3 = {}
         leaves2 = collections.defaultdict(list)
         for q, m in by_deg[3]:
-            if m in leaves3:
+            if m in leaves3 and m not in self.const3:
                 self.const3[m] = q
             else:
                 leaves2[m[:2]].append((q, m[2]))
@@ -112,7 +116,7 @@ class Schedule:
         self.const2 = {}
         leaves1 = collections.defaultdict(list)
         for q, m in by_deg[2]:
-            if m in nodes2:
+            if m in nodes2 and m not in self.const2:
                 self.const2[m] = q
             else:
                 leaves1[m[:1]].append((q, m[1]))
@@ -120,7 +124,7 @@ class Schedule:
         self.const1 = {}
         self.leaves0 = []
         for q, m in by_deg[1]:
-            if m in nodes1:
+            if m in nodes1 and m not in self.const1:
                 self.const1[m] = q
             else:
                 self.leaves0.append((q, m[0]))
@@ -311,9 +315,11 @@ def _lhs(stmt):
     return lhs.replace("+", "").strip()
 
 
-def full_terms(monos):
-    """Terms of the full polynomial: coefficient slot q == coefficient index k, scale 1."""
-    return [(k, m) for k, m in monos], None
+@functools.lru_cache(maxsize=None)
+def adapted(name):
+    """(nvars, fitted coefficients, the polynomial in symmetry-adapted coordinates)."""
+    nvars, coef, monos = load_table(name)
+    return nvars, coef, symmetry.Adapted(name, nvars, monos, coef)
 
 
 # The polynomial is cut into NPARTS pieces so that 1, 2, 4 or 8 wavefronts can share one
@@ -416,19 +422,19 @@ def generate_holder(name, out_dir):
 
 
 def generate(name, fn, out_dir):
-    nvars, coef, monos = load_table(name)
-    terms, _ = full_terms(monos)
-    s = Schedule(nvars, terms)
+    nvars, coef, sym = adapted(name)
+    s = Schedule(nvars, sym.terms)
     c = s.counts()
     hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
            "// Schedule: %s" % ", ".join("%s=%d" % kv for kv in c.items()),
-           "// Coefficient slots index the fitted coefficient vector directly (%d slots)." % len(coef),
+           "// Symmetry-adapted coordinates: %s_sym transforms x before and g after; C holds %d slots "
+           "(gen/sym_%s.inc)." % (fn, len(sym.rows) + len(sym.low), name),
            "#pragma once",
            "#include \"poly_support.hpp\"", ""]
     assign = s.partition(NPARTS)
     hdr.insert(2, "// %d parts (op-count balance: %s); <fn>_parts(w, P, ...) evaluates parts w, w+P, ... "
                   "into g and returns their share of the value." % (NPARTS, ", ".join(str(v) for v in s.part_load)))
-    body = []
+    body = [symmetry.emit_transform(fn + "_sym", sym.blocks)]
     for grad, suffix in ((True, ""), (False, "_e")):
         for k in range(NPARTS):
             body.append(s.emit("%s%s_p%d" % (fn, suffix, k), grad=grad, part=k, assign=assign))
@@ -447,6 +453,8 @@ def generate(name, fn, out_dir):
     write_if_changed(path, src)
     # fitted coefficients, for the host runtime's default table
     write_if_changed(os.path.join(out_dir, "coef_%s.inc" % name), coef_source(name, coef))
+    write_if_changed(os.path.join(out_dir, "sym_%s.inc" % name),
+                     symmetry.emit_tables(name, sym, len(coef), name in AD_POLYS))
     return path, c
 
 
