@@ -28,6 +28,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -38,7 +40,16 @@
 #include "gen/coef_mbpol_2b.inc"
 #include "gen/coef_mbpol_3b.inc"
 #define MBXG_SYM_SPACE static
+#include "gen/sym_alkali_h2o2_3b.inc"
+#include "gen/sym_alkali_h2o_2b.inc"
+#include "gen/sym_ch4ch4_2b.inc"
 #include "gen/sym_ch4h2o2_3b.inc"
+#include "gen/sym_ch4h2o_2b.inc"
+#include "gen/sym_co2co2_2b.inc"
+#include "gen/sym_co2x3_3b.inc"
+#include "gen/sym_h2ox4_4b.inc"
+#include "gen/sym_halide_h2o2_3b.inc"
+#include "gen/sym_halide_h2o_2b.inc"
 #include "gen/sym_mbpol_2b.inc"
 #include "gen/sym_mbpol_3b.inc"
 #include "mbxg_kernels.hpp"
@@ -95,9 +106,41 @@ std::vector<double> kernel_coefficients(const SymTable* t, const double* a, int 
     return b;
 }
 
-#define MBXG_SYM(name) {kSymRow_##name, kSymK_##name, kSymW_##name, kSymLow_##name, kNRow_##name, kNLow_##name}
-const SymTable kSymMbpol2b = MBXG_SYM(mbpol_2b), kSymMbpol3b = MBXG_SYM(mbpol_3b), kSymCh4h2o2 = MBXG_SYM(ch4h2o2_3b);
+// The table of a polynomial structure (nullptr: the coefficients are taken as they are).
+const SymTable* sym_table(const std::string& structure) {
+#define MBXG_SYM(name)                                                                                        \
+    if (structure == #name) {                                                                                 \
+        static const SymTable t = {kSymRow_##name, kSymK_##name,   kSymW_##name, kSymLow_##name, kNRow_##name, \
+                                   kNLow_##name};                                                             \
+        return &t;                                                                                            \
+    }
+    MBXG_SYM(mbpol_2b)
+    MBXG_SYM(mbpol_3b)
+    MBXG_SYM(ch4h2o_2b)
+    MBXG_SYM(ch4ch4_2b)
+    MBXG_SYM(ch4h2o2_3b)
+    MBXG_SYM(halide_h2o_2b)
+    MBXG_SYM(halide_h2o2_3b)
+    MBXG_SYM(alkali_h2o_2b)
+    MBXG_SYM(alkali_h2o2_3b)
+    MBXG_SYM(co2co2_2b)
+    MBXG_SYM(co2x3_3b)
+    MBXG_SYM(h2ox4_4b)
 #undef MBXG_SYM
+    return nullptr;
+}
+
+// The fitted coefficients' kernel form, computed once per process (some 0.3 ms for all the tables).
+const std::vector<double>& default_coefficients(const SymTable* t, const double* fit, int n) {
+    static std::mutex mu;
+    static std::map<const double*, std::vector<double>> done;
+    std::lock_guard<std::mutex> lock(mu);
+    auto it = done.find(fit);
+    if (it == done.end()) it = done.emplace(fit, kernel_coefficients(t, fit, n)).first;
+    return it->second;
+}
+
+int kernel_slots(const SymTable* t, int n) { return t ? t->nrow + t->nlow : n; }
 
 template <class T>
 struct DBuf {
@@ -271,36 +314,34 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
     for (int f = 0; f < kXFam; ++f) {
         int nx = 0;
         xfam_default_coef(f, &nx);
-        xbad = xbad || c->d_xcoef[f].reserve(nx);
+        xbad = xbad || c->d_xcoef[f].reserve(kernel_slots(sym_table(xfam_structure(f)), nx));
     }
     if (xbad || c->d_xfam_tot.reserve(kXFam * kPartials) || c->d_coef2.reserve(kNSlot_mbpol_2b) ||
         c->d_coef3.reserve(kNSlot_mbpol_3b) || c->d_totals.reserve(4 * kPartials) || c->d_coef1b.reserve(n1b) ||
         c->d_coef1b_co2.reserve(n1b_co2) ||
         c->d_box.reserve(1) || c->d_fam_tot.reserve(kFamilies * kPartials) ||
-        c->d_coefn[FAM_CH4H2O_2B].reserve(kNCoef_ch4h2o_2b) || c->d_coefn[FAM_CH4CH4_2B].reserve(kNCoef_ch4ch4_2b) ||
+        c->d_coefn[FAM_CH4H2O_2B].reserve(kNSlot_ch4h2o_2b) || c->d_coefn[FAM_CH4CH4_2B].reserve(kNSlot_ch4ch4_2b) ||
         c->d_coefn[FAM_CH4H2O2_3B].reserve(kNSlot_ch4h2o2_3b)) {
         delete c;
         return fail(MBXG_ENOMEM, "mbxg_create: device allocation failed");
     }
     auto upload = [](double* dst, const SymTable* t, const double* fit, int n) {
-        const std::vector<double> b = kernel_coefficients(t, fit, n);  // some 10 us a table
+        const std::vector<double>& b = default_coefficients(t, fit, n);
         return hipMemcpy(dst, b.data(), sizeof(double) * b.size(), hipMemcpyHostToDevice);
     };
-    HIPCHK(upload(c->d_coef2.p, &kSymMbpol2b, kFit_mbpol_2b, kNCoef_mbpol_2b));
+    HIPCHK(upload(c->d_coef2.p, sym_table("mbpol_2b"), kFit_mbpol_2b, kNCoef_mbpol_2b));
     HIPCHK(hipMemcpy(c->d_coef1b.p, fit1b, sizeof(double) * n1b, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->d_coef1b_co2.p, fit1b_co2, sizeof(double) * n1b_co2, hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->d_totals.p, 0, sizeof(double) * 4 * kPartials));
     for (int f = 0; f < kXFam; ++f) {
         int nx = 0;
         const double* fit = xfam_default_coef(f, &nx);
-        HIPCHK(hipMemcpy(c->d_xcoef[f].p, fit, sizeof(double) * nx, hipMemcpyHostToDevice));
+        HIPCHK(upload(c->d_xcoef[f].p, sym_table(xfam_structure(f)), fit, nx));
     }
-    HIPCHK(upload(c->d_coef3.p, &kSymMbpol3b, kFit_mbpol_3b, kNCoef_mbpol_3b));
-    HIPCHK(hipMemcpy(c->d_coefn[FAM_CH4H2O_2B].p, kFit_ch4h2o_2b, sizeof(double) * kNCoef_ch4h2o_2b,
-                     hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_coefn[FAM_CH4CH4_2B].p, kFit_ch4ch4_2b, sizeof(double) * kNCoef_ch4ch4_2b,
-                     hipMemcpyHostToDevice));
-    HIPCHK(upload(c->d_coefn[FAM_CH4H2O2_3B].p, &kSymCh4h2o2, kFit_ch4h2o2_3b, kNCoef_ch4h2o2_3b));
+    HIPCHK(upload(c->d_coef3.p, sym_table("mbpol_3b"), kFit_mbpol_3b, kNCoef_mbpol_3b));
+    HIPCHK(upload(c->d_coefn[FAM_CH4H2O_2B].p, sym_table("ch4h2o_2b"), kFit_ch4h2o_2b, kNCoef_ch4h2o_2b));
+    HIPCHK(upload(c->d_coefn[FAM_CH4CH4_2B].p, sym_table("ch4ch4_2b"), kFit_ch4ch4_2b, kNCoef_ch4ch4_2b));
+    HIPCHK(upload(c->d_coefn[FAM_CH4H2O2_3B].p, sym_table("ch4h2o2_3b"), kFit_ch4h2o2_3b, kNCoef_ch4h2o2_3b));
     c->box.periodic = 0;
     *out = c;
     return MBXG_OK;
@@ -643,15 +684,13 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
     std::string m(model);
     double* dst;
     const double* fit;
-    const SymTable* sym = nullptr;
+    const SymTable* sym = sym_table(m);
     int need;
     if (m == "mbpol_2b") {
-        sym = &kSymMbpol2b;
         dst = c->d_coef2.p;
         fit = kFit_mbpol_2b;
         need = kNCoef_mbpol_2b;
     } else if (m == "mbpol_3b") {
-        sym = &kSymMbpol3b;
         dst = c->d_coef3.p;
         fit = kFit_mbpol_3b;
         need = kNCoef_mbpol_3b;
@@ -664,7 +703,6 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
         fit = kFit_ch4ch4_2b;
         need = kNCoef_ch4ch4_2b;
     } else if (m == "ch4h2o2_3b") {
-        sym = &kSymCh4h2o2;
         dst = c->d_coefn[FAM_CH4H2O2_3B].p;
         fit = kFit_ch4h2o2_3b;
         need = kNCoef_ch4h2o2_3b;
@@ -677,6 +715,7 @@ extern "C" int mbxg_set_coefficients(mbxg_ctx* c, const char* model, const doubl
     } else if (xfam_index(m) >= 0) {
         const int f = xfam_index(m);
         dst = c->d_xcoef[f].p;
+        sym = sym_table(xfam_structure(f));
         fit = xfam_default_coef(f, &need);
     } else {
         return fail(MBXG_EINVAL, "mbxg_set_coefficients: unknown model '%s'", model);

@@ -1,5 +1,5 @@
 // MB-nrg CH4 families on the GPU: variable and chain-rule stages for the holders described in
-// gen/holder_<name>.inc, with the polynomial pieces of gen/poly_<name>_p<k>.hip between them.
+// gen/holder_<name>.inc, with the polynomials (gen/poly_<name>.hip, poly_ch4h2o2_3b.hip) between them.
 //
 // Restates, per n-mer (one lane each):
 //   x2b_A1B2Z2_C1D4_v1x::eval   potential/2b/x2b_A1B2Z2_C1D4_deg3_exp0_v1x.cpp:954-1220 (h2o, ch4)
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(64) k_vars_nrg(const int* __restrict__ list, c
 constexpr int kGradBlockNrg = 128;
 
 // Stage 3: energy; with GRAD the chain rule, virial and gradient scatter.  gs / ps hold the
-// polynomial's pieces ([piece][var][ld], [piece][ld]), summed here in piece order.
+// polynomial's gradient ([var][ld]) and value.
 template <class H, bool GRAD>
 __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restrict__ list, const int* __restrict__ n_dev,
                                                             int cap, NmerCtx N, const double* __restrict__ xs,
@@ -210,9 +210,7 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
     double e_sum = 0.0;
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     if (t < n) {
-        double P = 0.0;
-#pragma unroll
-        for (int q = 0; q < H::kPieces; ++q) P += ps[(size_t)q * ld + t];
+        const double P = ps[t];
         double e;
         if (GRAD) {
             double x[3 * H::kNSites], oh1[3], oh2[3];
@@ -226,9 +224,7 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
             for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
             static_for<H::kNVars>([&](auto J) {
                 constexpr int j = decltype(J)::value;
-                double gj = 0.0;
-#pragma unroll
-                for (int q = 0; q < H::kPieces; ++q) gj += gs[((size_t)q * H::kNVars + j) * ld + t];
+                double gj = gs[(size_t)j * ld + t];
                 if (H::kMon == 3) gj *= sw;  // the 3B holder scales the polynomial gradient first
                 double dv[3], gg;
                 nrg_value<H, j>(x, dv, gg);
@@ -327,38 +323,14 @@ namespace {
 template <class H>
 size_t workspace_nrg(int cap) {
     const size_t ld = ((size_t)cap + 63) / 64 * 64;
-    return ((size_t)H::kNVars * (1 + H::kPieces) + H::kPieces + 1) * ld;
+    return ((size_t)H::kNVars * 2 + 2) * ld;
 }
 
-typedef hipError_t (*piece_launch)(const double*, const int*, int, int, const double*, int, double*, double*,
-                                   hipStream_t);
+typedef hipError_t (*poly_launch)(const double*, const int*, int, int, const double*, int, double*, double*, int,
+                                  hipStream_t);
 
-// The polynomial stage of a pieced family: one kernel per piece, each into its own slice.
-struct Pieced {
-    const piece_launch* pieces;
-    int count;
-    hipError_t operator()(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads,
-                          double* gs, double* ps, int nv, hipStream_t st) const {
-        for (int q = 0; q < count; ++q) {
-            hipError_t e = pieces[q](xs, n_dev, cap, ld, coef, do_grads, gs + (size_t)q * nv * ld, ps + (size_t)q * ld, st);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
-};
-
-// The polynomial stage of a blocked family: one kernel, `split` wavefronts per 64 n-mers.
-struct Blocked {
-    hipError_t (*launch)(const double*, const int*, int, int, const double*, int, double*, double*, int, hipStream_t);
-    int split;
-    hipError_t operator()(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads,
-                          double* gs, double* ps, int, hipStream_t st) const {
-        return launch(xs, n_dev, cap, ld, coef, do_grads, gs, ps, split, st);
-    }
-};
-
-template <class H, class Poly>
-hipError_t launch_nrg(const Poly& poly, const int* list, const int* n_dev, int cap, const NmerCtx& N,
+template <class H>
+hipError_t launch_nrg(poly_launch poly, int split, const int* list, const int* n_dev, int cap, const NmerCtx& N,
                       const double* coef, int do_grads, double* grad, double* e_out, double* vir_out,
                       double* partials, double* ws, hipStream_t st, hipEvent_t* ev) {
     if (cap <= 0) return hipSuccess;
@@ -366,14 +338,14 @@ hipError_t launch_nrg(const Poly& poly, const int* list, const int* n_dev, int c
     const int ld = nb * 64;
     double* xs = ws;
     double* gs = xs + (size_t)H::kNVars * ld;
-    double* ps = gs + (size_t)H::kPieces * H::kNVars * ld;
-    double* sw = ps + (size_t)H::kPieces * ld;
+    double* ps = gs + (size_t)H::kNVars * ld;
+    double* sw = ps + ld;
     if (ev) (void)hipEventRecord(ev[0], st);
     hipLaunchKernelGGL(k_vars_nrg<H>, dim3(nb), dim3(64), 0, st, list, n_dev, cap, N, xs, sw, ld);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[1], st);
-    e = poly(xs, n_dev, cap, ld, coef, do_grads, gs, ps, H::kNVars, st);
+    e = poly(xs, n_dev, cap, ld, coef, do_grads, gs, ps, split, st);
     if (e != hipSuccess) return e;
     if (ev) (void)hipEventRecord(ev[2], st);
     const int ngb = (cap + kGradBlockNrg - 1) / kGradBlockNrg;
@@ -390,21 +362,11 @@ hipError_t launch_nrg(const Poly& poly, const int* list, const int* n_dev, int c
 
 }  // namespace
 
-// The polynomial pieces (gen/poly_<name>_p<k>.hip).
-hipError_t launch_poly_ch4h2o_2b_p0(const double*, const int*, int, int, const double*, int, double*, double*,
-                                    hipStream_t);
-#define MBXG_CH4CH4_PIECE(k)                                                                                      \
-    hipError_t launch_poly_ch4ch4_2b_p##k(const double*, const int*, int, int, const double*, int, double*, double*, \
-                                          hipStream_t);
-MBXG_CH4CH4_PIECE(0)
-MBXG_CH4CH4_PIECE(1)
-MBXG_CH4CH4_PIECE(2)
-MBXG_CH4CH4_PIECE(3)
-MBXG_CH4CH4_PIECE(4)
-MBXG_CH4CH4_PIECE(5)
-MBXG_CH4CH4_PIECE(6)
-MBXG_CH4CH4_PIECE(7)
-#undef MBXG_CH4CH4_PIECE
+// The 2B polynomials (gen/poly_<name>.hip); the CH4-H2O-H2O one is in poly_ch4h2o2_3b.hip.
+hipError_t launch_poly_ch4h2o_2b(const double*, const int*, int, int, const double*, int, double*, double*, int,
+                                 hipStream_t);
+hipError_t launch_poly_ch4ch4_2b(const double*, const int*, int, int, const double*, int, double*, double*, int,
+                                 hipStream_t);
 
 size_t workspace_nrg_family(int family, int cap) {
     switch (family) {
@@ -422,21 +384,16 @@ size_t workspace_nrg_family(int family, int cap) {
 hipError_t launch_nrg_family(int family, const int* list, const int* n_dev, int cap, const NmerCtx& N,
                              const double* coef, int do_grads, double* grad, double* e_out, double* vir_out,
                              double* partials, double* ws, int split, hipStream_t st, hipEvent_t* ev) {
-    static const piece_launch p_ch4h2o[1] = {launch_poly_ch4h2o_2b_p0};
-    static const piece_launch p_ch4ch4[8] = {launch_poly_ch4ch4_2b_p0, launch_poly_ch4ch4_2b_p1,
-                                             launch_poly_ch4ch4_2b_p2, launch_poly_ch4ch4_2b_p3,
-                                             launch_poly_ch4ch4_2b_p4, launch_poly_ch4ch4_2b_p5,
-                                             launch_poly_ch4ch4_2b_p6, launch_poly_ch4ch4_2b_p7};
     switch (family) {
         case FAM_CH4H2O_2B:
-            return launch_nrg<Holder_ch4h2o_2b>(Pieced{p_ch4h2o, 1}, list, n_dev, cap, N, coef, do_grads, grad, e_out, vir_out,
-                                                partials, ws, st, ev);
+            return launch_nrg<Holder_ch4h2o_2b>(launch_poly_ch4h2o_2b, poly_split(cap, poly_wpe(38)), list, n_dev, cap, N,
+                                                coef, do_grads, grad, e_out, vir_out, partials, ws, st, ev);
         case FAM_CH4CH4_2B:
-            return launch_nrg<Holder_ch4ch4_2b>(Pieced{p_ch4ch4, 8}, list, n_dev, cap, N, coef, do_grads, grad, e_out, vir_out,
-                                                partials, ws, st, ev);
+            return launch_nrg<Holder_ch4ch4_2b>(launch_poly_ch4ch4_2b, poly_split(cap, poly_wpe(45)), list, n_dev, cap, N,
+                                                coef, do_grads, grad, e_out, vir_out, partials, ws, st, ev);
         case FAM_CH4H2O2_3B:
-            return launch_nrg<Holder_ch4h2o2_3b>(Blocked{launch_poly_ch4h2o2_3b, split}, list, n_dev, cap, N, coef, do_grads, grad, e_out,
-                                                 vir_out, partials, ws, st, ev);
+            return launch_nrg<Holder_ch4h2o2_3b>(launch_poly_ch4h2o2_3b, split, list, n_dev, cap, N, coef, do_grads,
+                                                 grad, e_out, vir_out, partials, ws, st, ev);
         default:
             return hipErrorInvalidValue;
     }

@@ -222,12 +222,25 @@ hipError_t launch_poly_mbpol_pair_chain3(double* ws3, const int* list3, const in
                                          double* e3_out, double* vir3_out, double* partials3, hipStream_t st);
 // MB-nrg families (eval_nrg.hip): the same three stages for FAM_CH4H2O_2B, FAM_CH4CH4_2B and
 // FAM_CH4H2O2_3B; list entries in emission order (the kernels order each n-mer's monomers
-// for its holder).  `split` (1, 2, 4 or 8) is the wavefronts per 64 n-mers of the blocked
-// CH4-H2O-H2O polynomial; the pieced 2B polynomials ignore it.
+// for its holder).  `split` (1, 2, 4 or 8) is the wavefronts per 64 n-mers of the CH4-H2O-H2O
+// polynomial; the 2B polynomials take poly_split's.
 size_t workspace_nrg_family(int family, int cap);
 hipError_t launch_nrg_family(int family, const int* list, const int* n_dev, int cap, const NmerCtx& N,
                              const double* coef, int do_grads, double* grad, double* e_out, double* vir_out,
                              double* partials, double* ws, int split, hipStream_t st, hipEvent_t* ev);
+
+// Wavefronts per 64 n-mers for a polynomial kernel of `wpe` wavefronts per SIMD, from the n-mers'
+// capacity.  Few groups of 64 leave the chip idle, so each is cut into more and shorter wavefronts; the
+// cut costs a reduction and variables loaded again, so it stops once the chip is full.  Measured on
+// the MB-pol pair with its 3B chain rule (wpe 3; us at split 2 / 4 / 8): 1 group 51 / 37 / 35, 24
+// groups 53 / 39 / 37, 260 61 / 55 / 59, 705 82 / 72 / 88, 1055 95 / 94 / 124, 1742 124 / 123 / 174,
+// 3465 198 / 212 / 322, 10562 539 / 606 / 994 (split 1: 67-80% slower below 1000, 545 at 10562).
+// poly_wpe: wavefronts per SIMD of a value + gradient kernel of nv variables (the generator's rule).
+constexpr int poly_wpe(int nv) { return 512 / (4 * nv + 24) > 4 ? 4 : 512 / (4 * nv + 24) > 1 ? 512 / (4 * nv + 24) : 1; }
+inline int poly_split(int cap, int wpe) {
+    const int groups = (cap + 63) / 64;
+    return groups <= 128 ? 8 : groups <= 400 * wpe ? 4 : 2;
+}
 
 // Polynomial stage alone: xs/gs variable-major with leading dimension ld (= cap rounded up
 // to 64); ps values; n read from n_dev as above; `split` wavefronts (1, 2, 4 or 8) share each

@@ -91,10 +91,13 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
     }
 }
 
-// Energy and gradient, WPE waves per SIMD: 3 for MB-pol (at most 168 VGPRs), 2 for the
-// 55-variable CH4-H2O-H2O polynomial (x and g alone take 220 VGPRs).
+// Energy and gradient, WPE waves per SIMD: x and g take 4 registers a variable and the trie some 24, so
+// 4 up to 26 variables, 3 up to 36 (MB-pol: at most 168 VGPRs), 2 up to 58 (CH4-H2O-H2O: 55), 1 for the
+// 66 of the water 4B polynomial.
+constexpr int poly_max_split(int wpe) { return wpe == 1 ? 4 : 8; }  // a block's wavefronts have to fit one CU
+
 template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM, int WPE>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+__global__ void __launch_bounds__(64 * poly_max_split(WPE)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_poly_eg(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap, int ld, uint64_t coef_addr,
               double* __restrict__ gs, double* __restrict__ ps) {
     extern __shared__ double red[];  // [P-1][kRedChunk+1][64]
@@ -148,20 +151,27 @@ __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, c
     }
 }
 
-// Launch helper: P wavefronts per 64 n-mers (P in {1, 2, 4, 8}, dividing Q).
+// Launch helpers: P wavefronts per 64 n-mers (P in {1, 2, 4, 8}, dividing Q; the widest polynomials
+// take 4 at most).
+template <int NV, int Q, poly_eg_part_fn PEG, poly_sym_fn SYM, int WPE>
+hipError_t launch_poly_eg(const double* xs, const int* n_dev, int cap, int ld, const double* coef, double* gs,
+                          double* ps, int P, hipStream_t st) {
+    if (cap <= 0) return hipSuccess;
+    if (P != 1 && P != 2 && P != 4 && P != 8) return hipErrorInvalidValue;
+    if (P > poly_max_split(WPE)) P = poly_max_split(WPE);
+    hipLaunchKernelGGL((k_poly_eg<NV, Q, PEG, SYM, WPE>), dim3((cap + 63) / 64), dim3(64 * P), poly_lds_bytes(P), st, xs,
+                       n_dev, cap, ld, (uint64_t)(uintptr_t)coef, gs, ps);
+    return hipGetLastError();
+}
+
 template <int NV, int Q, poly_eg_part_fn PEG, poly_e_part_fn PE, poly_sym_fn SYM, int WPE = 3>
 hipError_t launch_poly(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads,
                        double* gs, double* ps, int P, hipStream_t st) {
     if (cap <= 0) return hipSuccess;
+    if (do_grads) return launch_poly_eg<NV, Q, PEG, SYM, WPE>(xs, n_dev, cap, ld, coef, gs, ps, P, st);
     if (P != 1 && P != 2 && P != 4 && P != 8) return hipErrorInvalidValue;
-    const int nb = (cap + 63) / 64;
-    const uint64_t ca = (uint64_t)(uintptr_t)coef;
-    if (do_grads)
-        hipLaunchKernelGGL((k_poly_eg<NV, Q, PEG, SYM, WPE>), dim3(nb), dim3(64 * P), poly_lds_bytes(P), st, xs, n_dev, cap,
-                           ld, ca, gs, ps);
-    else
-        hipLaunchKernelGGL((k_poly_e<NV, Q, PE, SYM>), dim3(nb), dim3(64 * P), (size_t)(P - 1) * 64 * sizeof(double), st,
-                           xs, n_dev, cap, ld, ca, ps);
+    hipLaunchKernelGGL((k_poly_e<NV, Q, PE, SYM>), dim3((cap + 63) / 64), dim3(64 * P),
+                       (size_t)(P - 1) * 64 * sizeof(double), st, xs, n_dev, cap, ld, (uint64_t)(uintptr_t)coef, ps);
     return hipGetLastError();
 }
 

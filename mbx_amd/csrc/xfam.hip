@@ -21,7 +21,7 @@
 //   k_xclass    family, holder order and skip rule of every listed n-mer; per-block counts
 //   k_xscan     block offsets and family totals (one workgroup, fixed order)
 //   k_xemit     each evaluated n-mer at its family's list, in listed order (deterministic)
-// then per family: k_xvars (sites, variables, switch) -> polynomial pieces (gen/xpoly_*.hip)
+// then per family: k_xvars (sites, variables, switch) -> polynomial (gen/xpoly_*.hip)
 // -> k_xgrad (chain rule, switch derivatives, energy, virial, gradient scatter).
 // Tetramers (System::Get4B, AddClusters with nmax = 4, sys_tools.cpp:594-634): k_tetra counts
 // and writes, per query, every match triple the center-3-neighbour rule keeps.
@@ -135,29 +135,29 @@ __device__ __forceinline__ void sort_network(const int* rank_in, int* ix) {
     }
 }
 
-// The families in the order of XFam: enum, holder, polynomial pieces.
+// The families in the order of XFam: enum, holder, polynomial structure.
 #define MBXG_XFAMILIES(X)                              \
-    X(XF_F_H2O_2B, f_h2o_2b, kPHalide2)                \
-    X(XF_CL_H2O_2B, cl_h2o_2b, kPHalide2)              \
-    X(XF_BR_H2O_2B, br_h2o_2b, kPHalide2)              \
-    X(XF_I_H2O_2B, i_h2o_2b, kPHalide2)                \
-    X(XF_CO2CO2_2B, co2co2_2b, kPCo2_2)                \
-    X(XF_F_H2O2_3B, f_h2o2_3b, kPHalide3)              \
-    X(XF_CL_H2O2_3B, cl_h2o2_3b, kPHalide3)            \
-    X(XF_BR_H2O2_3B, br_h2o2_3b, kPHalide3)            \
-    X(XF_I_H2O2_3B, i_h2o2_3b, kPHalide3)              \
-    X(XF_CO2X3_3B, co2x3_3b, kPCo2_3)                  \
-    X(XF_H2OX4_4B, h2ox4_4b, kPH2o_4)                  \
-    X(XF_LI_H2O_2B, li_h2o_2b, kPAlkali2)              \
-    X(XF_NA_H2O_2B, na_h2o_2b, kPAlkali2)              \
-    X(XF_K_H2O_2B, k_h2o_2b, kPAlkali2)                \
-    X(XF_RB_H2O_2B, rb_h2o_2b, kPAlkali2)              \
-    X(XF_CS_H2O_2B, cs_h2o_2b, kPAlkali2)              \
-    X(XF_LI_H2O2_3B, li_h2o2_3b, kPAlkali3)            \
-    X(XF_NA_H2O2_3B, na_h2o2_3b, kPAlkali3)            \
-    X(XF_K_H2O2_3B, k_h2o2_3b, kPAlkali3)              \
-    X(XF_RB_H2O2_3B, rb_h2o2_3b, kPAlkali3)            \
-    X(XF_CS_H2O2_3B, cs_h2o2_3b, kPAlkali3)
+    X(XF_F_H2O_2B, f_h2o_2b, halide_h2o_2b)                \
+    X(XF_CL_H2O_2B, cl_h2o_2b, halide_h2o_2b)              \
+    X(XF_BR_H2O_2B, br_h2o_2b, halide_h2o_2b)              \
+    X(XF_I_H2O_2B, i_h2o_2b, halide_h2o_2b)                \
+    X(XF_CO2CO2_2B, co2co2_2b, co2co2_2b)                \
+    X(XF_F_H2O2_3B, f_h2o2_3b, halide_h2o2_3b)              \
+    X(XF_CL_H2O2_3B, cl_h2o2_3b, halide_h2o2_3b)            \
+    X(XF_BR_H2O2_3B, br_h2o2_3b, halide_h2o2_3b)            \
+    X(XF_I_H2O2_3B, i_h2o2_3b, halide_h2o2_3b)              \
+    X(XF_CO2X3_3B, co2x3_3b, co2x3_3b)                  \
+    X(XF_H2OX4_4B, h2ox4_4b, h2ox4_4b)                  \
+    X(XF_LI_H2O_2B, li_h2o_2b, alkali_h2o_2b)              \
+    X(XF_NA_H2O_2B, na_h2o_2b, alkali_h2o_2b)              \
+    X(XF_K_H2O_2B, k_h2o_2b, alkali_h2o_2b)                \
+    X(XF_RB_H2O_2B, rb_h2o_2b, alkali_h2o_2b)              \
+    X(XF_CS_H2O_2B, cs_h2o_2b, alkali_h2o_2b)              \
+    X(XF_LI_H2O2_3B, li_h2o2_3b, alkali_h2o2_3b)            \
+    X(XF_NA_H2O2_3B, na_h2o2_3b, alkali_h2o2_3b)            \
+    X(XF_K_H2O2_3B, k_h2o2_3b, alkali_h2o2_3b)              \
+    X(XF_RB_H2O2_3B, rb_h2o2_3b, alkali_h2o2_3b)            \
+    X(XF_CS_H2O2_3B, cs_h2o2_3b, alkali_h2o2_3b)
 
 // Family descriptions for the classification: order, the holder's monomer kinds in argument
 // order, the skip radius and how many first-atom separations beyond it skip the n-mer (all of
@@ -175,7 +175,7 @@ constexpr XDesc xdesc() {
     return XDesc{H::kMon, {H::kKind[0], H::kKind[1], H::kKind[2], H::kKind[3]}, H::kROut, H::kSkipMin};
 }
 
-#define MBXG_XDESC(F, name, pieces) xdesc<XHolder_##name>(),
+#define MBXG_XDESC(F, name, poly) xdesc<XHolder_##name>(),
 __constant__ const XDesc kXDesc[kXFam] = {MBXG_XFAMILIES(MBXG_XDESC)};
 #undef MBXG_XDESC
 
@@ -494,8 +494,7 @@ constexpr int kGradBlockX = 128;
 
 // Stage 3: energy; the polynomial gradient scaled by the switch combination, to the sites, the
 // lone-pair sites' gradients back to O, H, H (water_monomer_lp.cpp:25-48), the switch derivative
-// along every pair; virial -sum_atoms x (x) g; gradient scatter.  gs / ps hold the polynomial's
-// pieces ([piece][var][ld], [piece][ld]), summed in piece order.  grad == nullptr: energies only
+// along every pair; virial -sum_atoms x (x) g; gradient scatter.  grad == nullptr: energies only
 // (the reference computes the virial with the gradients only).
 template <class H>
 __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ list, const int* __restrict__ n_dev,
@@ -512,9 +511,7 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     if (t < n && !grad) {
         const int* ent = list + (size_t)(H::kMon + 1) * t;
-        double P = 0.0;
-#pragma unroll
-        for (int q = 0; q < H::kPieces; ++q) P += ps[(size_t)q * ld + t];
+        const double P = ps[t];
         double x[3 * H::kNSites], oh1[2][3], oh2[2][3];
         xsites<H>(N, ent, x, oh1, oh2);
         double d[6][3], r[6], s[6], gsw[6];
@@ -522,9 +519,7 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
         e_out[t] = e_sum;
     } else if (t < n) {
         const int* ent = list + (size_t)(H::kMon + 1) * t;
-        double P = 0.0;
-#pragma unroll
-        for (int q = 0; q < H::kPieces; ++q) P += ps[(size_t)q * ld + t];
+        const double P = ps[t];
         double x[3 * H::kNSites], oh1[2][3], oh2[2][3];
         xsites<H>(N, ent, x, oh1, oh2);
         double d[6][3], r[6], s[6], gsw[6];
@@ -534,10 +529,7 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
         for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
         static_for<H::kNVars>([&](auto J) {
             constexpr int j = decltype(J)::value;
-            double gj = 0.0;
-#pragma unroll
-            for (int q = 0; q < H::kPieces; ++q) gj += gs[((size_t)q * H::kNVars + j) * ld + t];
-            gj *= sw;
+            const double gj = gs[(size_t)j * ld + t] * sw;
             double dv[3], gg;
             xvalue<H, j>(x, dv, gg);
             constexpr int a1 = H::kVars[j].s1, a2 = H::kVars[j].s2;
@@ -784,77 +776,50 @@ __global__ void __launch_bounds__(1024) k_scan_int(const int* __restrict__ cnt, 
 // ---------------------------------------------------------------------------------------------
 // Host launchers
 
-#define MBXG_XPIECE(poly, k)                                                                           \
-    hipError_t launch_xpoly_##poly##_p##k(const double*, const int*, int, int, const double*, double*, \
-                                          double*, hipStream_t);
-MBXG_XPIECE(halide_h2o_2b, 0)
-MBXG_XPIECE(co2co2_2b, 0)
-MBXG_XPIECE(co2co2_2b, 1)
-MBXG_XPIECE(halide_h2o2_3b, 0)
-MBXG_XPIECE(halide_h2o2_3b, 1)
-MBXG_XPIECE(halide_h2o2_3b, 2)
-MBXG_XPIECE(halide_h2o2_3b, 3)
-MBXG_XPIECE(co2x3_3b, 0)
-MBXG_XPIECE(co2x3_3b, 1)
-MBXG_XPIECE(co2x3_3b, 2)
-MBXG_XPIECE(co2x3_3b, 3)
-MBXG_XPIECE(h2ox4_4b, 0)
-MBXG_XPIECE(h2ox4_4b, 1)
-MBXG_XPIECE(h2ox4_4b, 2)
-MBXG_XPIECE(h2ox4_4b, 3)
-MBXG_XPIECE(h2ox4_4b, 4)
-MBXG_XPIECE(h2ox4_4b, 5)
-MBXG_XPIECE(h2ox4_4b, 6)
-MBXG_XPIECE(h2ox4_4b, 7)
-MBXG_XPIECE(alkali_h2o_2b, 0)
-MBXG_XPIECE(alkali_h2o2_3b, 0)
-MBXG_XPIECE(alkali_h2o2_3b, 1)
-#undef MBXG_XPIECE
+// The polynomial structures (gen/xpoly_<structure>.hip).
+#define MBXG_XPOLY(poly)                                                                                       \
+    hipError_t launch_xpoly_##poly(const double*, const int*, int, int, const double*, double*, double*, int, \
+                                   hipStream_t);
+MBXG_XPOLY(halide_h2o_2b)
+MBXG_XPOLY(co2co2_2b)
+MBXG_XPOLY(halide_h2o2_3b)
+MBXG_XPOLY(co2x3_3b)
+MBXG_XPOLY(h2ox4_4b)
+MBXG_XPOLY(alkali_h2o_2b)
+MBXG_XPOLY(alkali_h2o2_3b)
+#undef MBXG_XPOLY
 
 namespace {
 
-typedef hipError_t (*xpiece_launch)(const double*, const int*, int, int, const double*, double*, double*, hipStream_t);
+typedef hipError_t (*xpoly_launch)(const double*, const int*, int, int, const double*, double*, double*, int,
+                                   hipStream_t);
 
 template <class H>
 size_t xworkspace(int cap) {
     const size_t ld = ((size_t)cap + 63) / 64 * 64;
-    return ((size_t)H::kNVars * (1 + H::kPieces) + H::kPieces + 1) * ld;
+    return ((size_t)H::kNVars * 2 + 2) * ld;
 }
 
 template <class H>
-hipError_t xlaunch(const xpiece_launch* pieces, const int* list, const int* n_dev, int cap, const NmerCtx& N,
-                   const double* coef, double* grad, double* e_out, double* partials, double* ws, hipStream_t st) {
+hipError_t xlaunch(xpoly_launch poly, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
+                   double* grad, double* e_out, double* partials, double* ws, hipStream_t st) {
     if (cap <= 0) return hipSuccess;
     const int nb = (cap + 63) / 64;
     const int ld = nb * 64;
     double* xs = ws;
     double* gs = xs + (size_t)H::kNVars * ld;
-    double* ps = gs + (size_t)H::kPieces * H::kNVars * ld;
-    double* sw = ps + (size_t)H::kPieces * ld;
+    double* ps = gs + (size_t)H::kNVars * ld;
+    double* sw = ps + ld;
     hipLaunchKernelGGL(k_xvars<H>, dim3(nb), dim3(64), 0, st, list, n_dev, cap, N, xs, sw, ld);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    for (int q = 0; q < H::kPieces; ++q) {
-        e = pieces[q](xs, n_dev, cap, ld, coef, gs + (size_t)q * H::kNVars * ld, ps + (size_t)q * ld, st);
-        if (e != hipSuccess) return e;
-    }
+    e = poly(xs, n_dev, cap, ld, coef, gs, ps, poly_split(cap, poly_wpe(H::kNVars)), st);
+    if (e != hipSuccess) return e;
     const int ngb = (cap + kGradBlockX - 1) / kGradBlockX;
     hipLaunchKernelGGL(k_xgrad<H>, dim3(ngb), dim3(kGradBlockX), 0, st, list, n_dev, cap, N, gs, ps, ld, grad, e_out,
                        partials);
     return hipGetLastError();
 }
-
-const xpiece_launch kPHalide2[1] = {launch_xpoly_halide_h2o_2b_p0};
-const xpiece_launch kPCo2_2[2] = {launch_xpoly_co2co2_2b_p0, launch_xpoly_co2co2_2b_p1};
-const xpiece_launch kPHalide3[4] = {launch_xpoly_halide_h2o2_3b_p0, launch_xpoly_halide_h2o2_3b_p1,
-                                    launch_xpoly_halide_h2o2_3b_p2, launch_xpoly_halide_h2o2_3b_p3};
-const xpiece_launch kPCo2_3[4] = {launch_xpoly_co2x3_3b_p0, launch_xpoly_co2x3_3b_p1, launch_xpoly_co2x3_3b_p2,
-                                  launch_xpoly_co2x3_3b_p3};
-const xpiece_launch kPH2o_4[8] = {launch_xpoly_h2ox4_4b_p0, launch_xpoly_h2ox4_4b_p1, launch_xpoly_h2ox4_4b_p2,
-                                  launch_xpoly_h2ox4_4b_p3, launch_xpoly_h2ox4_4b_p4, launch_xpoly_h2ox4_4b_p5,
-                                  launch_xpoly_h2ox4_4b_p6, launch_xpoly_h2ox4_4b_p7};
-const xpiece_launch kPAlkali2[1] = {launch_xpoly_alkali_h2o_2b_p0};
-const xpiece_launch kPAlkali3[2] = {launch_xpoly_alkali_h2o2_3b_p0, launch_xpoly_alkali_h2o2_3b_p1};
 
 }  // namespace
 
@@ -865,7 +830,7 @@ __host__ __device__ int xfam_order(int f) {
 
 size_t xfam_workspace(int f, int cap) {
     switch (f) {
-#define MBXG_XW(F, name, pieces) \
+#define MBXG_XW(F, name, poly) \
     case F: return xworkspace<XHolder_##name>(cap);
         MBXG_XFAMILIES(MBXG_XW)
 #undef MBXG_XW
@@ -876,8 +841,8 @@ size_t xfam_workspace(int f, int cap) {
 hipError_t launch_xfam(int f, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
                        double* grad, double* e_out, double* partials, double* ws, hipStream_t st) {
     switch (f) {
-#define MBXG_XL(F, name, pieces) \
-    case F: return xlaunch<XHolder_##name>(pieces, list, n_dev, cap, N, coef, grad, e_out, partials, ws, st);
+#define MBXG_XL(F, name, poly) \
+    case F: return xlaunch<XHolder_##name>(launch_xpoly_##poly, list, n_dev, cap, N, coef, grad, e_out, partials, ws, st);
         MBXG_XFAMILIES(MBXG_XL)
 #undef MBXG_XL
         default: return hipErrorInvalidValue;
@@ -941,9 +906,19 @@ hipError_t launch_tetra(const PtInfo* pinfo, const double* cx, const double* cy,
     return hipGetLastError();
 }
 
+const char* xfam_structure(int f) {
+    switch (f) {
+#define MBXG_XS(F, name, poly) \
+    case F: return #poly;
+        MBXG_XFAMILIES(MBXG_XS)
+#undef MBXG_XS
+        default: return "";
+    }
+}
+
 const double* xfam_default_coef(int f, int* n) {
     switch (f) {
-#define MBXG_XC(F, name, pieces) \
+#define MBXG_XC(F, name, poly) \
     case F:                      \
         *n = kNCoefX_##name;     \
         return kFitX_##name;

@@ -45,6 +45,7 @@ struct XLists {
 __host__ __device__ int xfam_order(int f);
 size_t xfam_workspace(int f, int cap);  // doubles
 const double* xfam_default_coef(int f, int* n);
+const char* xfam_structure(int f);  // the polynomial structure's name (its table of mbx_amd/tables)
 size_t xclass_blocks(int n);
 
 // Classification of n listed n-mers of one order: code[n], per-block counts blk / offsets

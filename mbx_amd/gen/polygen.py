@@ -329,8 +329,12 @@ def adapted(name):
 NPARTS = 8
 
 
+WRITTEN = set()
+
+
 def write_if_changed(path, text):
     """Write only when the content differs, so make does not rebuild unchanged kernels."""
+    WRITTEN.add(os.path.basename(path))
     try:
         if open(path).read() == text:
             return
@@ -350,41 +354,9 @@ def coef_source(name, coef):
     return "\n".join(out) + "\n"
 
 
-# MB-nrg polynomials: each piece is its own translation unit (compiled in parallel) with its
-# own kernel writing a partial value and gradient; the chain-rule stage sums the pieces.  The
-# CH4-H2O-H2O 3B polynomial instead takes the blocked form of the MB-pol ones (generate(): one
-# translation unit, NPARTS parts shared by the wavefronts of a block, one output slice).
-NRG_PARTS = {"ch4h2o_2b": 1, "ch4ch4_2b": 8}
-NRG_BLOCKED = ("ch4h2o2_3b",)
-
-
-def generate_nrg(name, out_dir):
-    nvars, coef, monos = load_table(name)
-    s = Schedule(nvars, [(k, m) for k, m in monos])
-    q = NRG_PARTS[name]
-    assign = s.partition(q)
-    c = s.counts()
-    for k in range(q):
-        hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
-               "// Schedule: %s" % ", ".join("%s=%d" % kv for kv in c.items()),
-               "// Piece %d of %d (op-count balance: %s)." % (k, q, ", ".join(str(v) for v in s.part_load)),
-               "#pragma once", "#include \"poly_support.hpp\"", ""]
-        src = "\n".join(hdr) + s.emit("poly_%s_p%d" % (name, k), grad=True, part=k, assign=assign) + "\n" + \
-            s.emit("poly_%s_e_p%d" % (name, k), grad=False, part=k, assign=assign)
-        write_if_changed(os.path.join(out_dir, "poly_%s_p%d.inc" % (name, k)), src)
-        tu = ["// GENERATED by mbx_amd/gen/polygen.py -- do not edit.",
-              "// Piece %d of %d of the %s polynomial (%d variables): its own kernel, so the pieces "
-              "compile in parallel." % (k, q, name, nvars),
-              "#include \"gen/poly_%s_p%d.inc\"" % (name, k), "#include \"nrg_kernel.hpp\"", "",
-              "namespace mbxg {", "",
-              "hipError_t launch_poly_%s_p%d(const double* xs, const int* n_dev, int cap, int ld, const double* coef, "
-              "int do_grads, double* gs, double* ps, hipStream_t st) {" % (name, k),
-              "    return launch_poly_piece<%d, poly_%s_p%d, poly_%s_e_p%d>(xs, n_dev, cap, ld, coef, do_grads, gs, ps, "
-              "st);" % (nvars, name, k, name, k),
-              "}", "", "}  // namespace mbxg", ""]
-        write_if_changed(os.path.join(out_dir, "poly_%s_p%d.hip" % (name, k)), "\n".join(tu))
-    write_if_changed(os.path.join(out_dir, "coef_%s.inc" % name), coef_source(name, coef))
-    return c
+# MB-nrg polynomials in the blocked form (generate_blocked(): a translation unit of its own each, so they
+# compile in parallel).  CH4-H2O-H2O has its launcher in poly_ch4h2o2_3b.hip.
+NRG_BLOCKED = ("ch4h2o_2b", "ch4ch4_2b", "ch4h2o2_3b")
 
 
 def generate_holder(name, out_dir):
@@ -413,7 +385,6 @@ def generate_holder(name, out_dir):
            "    static constexpr double kRIn = %.17g;" % h["switch"]["inner"],
            "    static constexpr double kROut = %.17g;" % h["switch"]["outer"],
            "    static constexpr int kNVars = %d;" % len(h["vars"]),
-           "    static constexpr int kPieces = %d;" % NRG_PARTS.get(name, 1),
            "    static constexpr NrgVar kVars[%d] = {" % len(h["vars"])]
     for f, k, d, s1, s2 in h["vars"]:
         out.append("        {%d, %.17g, %.17g, %d, %d}," % (forms[f], k, d, s1, s2))
@@ -421,21 +392,25 @@ def generate_holder(name, out_dir):
     write_if_changed(os.path.join(out_dir, "holder_%s.inc" % name), "\n".join(out))
 
 
-def generate(name, fn, out_dir):
+def blocked_source(name, fn, energy_only=True):
+    """The .inc of a polynomial in symmetry-adapted coordinates, cut into NPARTS parts."""
     nvars, coef, sym = adapted(name)
-    s = Schedule(nvars, sym.terms)
+    deep = max(len(m) for _, m in sym.terms) > 4
+    s = (TrieSchedule if deep else Schedule)(nvars, sym.terms)
+    assign = s.partition(NPARTS)
     c = s.counts()
     hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
            "// Schedule: %s" % ", ".join("%s=%d" % kv for kv in c.items()),
+           "// %d parts (op-count balance: %s); <fn>_parts(w, P, ...) evaluates parts w, w+P, ... "
+           "into g and returns their share of the value." % (NPARTS, ", ".join(str(v) for v in s.part_load)),
            "// Symmetry-adapted coordinates: %s_sym transforms x before and g after; C holds %d slots "
            "(gen/sym_%s.inc)." % (fn, len(sym.rows) + len(sym.low), name),
            "#pragma once",
            "#include \"poly_support.hpp\"", ""]
-    assign = s.partition(NPARTS)
-    hdr.insert(2, "// %d parts (op-count balance: %s); <fn>_parts(w, P, ...) evaluates parts w, w+P, ... "
-                  "into g and returns their share of the value." % (NPARTS, ", ".join(str(v) for v in s.part_load)))
     body = [symmetry.emit_transform(fn + "_sym", sym.blocks)]
     for grad, suffix in ((True, ""), (False, "_e")):
+        if not grad and not energy_only:
+            continue
         for k in range(NPARTS):
             body.append(s.emit("%s%s_p%d" % (fn, suffix, k), grad=grad, part=k, assign=assign))
         args, call = (("mbxg_cptr C, const double* x, double* g", "C, x, g, E") if grad
@@ -448,7 +423,12 @@ def generate(name, fn, out_dir):
             d.append("    if (%d %% P == w) E = %s%s_p%d(%s);" % (k, fn, suffix, k, call))
         d += ["    return E;", "}", ""]
         body.append("\n".join(d))
-    src = "\n".join(hdr) + "\n".join(body)
+    return "\n".join(hdr) + "\n".join(body), c
+
+
+def generate(name, fn, out_dir):
+    _, coef, sym = adapted(name)
+    src, c = blocked_source(name, fn)
     path = os.path.join(out_dir, "poly_%s.inc" % name)
     write_if_changed(path, src)
     # fitted coefficients, for the host runtime's default table
@@ -456,6 +436,35 @@ def generate(name, fn, out_dir):
     write_if_changed(os.path.join(out_dir, "sym_%s.inc" % name),
                      symmetry.emit_tables(name, sym, len(coef), name in AD_POLYS))
     return path, c
+
+
+def waves_per_simd(nvars):
+    """Wavefronts per SIMD of a value + gradient kernel: x and g take 4 registers a variable, the trie
+    about 24, of 512 registers a lane and SIMD."""
+    return max(1, min(4, 512 // (4 * nvars + 24)))
+
+
+def generate_launcher(prefix, name, out_dir, energy_only):
+    """gen/<prefix><name>.hip: the launcher of a blocked polynomial, a translation unit of its own."""
+    nvars = load_table(name)[0]
+    fn = prefix + name
+    wpe = waves_per_simd(nvars)
+    out = ["// GENERATED by mbx_amd/gen/polygen.py -- do not edit.",
+           "// The %s polynomial (%d variables): its own translation unit, %d wavefronts per SIMD." % (name, nvars, wpe),
+           "#include \"gen/%s.inc\"" % fn, "#include \"poly_kernel.hpp\"", "", "namespace mbxg {", ""]
+    if energy_only:
+        out += ["hipError_t launch_%s(const double* xs, const int* n_dev, int cap, int ld, const double* coef, int do_grads," % fn,
+                "    double* gs, double* ps, int P, hipStream_t st) {",
+                "    return launch_poly<%d, %d, %s_parts, %s_e_parts, %s_sym, %d>(xs, n_dev, cap, ld, coef, do_grads, gs, ps," % (
+                    nvars, NPARTS, fn, fn, fn, wpe),
+                "        P, st);", "}"]
+    else:
+        out += ["hipError_t launch_%s(const double* xs, const int* n_dev, int cap, int ld, const double* coef, double* gs," % fn,
+                "    double* ps, int P, hipStream_t st) {",
+                "    return launch_poly_eg<%d, %d, %s_parts, %s_sym, %d>(xs, n_dev, cap, ld, coef, gs, ps, P, st);" % (
+                    nvars, NPARTS, fn, fn, wpe), "}"]
+    out += ["", "}  // namespace mbxg", ""]
+    write_if_changed(os.path.join(out_dir, fn + ".hip"), "\n".join(out))
 
 
 # ------------------------------------------------------------------------------------------
@@ -822,82 +831,116 @@ def generate_1b(name, out_dir):
 # ------------------------------------------------------------------------------------------
 # Further MB-nrg families (halide-water 2B / 3B, CO2 2B / 3B, water 4B, alkali-ion-water 2B / 3B):
 # holders as data (gen/xholder_<holder>.inc), each parameter set's coefficients
-# (gen/xcoef_<holder>.inc) and the polynomial structures in pieces (gen/xpoly_<structure>_p<k>.{inc,hip},
-# one kernel each).
+# (gen/xcoef_<holder>.inc) and the polynomial structures (gen/xpoly_<structure>.{inc,hip}).
 ALKALI = ("li", "na", "k", "rb", "cs")
 XHOLDERS = ("f_h2o_2b", "cl_h2o_2b", "br_h2o_2b", "i_h2o_2b", "f_h2o2_3b", "cl_h2o2_3b", "br_h2o2_3b", "i_h2o2_3b",
             "co2co2_2b", "co2x3_3b", "h2ox4_4b") + tuple("%s_h2o_2b" % a for a in ALKALI) + \
     tuple("%s_h2o2_3b" % a for a in ALKALI)
-XPOLY_PIECES = {"halide_h2o_2b": 1, "co2co2_2b": 2, "halide_h2o2_3b": 4, "co2x3_3b": 4, "h2ox4_4b": 8,
-                "alkali_h2o_2b": 1, "alkali_h2o2_3b": 2}
+XPOLYS = ("halide_h2o_2b", "co2co2_2b", "halide_h2o2_3b", "co2x3_3b", "h2ox4_4b", "alkali_h2o_2b", "alkali_h2o2_3b")
 XKIND = {"h2o": "MON_H2O", "ch4": "MON_CH4", "co2": "MON_CO2", "f-": "MON_F", "cl-": "MON_CL", "br-": "MON_BR",
          "i-": "MON_I", "li+": "MON_LI", "na+": "MON_NA", "k+": "MON_K", "rb+": "MON_RB", "cs+": "MON_CS"}
 
 
-def emit_trie_piece(fn, nvars, monos, fence_every=48):
-    """emit_trie for monomials of any degree as a piece function (mbxg_cptr coefficients, value
-    returned on top of E0), with a region fence every `fence_every` statements so coefficient
-    loads stay near their FMAs."""
-    body = emit_trie(fn + "_trie", nvars, monos).replace("const double* __restrict__ C", "mbxg_cptr C")
-    lines = body.split("\n")
-    out, n, last = [], 0, "x[0]"
-    for ln in lines:
-        out.append(ln)
-        m = re.match(r"\s+(?:const )?double (\w+) = ", ln) or re.match(r"\s+(\w+) = __fma_rn", ln)
-        if m:
-            last = m.group(1)
-            n += 1
-            if n % fence_every == 0:
-                out.append("    MBXG_NODE_FENCE(C, %s);" % last)
-    src = "\n".join(out)
-    src += ("__device__ __forceinline__ double %s(mbxg_cptr C, const double* x, double* g, double E0) {\n"
-            "    return E0 + %s_trie(C, x, g);\n}\n" % (fn, fn))
-    return src
+class TrieSchedule:
+    """Terms of any degree in reverse mode over the full monomial trie (as emit_trie), with the parts
+    interface of Schedule: a part is a set of level-2 subtrees, each level-1 node's own terms and the
+    terms of degree 0.  A second coefficient of a monomial (symmetry.py) is applied where its node meets
+    its parent, so it is not rounded away against the first."""
+
+    def __init__(self, nvars, terms):
+        self.nvars = nvars
+        self.coef = collections.defaultdict(list)
+        for q, m in terms:
+            self.coef[tuple(sorted(m))].append(q)
+        self.children = collections.defaultdict(set)
+        for m in self.coef:
+            for d in range(1, len(m) + 1):
+                self.children[m[:d - 1]].add(m[d - 1])
+
+    def _size(self, node):
+        return 2 * len(self.coef.get(node, [])) + sum(3 + self._size(node + (v,)) for v in self.children.get(node, ()))
+
+    def counts(self):
+        n = sum(len(v) for v in self.children.values())
+        second = sum(len(q) - 1 for q in self.coef.values())
+        return dict(nodes=n, monomials=len(self.coef), second=second, fp64_ops_eg=3 * n + 2 * second)
+
+    def partition(self, nparts):
+        items = [(1, ())]
+        for v in self.children[()]:
+            items.append((4, (v,)))
+            items += [(4 + self._size((v, w)), (v, w)) for w in self.children.get((v,), ())]
+        load, assign = [0] * nparts, {}
+        for c, it in sorted(items, key=lambda t: (-t[0], t[1])):
+            k = min(range(nparts), key=lambda j: (load[j], j))
+            assign[it] = k
+            load[k] += c
+        self.part_load = load
+        return assign
+
+    def emit(self, fn, grad=True, part=None, assign=None, fence_every=48):
+        assert grad
+        out = ["__device__ __forceinline__ double %s(mbxg_cptr C, const double* x, double* g, double E0) {" % fn,
+               "    double E = E0;"]
+        count = [0]
+
+        def w(t, result=None):
+            out.append("    " + t)
+            if result:
+                count[0] += 1
+                if count[0] % fence_every == 0:
+                    out.append("    MBXG_NODE_FENCE(C, %s);" % result)
+
+        names = [0]
+
+        def walk(node, product, own=True, kids=None):
+            """Statements of the subtree; returns the name of its adjoint R."""
+            names[0] += 1
+            r = "R%d" % names[0]
+            q = self.coef.get(node, []) if own else []
+            w("double %s = %s;" % (r, "C[%d]" % q[0] if q else "0.0"), r)
+            for v in sorted(self.children.get(node, ()) if kids is None else kids):
+                child = node + (v,)
+                pc = None
+                if self.children.get(child):
+                    names[0] += 1
+                    pc = "P%d" % names[0]
+                    w("const double %s = %s;" % (pc, "%s * x[%d]" % (product, v)))
+                meet(child, v, walk(child, pc), r, product)
+            return r
+
+        def meet(child, v, rc, r, product):
+            """The child's adjoint, and its monomial's second coefficients, into g and the parent's r."""
+            for c in [rc] + ["C[%d]" % q for q in self.coef.get(child, [])[1:]]:
+                w("g[%d] = __fma_rn(%s, %s, g[%d]);" % (v, product, c, v))
+                w("%s = __fma_rn(x[%d], %s, %s);" % (r, v, c, r), r)
+
+        if assign[()] == part:
+            for q in self.coef.get((), []):
+                w("E += C[%d];" % q)
+        for v in sorted(self.children[()]):
+            kids = [u for u in self.children.get((v,), ()) if assign[(v, u)] == part]
+            own = assign[(v,)] == part
+            if not kids and not own:
+                continue
+            rc = walk((v,), "x[%d]" % v, own, kids)
+            w("g[%d] += %s;" % (v, rc))
+            w("E = __fma_rn(x[%d], %s, E);" % (v, rc))
+            for q in self.coef.get((v,), [])[1:] if own else []:
+                w("g[%d] += C[%d];" % (v, q))
+                w("E = __fma_rn(x[%d], C[%d], E);" % (v, q))
+        w("return E;")
+        out.append("}")
+        return "\n".join(out) + "\n"
 
 
 def generate_xpoly(name, out_dir):
-    nvars, coef, monos = load_table(name)
-    q = XPOLY_PIECES[name]
-    deg = max(len(m) for _, m in monos)
-    hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
-           "#pragma once", "#include \"poly_support.hpp\"", ""]
-    if deg > 4:
-        assert q == 1 or name == "co2co2_2b"
-        # degree 5-6: reverse mode over the full monomial trie, split by the first variable
-        firsts = sorted({m[0] for _, m in monos})
-        load = [0] * q
-        groups = [[] for _ in range(q)]
-        for v in sorted(firsts, key=lambda v: -sum(1 for _, m in monos if m[0] == v)):
-            k = min(range(q), key=lambda j: load[j])
-            groups[k].append(v)
-            load[k] += sum(1 for _, m in monos if m[0] == v)
-        parts = [[(k, m) for k, m in monos if m[0] in set(g)] for g in groups]
-        for k in range(q):
-            src = "\n".join(hdr) + "// Piece %d of %d: the monomials whose first variable is one of %s (%d of %d).\n" % (
-                k, q, groups[k], len(parts[k]), len(monos)) + emit_trie_piece("xpoly_%s_p%d" % (name, k), nvars,
-                                                                            parts[k])
-            write_if_changed(os.path.join(out_dir, "xpoly_%s_p%d.inc" % (name, k)), src)
-    else:
-        s = Schedule(nvars, [(k, m) for k, m in monos])
-        assign = s.partition(q)
-        c = s.counts()
-        for k in range(q):
-            src = "\n".join(hdr) + "// Schedule: %s\n// Piece %d of %d (op-count balance: %s).\n" % (
-                ", ".join("%s=%d" % kv for kv in c.items()), k, q, ", ".join(str(v) for v in s.part_load)) + \
-                s.emit("xpoly_%s_p%d" % (name, k), grad=True, part=k, assign=assign)
-            write_if_changed(os.path.join(out_dir, "xpoly_%s_p%d.inc" % (name, k)), src)
-    for k in range(q):
-        tu = ["// GENERATED by mbx_amd/gen/polygen.py -- do not edit.",
-              "// Piece %d of %d of the %s polynomial (%d variables, degree %d): its own kernel." % (
-                  k, q, name, nvars, deg),
-              "#include \"gen/xpoly_%s_p%d.inc\"" % (name, k), "#include \"nrg_kernel.hpp\"", "",
-              "namespace mbxg {", "",
-              "hipError_t launch_xpoly_%s_p%d(const double* xs, const int* n_dev, int cap, int ld, const double* coef, "
-              "double* gs, double* ps, hipStream_t st) {" % (name, k),
-              "    return launch_xpoly_piece<%d, xpoly_%s_p%d>(xs, n_dev, cap, ld, coef, gs, ps, st);" % (nvars, name, k),
-              "}", "", "}  // namespace mbxg", ""]
-        write_if_changed(os.path.join(out_dir, "xpoly_%s_p%d.hip" % (name, k)), "\n".join(tu))
-    return dict(pieces=q, degree=deg, monomials=len(monos))
+    src, c = blocked_source(name, "xpoly_" + name, energy_only=False)
+    write_if_changed(os.path.join(out_dir, "xpoly_%s.inc" % name), src)
+    generate_launcher("xpoly_", name, out_dir, False)
+    _, coef, sym = adapted(name)
+    write_if_changed(os.path.join(out_dir, "sym_%s.inc" % name), symmetry.emit_tables(name, sym, len(coef)))
+    return c
 
 
 def generate_xholder(name, out_dir):
@@ -936,7 +979,6 @@ def generate_xholder(name, out_dir):
            "    static constexpr int kTMask[%d] = {%s};" % (len(sw["terms"]), ", ".join(
                str(sum(1 << q for q in t[1])) for t in sw["terms"])),
            "    static constexpr int kNVars = %d;" % len(h["vars"]),
-           "    static constexpr int kPieces = %d;" % XPOLY_PIECES[h["poly"]],
            "    static constexpr NrgVar kVars[%d] = {" % len(h["vars"])]
     for f, k, d, s1, s2 in h["vars"]:
         out.append("        {%d, %.17g, %.17g, %d, %d}," % (forms[f], k, d, s1, s2))
@@ -960,19 +1002,22 @@ def main():
         print(path, c)
     for name in AD_POLYS:
         generate_ad(name, out_dir)
-    for name in NRG_PARTS:
-        print(name, generate_nrg(name, out_dir))
-        generate_holder(name, out_dir)
     for name in NRG_BLOCKED:
         print(generate(name, "poly_" + name, out_dir))
         generate_holder(name, out_dir)
+        if name != "ch4h2o2_3b":
+            generate_launcher("poly_", name, out_dir, True)
     print(generate_ps(out_dir))
     for name in ONE_BODY:
         print(name, generate_1b(name, out_dir))
     for name in XHOLDERS:
         generate_xholder(name, out_dir)
-    for name in XPOLY_PIECES:
+    for name in XPOLYS:
         print(name, generate_xpoly(name, out_dir))
+    # what earlier versions generated under the untracked names would still be compiled
+    for f in os.listdir(out_dir):
+        if f.startswith(("poly_ch4", "xpoly_", "ad_", "sym_")) and f not in WRITTEN:
+            os.remove(os.path.join(out_dir, f))
 
 
 if __name__ == "__main__":

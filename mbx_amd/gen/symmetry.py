@@ -48,13 +48,17 @@ EXCHANGES = {
     "ch4h2o_2b": [[(1, 2)], [(8, 9)]] + _methane(3),
     "ch4ch4_2b": _methane(0) + _methane(5),
     "ch4h2o2_3b": _methane(0) + [[(6, 7)], [(9, 10)]],
+    "halide_h2o_2b": [[(2, 3)], [(4, 5)]],
+    "alkali_h2o_2b": [[(1, 2)], [(4, 5)]],
+    "co2co2_2b": _WATERS[2],
     "halide_h2o2_3b": [[(2, 3)], [(5, 6)], [(7, 8)], [(9, 10)]],
     "alkali_h2o2_3b": _WATERS[2],
     "co2x3_3b": _WATERS[3],
     "h2ox4_4b": _WATERS[4],
 }
 # a holder with the structure's variables, where the structure serves several
-_HOLDER = {"halide_h2o2_3b": "cl_h2o2_3b", "alkali_h2o2_3b": "na_h2o2_3b"}
+_HOLDER = {"halide_h2o_2b": "cl_h2o_2b", "alkali_h2o_2b": "na_h2o_2b", "halide_h2o2_3b": "cl_h2o2_3b",
+           "alkali_h2o2_3b": "na_h2o2_3b"}
 
 # MB-pol: (rate, offset, Coulomb-like) of each variable class (2B x2b-v9x.cpp:1330-1345, 3B x3b-v2x.cpp:1256-1271)
 _MBPOL_CLASS = {
