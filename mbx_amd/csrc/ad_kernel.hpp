@@ -11,6 +11,10 @@
 // tangent), coefficients in slices (grid.y = slice).  Each block writes one row of per-block
 // partial sums; k_ad_colsum adds the rows in a fixed order, so the result is deterministic.
 //
+// Both work in symmetry-adapted coordinates (SYM, as in poly_kernel.hpp): "coefficient k" is a slot,
+// H xd goes back to the variables by the same transform.  Like the polynomials they are bound by the
+// monomials' FP64 operations (MB-pol 3B: 6,773 monomials instead of 33,525).
+//
 // Buffers are variable-major: entry (j, t) at j*ld + t.
 #pragma once
 
@@ -47,8 +51,9 @@ __device__ __forceinline__ void ad_opaque(double* x, double* xd) {
 
 typedef void (*ad_tan_fn)(int, mbxg_cptr, const double*, const double*, double*);
 typedef void (*ad_basis_fn)(int, double*, double*, double, double, double*, double*, int);
+typedef void (*ad_sym_fn)(double*);
 
-template <int NV, int PARTS, ad_tan_fn FN>
+template <int NV, int PARTS, ad_tan_fn FN, ad_sym_fn SYM>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_ad_tan(const double* __restrict__ xs, const double* __restrict__ xds, int n, int ld, uint64_t coef_addr,
              double* __restrict__ gds) {
@@ -63,14 +68,17 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         xd[j] = xds[(size_t)j * ld + t];
         gd[j] = 0.0;
     }
+    SYM(x);
+    SYM(xd);
     FN(part, C, x, xd, gd);
+    SYM(gd);
     const size_t base = (size_t)part * NV * ld;
 #pragma unroll
     for (int j = 0; j < NV; ++j) gds[base + (size_t)j * ld + t] = gd[j];
 }
 
 // alpha_n = g_energy_n * sw_n + dsw_n (the weight of M_k), sw_n (the weight of dM_k).
-template <int NV, int NCOEF, ad_basis_fn FN>
+template <int NV, int NCOEF, ad_basis_fn FN, ad_sym_fn SYM>
 __global__ void __launch_bounds__(64) k_ad_basis(const double* __restrict__ xs, const double* __restrict__ xds,
                                                  const double* __restrict__ sw, const double* __restrict__ swd,
                                                  const double* __restrict__ g_energy, int n, int ld,
@@ -87,6 +95,8 @@ __global__ void __launch_bounds__(64) k_ad_basis(const double* __restrict__ xs, 
     }
     const double s = active ? sw[t] : 0.0;
     const double alpha = active ? g_energy[t] * s + swd[t] : 0.0;
+    SYM(x);
+    SYM(xd);
     FN(blockIdx.y, x, xd, alpha, s, red, partial + (size_t)blockIdx.x * NCOEF, lane);
 }
 

@@ -87,6 +87,14 @@ __device__ __forceinline__ double ad_slot(const int* row, const unsigned short* 
     return q < nrow ? b : err - (b - s);
 }
 
+// Entry k of the transposed map: the fitted coefficient's gradient from the slots' (row[q]).
+__device__ __forceinline__ double ad_coef_adjoint(const int* start, const unsigned short* slot, const double* w, int k,
+                                                  const double* __restrict__ row) {
+    double s = 0.0;
+    for (int i = start[k]; i < start[k + 1]; ++i) s = __fma_rn(row[slot[i]], w[i], s);
+    return s;
+}
+
 // Sites 0..5 = Oa Ha1 Ha2 Ob Hb1 Hb2, 6..9 = Xa1 Xa2 Xb1 Xb2 (x2b-v9x.cpp:1640-1675).
 struct Ad2b {
     static constexpr int kNV = 31, kNAt = 6, kNS = 10, kPairs = 1, kParts = kAdParts;
@@ -105,6 +113,10 @@ struct Ad2b {
     static constexpr int kNSlot = kNSlot_mbpol_2b;
     static __device__ __forceinline__ double slot(int q, const double* __restrict__ coef) {
         return ad_slot(kSymRow_mbpol_2b, kSymK_mbpol_2b, kSymW_mbpol_2b, kSymLow_mbpol_2b, kNRow_mbpol_2b, q, coef);
+    }
+    static constexpr int kNRow = kNRow_mbpol_2b;
+    static __device__ __forceinline__ double coef_adjoint(int k, const double* __restrict__ row) {
+        return ad_coef_adjoint(kSymTRow_mbpol_2b, kSymTK_mbpol_2b, kSymTW_mbpol_2b, k, row);
     }
 };
 
@@ -128,6 +140,10 @@ struct Ad3b {
     static constexpr int kNSlot = kNSlot_mbpol_3b;
     static __device__ __forceinline__ double slot(int q, const double* __restrict__ coef) {
         return ad_slot(kSymRow_mbpol_3b, kSymK_mbpol_3b, kSymW_mbpol_3b, kSymLow_mbpol_3b, kNRow_mbpol_3b, q, coef);
+    }
+    static constexpr int kNRow = kNRow_mbpol_3b;
+    static __device__ __forceinline__ double coef_adjoint(int k, const double* __restrict__ row) {
+        return ad_coef_adjoint(kSymTRow_mbpol_3b, kSymTK_mbpol_3b, kSymTW_mbpol_3b, k, row);
     }
 };
 
@@ -534,6 +550,17 @@ __global__ void __launch_bounds__(64) k_ad_colsum(const double* __restrict__ par
     if (threadIdx.x == 0) out[k] = s;
 }
 
+// The fitted coefficients' gradient from the blocks' slot gradients partial[nrows][F::kNRow]: one
+// wavefront per coefficient, rows 64 at a time, summed as in k_ad_colsum.
+template <class F>
+__global__ void __launch_bounds__(64) k_ad_coef_sum(const double* __restrict__ partial, int nrows,
+                                                    double* __restrict__ out) {
+    double s = 0.0;
+    for (int r = threadIdx.x; r < nrows; r += 64) s += F::coef_adjoint(blockIdx.x, partial + (size_t)r * F::kNRow);
+    s = wave_sum(s);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
 // Sum the parts' slices of the gradient tangent into slice 0 (entry e of part q at
 // q * rows + e, rows = nv * ld).  One thread per entry, parts added in order.
 __global__ void __launch_bounds__(256) k_ad_sum_parts(double* __restrict__ gds, size_t rows, int parts) {
@@ -595,7 +622,7 @@ AdLayout ad_layout(int nv, int ncoef, int n) {
     L.ps = take(sizeof(double) * ld);
     L.ndev = take(sizeof(int));
     L.slots = take(sizeof(double) * kMaxSlots);
-    L.basis = take(sizeof(double) * nblk * ncoef);
+    L.basis = take(sizeof(double) * nblk * kMaxSlots);
     L.theta = take(sizeof(double) * nblk * 16);
     L.total = o;
     return L;
@@ -823,22 +850,23 @@ extern "C" int mbxg_ad_backward(int family, int n, const double* xyz, const doub
         hipLaunchKernelGGL((k_ad_vars<Ad2b, true>), vars_grid<Ad2b>(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, coef, xs,
                            xds, sw, swd, slots, ndev);
         if (!from_forward) ADCHK(launch_poly_mbpol2b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
-        ADCHK(launch_ad_tan_mbpol_2b(xs, xds, n, ld, coef, gds, st));
+        ADCHK(launch_ad_tan_mbpol_2b(xs, xds, n, ld, slots, gds, st));
         ADCHK(launch_ad_basis_mbpol_2b(xs, xds, sw, swd, g_energy, n, ld, basis, st));
         hipLaunchKernelGGL(k_ad_sum_parts, dim3((rows + 255) / 256), dim3(256), 0, st, gds, rows, Ad2b::kParts);
         hipLaunchKernelGGL((k_ad_chain<Ad2b, true>), dim3(nb), dim3(64), 0, st, xyz, g_grad, theta, g_energy, n, ld, 1,
                            gs, gds, ps, xds, nullptr, d_xyz, thp);
+        hipLaunchKernelGGL(k_ad_coef_sum<Ad2b>, dim3(ncoef), dim3(64), 0, st, basis, nb, d_coef);
     } else {
         hipLaunchKernelGGL((k_ad_vars<Ad3b, true>), vars_grid<Ad3b>(nb), dim3(64), 0, st, xyz, g_grad, theta, n, ld, coef, xs,
                            xds, sw, swd, slots, ndev);
         if (!from_forward) ADCHK(launch_poly_mbpol3b(xs, ndev, n, ld, slots, 1, gs, ps, 8, st));
-        ADCHK(launch_ad_tan_mbpol_3b(xs, xds, n, ld, coef, gds, st));
+        ADCHK(launch_ad_tan_mbpol_3b(xs, xds, n, ld, slots, gds, st));
         ADCHK(launch_ad_basis_mbpol_3b(xs, xds, sw, swd, g_energy, n, ld, basis, st));
         hipLaunchKernelGGL(k_ad_sum_parts, dim3((rows + 255) / 256), dim3(256), 0, st, gds, rows, Ad3b::kParts);
         hipLaunchKernelGGL((k_ad_chain<Ad3b, true>), dim3(nb), dim3(64), 0, st, xyz, g_grad, theta, g_energy, n, ld, 1,
                            gs, gds, ps, xds, nullptr, d_xyz, thp);
+        hipLaunchKernelGGL(k_ad_coef_sum<Ad3b>, dim3(ncoef), dim3(64), 0, st, basis, nb, d_coef);
     }
-    hipLaunchKernelGGL(k_ad_colsum, dim3(ncoef), dim3(64), 0, st, basis, nb, ncoef, ncoef, d_coef);
     hipLaunchKernelGGL(k_ad_colsum, dim3(kNTheta), dim3(64), 0, st, thp, nb, kNTheta, 16, d_theta);
     ADCHK(hipGetLastError());
     return MBXG_OK;

@@ -474,7 +474,9 @@ def generate_launcher(prefix, name, out_dir, energy_only):
 # the variables, (i) P, dP = grad P . xd, grad P and d(grad P) = H xd (forward-over-reverse:
 # the reverse-mode trie schedule above, every value carried with its tangent), and (ii) the
 # coefficient gradient sum_n [alpha_n M_k(x_n) + sw_n dM_k(x_n; xd_n)], where M_k is the
-# basis function of coefficient k (the sum of its monomials) and dM_k its tangent.
+# basis function of coefficient k (the sum of its monomials) and dM_k its tangent.  Both are generated
+# in symmetry-adapted coordinates (k: a slot), with x and xd transformed first; the gradient of the
+# fitted coefficients is the transpose of the slots' map.
 
 _DECL = re.compile(r"^(const )?double (\w+) = (.*);$")
 _FMA = re.compile(r"^(\S+) = __fma_rn\((.*)\);$")
@@ -669,16 +671,19 @@ AD_POLYS = {"mbpol_2b": 16, "mbpol_3b": 16}  # name -> basis slices
 def generate_ad(name, out_dir):
     """gen/ad_<name>_tan.{inc,hip} and gen/ad_<name>_basis.{inc,hip}: two translation units
     (compiled in parallel), each with its kernel's launcher."""
-    nvars, coef, monos = load_table(name)
-    s = Schedule(nvars, [(k, m) for k, m in monos])
+    nvars, coef, sym = adapted(name)
+    s = Schedule(nvars, sym.terms)
     assign = s.partition(AD_PARTS)
     fn = "ad_%s" % name
-    sl = basis_slices(monos, len(coef), AD_POLYS[name])
+    nrow = len(sym.rows)
+    monos = [(q, m) for q, m in sym.terms if q < nrow]
+    sl = basis_slices(monos, nrow, AD_POLYS[name])
     head = lambda what: ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
                          "// %s" % what, "#pragma once", "#include \"poly_support.hpp\"", "#include \"ad_kernel.hpp\"",
                          "", "namespace mbxg {", ""]
     # gradient tangent (Hessian-vector product), AD_PARTS parts
     body = [emit_dual(s, "%s_tan_p%d" % (fn, k), k, assign, tangent_only=True) for k in range(AD_PARTS)]
+    body.insert(0, symmetry.emit_transform("%s_tan_sym" % fn, sym.blocks))
     d = ["__device__ __forceinline__ void %s_tan(int part, mbxg_cptr C, const double* x, const double* xd, "
          "double* gd) {" % fn]
     d += ["    if (part == %d) %s_tan_p%d(C, x, xd, gd);" % (k, fn, k) for k in range(AD_PARTS)]
@@ -687,18 +692,19 @@ def generate_ad(name, out_dir):
                      "\n".join(head("Gradient tangent of the polynomial (H xd) in %d parts." % AD_PARTS))
                      + "\n".join(body) + "\n".join(d))
     # coefficient basis, in slices of near-equal cost
-    body = [emit_basis("%s_basis_s%d" % (fn, i), monos, c0, c1) for i, (c0, c1) in enumerate(sl)]
+    body = [symmetry.emit_transform("%s_basis_sym" % fn, sym.blocks)]
+    body += [emit_basis("%s_basis_s%d" % (fn, i), monos, c0, c1) for i, (c0, c1) in enumerate(sl)]
     d = ["__device__ __forceinline__ void %s_basis(int slice, double* x, double* xd, double alpha, "
          "double sw, double* red, double* out, int lane) {" % fn]
     d += ["    if (slice == %d) %s_basis_s%d(x, xd, alpha, sw, red, out, lane);" % (i, fn, i) for i in range(len(sl))]
     d += ["}", "", "}  // namespace mbxg", ""]
     write_if_changed(os.path.join(out_dir, "ad_%s_basis.inc" % name),
-                     "\n".join(head("Coefficient basis and its tangent in %d slices (coefficient ranges %s)."
+                     "\n".join(head("Coefficient basis and its tangent in %d slices (slot ranges %s)."
                                     % (len(sl), ", ".join("%d-%d" % (c0, c1 - 1) for c0, c1 in sl))))
                      + "\n".join(body) + "\n".join(d))
     tu = lambda what, inc, launcher: "\n".join([
         "// GENERATED by mbx_amd/gen/polygen.py -- do not edit.",
-        "// %s of the %s polynomial (%d variables, %d coefficients)." % (what, name, nvars, len(coef)),
+        "// %s of the %s polynomial in symmetry-adapted coordinates (%d variables, %d slots)." % (what, name, nvars, nrow),
         "#include \"gen/%s\"" % inc, "", "namespace mbxg {", "", launcher, "", "}  // namespace mbxg", ""])
     write_if_changed(os.path.join(out_dir, "ad_%s_tan.hip" % name), tu(
         "Gradient tangent", "ad_%s_tan.inc" % name,
@@ -706,17 +712,17 @@ def generate_ad(name, out_dir):
         "double* gds, hipStream_t st) {\n"
         "    static_assert(kAdParts == %d, \"part count of the generated code\");\n"
         "    if (n <= 0) return hipSuccess;\n"
-        "    hipLaunchKernelGGL((k_ad_tan<%d, %d, %s_tan>), dim3((n + 63) / 64, %d), dim3(64), 0, st, xs, xds, n, ld,\n"
-        "                       (uint64_t)(uintptr_t)coef, gds);\n"
-        "    return hipGetLastError();\n}" % (name, AD_PARTS, nvars, AD_PARTS, fn, AD_PARTS)))
+        "    hipLaunchKernelGGL((k_ad_tan<%d, %d, %s_tan, %s_tan_sym>), dim3((n + 63) / 64, %d), dim3(64), 0, st, xs,\n"
+        "                       xds, n, ld, (uint64_t)(uintptr_t)coef, gds);\n"
+        "    return hipGetLastError();\n}" % (name, AD_PARTS, nvars, AD_PARTS, fn, fn, AD_PARTS)))
     write_if_changed(os.path.join(out_dir, "ad_%s_basis.hip" % name), tu(
         "Coefficient basis", "ad_%s_basis.inc" % name,
         "hipError_t launch_ad_basis_%s(const double* xs, const double* xds, const double* sw, const double* swd, "
         "const double* g_energy, int n, int ld, double* partial, hipStream_t st) {\n"
         "    if (n <= 0) return hipSuccess;\n"
-        "    hipLaunchKernelGGL((k_ad_basis<%d, %d, %s_basis>), dim3((n + 63) / 64, %d), dim3(64), 0, st, xs, xds, sw, "
-        "swd,\n                       g_energy, n, ld, partial);\n"
-        "    return hipGetLastError();\n}" % (name, nvars, len(coef), fn, len(sl))))
+        "    hipLaunchKernelGGL((k_ad_basis<%d, %d, %s_basis, %s_basis_sym>), dim3((n + 63) / 64, %d), dim3(64), 0, st, xs,\n"
+        "                       xds, sw, swd, g_energy, n, ld, partial);\n"
+        "    return hipGetLastError();\n}" % (name, nvars, nrow, fn, fn, len(sl))))
     return dict(parts=AD_PARTS, slices=len(sl))
 
 
