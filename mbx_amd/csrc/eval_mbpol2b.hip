@@ -37,15 +37,22 @@ __global__ void __launch_bounds__(kGradBlock2) k_grad_mbpol2b(const int* __restr
     __shared__ GradTable<256, 9> T;
     const int t = blockIdx.x * kGradBlock2 + threadIdx.x;
     const int n = min(*n_dev, cap);
-    if (GRAD) table_init(T);
-    __syncthreads();
+    if (GRAD) {
+        table_init(T);
+        __syncthreads();
+    }
     double e_sum = 0.0;
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int m1 = -1, m2 = -1;
+    double gd[18];
+#pragma unroll
+    for (int j = 0; j < 18; ++j) gd[j] = 0.0;
     if (t < n) {
         const double sw = sws[t];
         const double P = ps[t];
         if (GRAD) {
-            const int m1 = list[2 * t], m2 = list[2 * t + 1];
+            m1 = list[2 * t];
+            m2 = list[2 * t + 1];
             double s[30], oh1a[3], oh2a[3], oh1b[3], oh2b[3];
             load_dimer(N, m1, m2, s, oh1a, oh2a, oh1b, oh2b);
             double xg[30];
@@ -71,7 +78,6 @@ __global__ void __launch_bounds__(kGradBlock2) k_grad_mbpol2b(const int* __restr
             const double rOO = sqrt(dOO[0] * dOO[0] + dOO[1] * dOO[1] + dOO[2] * dOO[2]);
             double gsw;
             switch2(rOO, gsw);
-            double gd[18];
 #pragma unroll
             for (int j = 0; j < 18; ++j) gd[j] = sw * xg[j];
             const double gsc = gsw * (P / rOO);
@@ -89,8 +95,6 @@ __global__ void __launch_bounds__(kGradBlock2) k_grad_mbpol2b(const int* __restr
                 for (int at = 0; at < 6; ++at) acc -= s[3 * at + va[q]] * gd[3 * at + vb[q]];
                 vir[q] = acc;
             }
-            table_add(T, m1, gd, 9, grad, 3 * (size_t)N.first_atom[m1]);
-            table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
         }
         const double e = sw * P;
         e_out[t] = e;
@@ -100,8 +104,10 @@ __global__ void __launch_bounds__(kGradBlock2) k_grad_mbpol2b(const int* __restr
             for (int q = 0; q < 6; ++q) vir_out[(size_t)q * ld + t] = vir[q];
     }
     if (GRAD) {
+        table_add_runs<9>(T, t < n, m1, gd, grad, N.first_atom);
+        if (t < n) table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
         __syncthreads();
-        table_flush(T, N.first_atom, N.nat, grad);
+        table_flush(T, grad);
     }
     e_sum = wave_sum(e_sum);
     const int rec = blockIdx.x * (kGradBlock2 / 64) + threadIdx.x / 64;

@@ -202,26 +202,30 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
                                                             double* __restrict__ grad, double* __restrict__ e_out,
                                                             double* __restrict__ vir_out,
                                                             double* __restrict__ partials) {
-    __shared__ GradTable<128, 15> T;
+    // a block's 128 dimers hold up to 128 partners (a table near full is all probes), its trimers some 50
+    __shared__ GradTable<GRAD ? (H::kMon == 2 ? 256 : 128) : 1, 15> T;
     const int t = blockIdx.x * kGradBlockNrg + threadIdx.x;
     const int n = min(*n_dev, cap);
-    if (GRAD) table_init(T);
-    __syncthreads();
+    if (GRAD) {
+        table_init(T);
+        __syncthreads();
+    }
     double e_sum = 0.0;
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int mon[3] = {-1, -1, -1}, query = -2;
+    double xg[3 * H::kNSites];
+#pragma unroll
+    for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
     if (t < n) {
         const double P = ps[t];
         double e;
         if (GRAD) {
             double x[3 * H::kNSites], oh1[3], oh2[3];
-            int mon[3];
             holder_sites<H>(N, list + H::kMon * (size_t)t, x, mon, oh1, oh2);
+            query = list[H::kMon * (size_t)t];
             double d[3][3], r[3], s[3], gsw[3];
             holder_switches<H>(x, d, r, s, gsw);
             const double sw = H::kMon == 2 ? s[0] : s[0] * s[1] + s[0] * s[2] + s[1] * s[2];
-            double xg[3 * H::kNSites];
-#pragma unroll
-            for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
             static_for<H::kNVars>([&](auto J) {
                 constexpr int j = decltype(J)::value;
                 double gj = gs[(size_t)j * ld + t];
@@ -289,10 +293,6 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
                 for (int at = 0; at < H::kNReal; ++at) acc += -x[3 * at + va[q]] * xg[3 * at + vb[q]];
                 vir[q] = acc;
             }
-#pragma unroll
-            for (int s2 = 0; s2 < H::kMon; ++s2)
-                table_add(T, mon[s2], xg + 3 * slot_site<H>(s2), 3 * H::kNat[s2], grad,
-                          3 * (size_t)N.first_atom[mon[s2]]);
         } else {
             e = P * sws[t];
         }
@@ -303,8 +303,13 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
             for (int q = 0; q < 6; ++q) vir_out[(size_t)q * ld + t] = vir[q];
     }
     if (GRAD) {
+        static_for<H::kMon>([&](auto S) {  // the query monomer is in any slot
+            constexpr int s2 = decltype(S)::value;
+            table_add_slot<3 * H::kNat[s2]>(T, t < n, mon[s2] == query, mon[s2], xg + 3 * slot_site<H>(s2), grad,
+                                            N.first_atom);
+        });
         __syncthreads();
-        table_flush(T, N.first_atom, N.nat, grad);
+        table_flush(T, grad);
     }
     e_sum = wave_sum(e_sum);
     const int rec = blockIdx.x * (kGradBlockNrg / 64) + threadIdx.x / 64;

@@ -243,33 +243,16 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
             for (int q = 0; q < 6; ++q) vir_out[(size_t)q * ld + t] = vir[q];
     }
     if (GRAD) {
-        // The evaluate list is grouped by query monomer, so usually every active lane of the
-        // wavefront has the same monomer 1: its nine gradient values are then summed across the
-        // wavefront (inactive lanes hold zeros) and enter the table once instead of 64 times.
-        const bool act = t < n;
-        const unsigned long long am = __ballot(act);
-        if (am) {
-            const int lane = threadIdx.x & 63, lead = __ffsll((long long)am) - 1;
-            const int mq = __shfl(m1, lead, 64);
-            if (__ballot(act && m1 != mq) == 0) {
-                double r[9];
-#pragma unroll
-                for (int c = 0; c < 9; ++c) r[c] = wave_sum(gd[c]);
-                if (lane == lead) table_add(T, mq, r, 9, grad, 3 * (size_t)N.first_atom[mq]);
-            } else if (act) {
-                table_add(T, m1, gd, 9, grad, 3 * (size_t)N.first_atom[m1]);
-            }
-            if (act) {
-                table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
-                table_add(T, m3, gd + 18, 9, grad, 3 * (size_t)N.first_atom[m3]);
-            }
-        }
+        const bool act = t < n;  // inactive lanes hold zeros
+        table_add_runs<9>(T, act, m1, gd, grad, N.first_atom);
+        if (act) table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
+        if (act) table_add(T, m3, gd + 18, 9, grad, 3 * (size_t)N.first_atom[m3]);
         if (WAVE) {
             wave_lds_order();
-            table_flush_wave(T, N.first_atom, N.nat, grad);
+            table_flush_wave(T, grad);
         } else {
             __syncthreads();
-            table_flush(T, N.first_atom, N.nat, grad);
+            table_flush(T, grad);
         }
     }
     // one partial record per wavefront

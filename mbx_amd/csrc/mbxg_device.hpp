@@ -136,9 +136,25 @@ __device__ __forceinline__ void static_for(F&& f) {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// v of another lane through the data-parallel path (no LDS): CTRL picks the lane, lanes without a source get 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the wavefront's 64 lanes, the same in all of them.  Every lane has to be active.
 __device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v += dpp_move<0xB1, 0xf>(v);   // quad_perm [1 0 3 2]
+    v += dpp_move<0x4E, 0xf>(v);   // quad_perm [2 3 0 1]
+    v += dpp_move<0x141, 0xf>(v);  // row_half_mirror: the other four of eight
+    v += dpp_move<0x140, 0xf>(v);  // row_mirror: the other eight of sixteen
+    v += dpp_move<0x142, 0xa>(v);  // row_bcast15: row 0 into row 1, row 2 into row 3
+    v += dpp_move<0x143, 0xc>(v);  // row_bcast31: rows 0-1 into rows 2-3; lane 63 holds the sum
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
+    return __hiloint2double(hi, lo);
 }
 
 }  // namespace mbxg

@@ -6,59 +6,166 @@
 // (LDS FP64 atomics); after a barrier the table is flushed to the global gradient with one
 // set of device atomics per distinct monomer.  If the table fills, the lane falls back to
 // device atomics directly, so the result never depends on the table size.
+//
+// These kernels are bound by the atomics and by the latency around them, not by arithmetic.  What helped,
+// measured on the 2B chain rules (32 beads of 57 CH4 + 513 H2O: MB-pol / CH4-H2O; 2048; 6859 waters):
+// before 97 / 122; 23; 43 us, with the entries' values flushed by consecutive lanes from a list of the
+// occupied entries (no loads from memory, some eight cache lines a wavefront instead of 64), tables at
+// most half full and the query monomer's values summed across the wavefront 57 / 65; 18; 26 us.  CH4-H2O-H2O
+// 370 -> 315 us.  Device atomics without the table: 193 / 119; 40 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include "mbxg_device.hpp"
 
 namespace mbxg {
 
 template <int TB, int NA>
 struct GradTable {
-    int key[TB];
     double val[TB * NA];
+    int key[TB];   // monomer, -1: free
+    int dest[TB];  // its first value in the gradient * 32 + its number of values
+    int used[TB];  // the occupied entries, in the order they were taken
+    int count;
 };
+
+// LDS FP64 add.  The pointer is cast to the LDS address space: through a generic one unsafeAtomicAdd
+// becomes a flat atomic, which also waits for the device memory path.
+__device__ __forceinline__ void lds_add(double* p, double v) {
+    __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double*)p, v);
+}
+
+// Clear the table with threads first, first + step, ...
+template <int TB, int NA>
+__device__ __forceinline__ void table_init_from(GradTable<TB, NA>& T, int first, int step) {
+    for (int i = first; i < TB; i += step) T.key[i] = -1;
+    for (int i = first; i < TB * NA; i += step) T.val[i] = 0.0;
+    if (first == 0) T.count = 0;
+}
 
 template <int TB, int NA>
 __device__ __forceinline__ void table_init(GradTable<TB, NA>& T) {
-    for (int i = threadIdx.x; i < TB; i += blockDim.x) T.key[i] = -1;
-    for (int i = threadIdx.x; i < TB * NA; i += blockDim.x) T.val[i] = 0.0;
+    table_init_from(T, threadIdx.x, blockDim.x);
+}
+
+// The entry of monomer `mon`, whose cnt values start at grad + goff; -1: the table is full.
+template <int TB, int NA>
+__device__ __forceinline__ int table_entry(GradTable<TB, NA>& T, int mon, int cnt, size_t goff) {
+    unsigned h = ((unsigned)mon * 2654435761u) % TB;
+    for (int probe = 0; probe < TB; ++probe) {
+        int k = __atomic_load_n(&T.key[h], __ATOMIC_RELAXED);
+        if (k == -1) {
+            k = atomicCAS(&T.key[h], -1, mon);
+            if (k == -1) {  // taken here
+                T.dest[h] = (int)goff * 32 + cnt;
+                T.used[atomicAdd(&T.count, 1)] = h;
+                return h;
+            }
+        }
+        if (k == mon) return h;
+        h = (h + 1) % TB;
+    }
+    return -1;
 }
 
 // Add cnt (<= NA) values for monomer `mon`; falls back to device atomics at grad + goff if full.
 template <int TB, int NA>
 __device__ __forceinline__ void table_add(GradTable<TB, NA>& T, int mon, const double* g, int cnt, double* grad,
                                           size_t goff) {
-    unsigned h = ((unsigned)mon * 2654435761u) % TB;
-    for (int probe = 0; probe < TB; ++probe) {
-        int k = __atomic_load_n(&T.key[h], __ATOMIC_RELAXED);
-        if (k == -1) k = atomicCAS(&T.key[h], -1, mon);
-        if (k == -1 || k == mon) {
-#pragma unroll
-            for (int c = 0; c < NA; ++c)
-                if (c < cnt) unsafeAtomicAdd(&T.val[h * NA + c], g[c]);
-            return;
-        }
-        h = (h + 1) % TB;
-    }
+    const int h = table_entry(T, mon, cnt, goff);
 #pragma unroll
     for (int c = 0; c < NA; ++c)
-        if (c < cnt) unsafeAtomicAdd(grad + goff + c, g[c]);
+        if (c < cnt) {
+            if (h >= 0)
+                lds_add(&T.val[h * NA + c], g[c]);
+            else
+                unsafeAtomicAdd(grad + goff + c, g[c]);
+        }
 }
 
-// After a barrier: one set of device atomics per occupied entry (3 values per atom of the
-// entry's monomer).
-template <int TB, int NA>
-__device__ __forceinline__ void table_flush(const GradTable<TB, NA>& T, const int* first_atom, const int* nat,
-                                            double* grad) {
-    for (int i = threadIdx.x; i < TB; i += blockDim.x) {
-        const int mon = T.key[i];
-        if (mon < 0) continue;
-        double* gp = grad + 3 * (size_t)first_atom[mon];
-        const int cnt = 3 * nat[mon];
+// The sum of a run: lanes `in`'s CNT values added across the wavefront, value c left in lane c.
+template <int CNT>
+__device__ __forceinline__ double run_sum(bool in, const double* g) {
+    const int lane = threadIdx.x & 63;
+    double mine = 0.0;
 #pragma unroll
-        for (int c = 0; c < NA; ++c)
-            if (c < cnt) unsafeAtomicAdd(gp + c, T.val[i * NA + c]);
+    for (int c = 0; c < CNT; ++c) {
+        const double v = wave_sum(in ? g[c] : 0.0);
+        if (lane == c) mine = v;
     }
+    return mine;
+}
+
+// The evaluate lists are grouped by query monomer, so one slot of an n-mer has the same monomer in runs
+// of lanes, where 64 atomics on one address would be done one after the other.  table_add_runs
+// adds every active lane's CNT values for its monomer `mon` (the other lanes' values are zeros); all lanes
+// of the wavefront have to arrive together.  A run's values are summed across the wavefront first and
+// added once, one lane per value; lanes left after kRuns runs, and short runs, add for themselves.
+constexpr int kRuns = 3;      // a wavefront of a long list spans two query monomers, seldom three
+constexpr int kRunLanes = 8;  // a run's sum costs about as much as eight lanes on one address
+
+// One run of the lanes in `left`: sets mq and in, takes the run's lanes out of left; false: none worth it.
+__device__ __forceinline__ bool next_run(bool act, int mon, unsigned long long& left, int& mq, bool& in) {
+    mq = __builtin_amdgcn_readlane(mon, __ffsll((long long)left) - 1);
+    in = act && mon == mq;
+    const unsigned long long same = __ballot(in) & left;
+    if (__popcll(same) < kRunLanes) return false;
+    left &= ~same;
+    return true;
+}
+
+template <int CNT, int TB, int NA>
+__device__ __forceinline__ void table_add_runs(GradTable<TB, NA>& T, bool act, int mon, const double* g, double* grad,
+                                               const int* first_atom) {
+    const int lane = threadIdx.x & 63;
+    unsigned long long left = __ballot(act);
+    int mq;
+    bool in;
+#pragma nounroll
+    for (int run = 0; run < kRuns && left; ++run) {
+        if (!next_run(act, mon, left, mq, in)) break;
+        const double mine = run_sum<CNT>(in, g);
+        const size_t goff = 3 * (size_t)first_atom[mq];
+        int h = 0;
+        if (lane == 0) h = table_entry(T, mq, CNT, goff);
+        h = __builtin_amdgcn_readlane(h, 0);
+        if (lane < CNT) {
+            if (h >= 0)
+                lds_add(&T.val[h * NA + lane], mine);
+            else
+                unsafeAtomicAdd(grad + goff + lane, mine);
+        }
+    }
+    if (act && ((left >> lane) & 1)) table_add(T, mon, g, CNT, grad, 3 * (size_t)first_atom[mon]);
+}
+
+// One slot of an n-mer whose query monomer may be in any slot (`query`: this lane's is in this one).
+template <int CNT, int TB, int NA>
+__device__ __forceinline__ void table_add_slot(GradTable<TB, NA>& T, bool act, bool query, int mon, const double* g,
+                                               double* grad, const int* first_atom) {
+    if (__ballot(act && query))
+        table_add_runs<CNT>(T, act, mon, g, grad, first_atom);
+    else if (act)
+        table_add(T, mon, g, CNT, grad, 3 * (size_t)first_atom[mon]);
+}
+
+// The occupied entries into the gradient, by threads first, first + step, ...: one device atomic per
+// value, consecutive threads on consecutive values, so a wavefront's atomics fall on some eight cache
+// lines instead of one line per lane, and nothing is loaded from memory on the way.
+template <int TB, int NA>
+__device__ __forceinline__ void table_flush_from(const GradTable<TB, NA>& T, int first, int step, double* grad) {
+    const int n = T.count * NA;
+    for (int i = first; i < n; i += step) {
+        const int e = i / NA, c = i - e * NA, h = T.used[e], d = T.dest[h];
+        if (c < (d & 31)) unsafeAtomicAdd(grad + (d >> 5) + c, T.val[h * NA + c]);
+    }
+}
+
+// After a barrier: the whole block's threads.
+template <int TB, int NA>
+__device__ __forceinline__ void table_flush(const GradTable<TB, NA>& T, double* grad) {
+    table_flush_from(T, threadIdx.x, blockDim.x, grad);
 }
 
 // A table that one wavefront owns alone (the other wavefronts of its block never touch it):
@@ -72,23 +179,12 @@ __device__ __forceinline__ void wave_lds_order() {
 
 template <int TB, int NA>
 __device__ __forceinline__ void table_init_wave(GradTable<TB, NA>& T) {
-    const int lane = threadIdx.x & 63;
-    for (int i = lane; i < TB; i += 64) T.key[i] = -1;
-    for (int i = lane; i < TB * NA; i += 64) T.val[i] = 0.0;
+    table_init_from(T, threadIdx.x & 63, 64);
 }
 
 template <int TB, int NA>
-__device__ __forceinline__ void table_flush_wave(const GradTable<TB, NA>& T, const int* first_atom, const int* nat,
-                                                 double* grad) {
-    for (int i = threadIdx.x & 63; i < TB; i += 64) {
-        const int mon = T.key[i];
-        if (mon < 0) continue;
-        double* gp = grad + 3 * (size_t)first_atom[mon];
-        const int cnt = 3 * nat[mon];
-#pragma unroll
-        for (int c = 0; c < NA; ++c)
-            if (c < cnt) unsafeAtomicAdd(gp + c, T.val[i * NA + c]);
-    }
+__device__ __forceinline__ void table_flush_wave(const GradTable<TB, NA>& T, double* grad) {
+    table_flush_from(T, threadIdx.x & 63, 64, grad);
 }
 
 }  // namespace mbxg

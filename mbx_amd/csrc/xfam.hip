@@ -502,13 +502,19 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
                                                        const double* __restrict__ ps, int ld,
                                                        double* __restrict__ grad, double* __restrict__ e_out,
                                                        double* __restrict__ partials) {
-    __shared__ GradTable<128, 9> T;
+    __shared__ GradTable<H::kMon == 2 ? 256 : 128, 9> T;  // (as k_grad_nrg)
     const int t = blockIdx.x * kGradBlockX + threadIdx.x;
     const int n = min(*n_dev, cap);
-    if (grad) table_init(T);
-    __syncthreads();
+    if (grad) {
+        table_init(T);
+        __syncthreads();
+    }
     double e_sum = 0.0;
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int mon[4] = {-1, -1, -1, -1}, anchor = -1;
+    double xg[3 * H::kNSites];
+#pragma unroll
+    for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
     if (t < n && !grad) {
         const int* ent = list + (size_t)(H::kMon + 1) * t;
         const double P = ps[t];
@@ -524,9 +530,6 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
         xsites<H>(N, ent, x, oh1, oh2);
         double d[6][3], r[6], s[6], gsw[6];
         const double sw = xswitches<H>(x, d, r, s, gsw);
-        double xg[3 * H::kNSites];
-#pragma unroll
-        for (int i = 0; i < 3 * H::kNSites; ++i) xg[i] = 0.0;
         static_for<H::kNVars>([&](auto J) {
             constexpr int j = decltype(J)::value;
             const double gj = gs[(size_t)j * ld + t] * sw;
@@ -591,14 +594,20 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
             vir[q] = acc;
         }
 #pragma unroll
-        for (int s2 = 0; s2 < H::kMon; ++s2)
-            table_add(T, ent[s2], xg + 3 * xslot_site<H>(s2), 3 * H::kNat[s2], grad,
-                      3 * (size_t)N.first_atom[ent[s2]]);
+        for (int s2 = 0; s2 < H::kMon; ++s2) mon[s2] = ent[s2];
+        anchor = ent[H::kMon];
         e_out[t] = e;
         e_sum = e;
     }
-    __syncthreads();
-    if (grad) table_flush(T, N.first_atom, N.nat, grad);
+    if (grad) {
+        static_for<H::kMon>([&](auto S) {  // the query monomer is in any slot
+            constexpr int s2 = decltype(S)::value;
+            table_add_slot<3 * H::kNat[s2]>(T, t < n, anchor == s2, mon[s2], xg + 3 * xslot_site<H>(s2), grad,
+                                            N.first_atom);
+        });
+        __syncthreads();
+        table_flush(T, grad);
+    }
     e_sum = wave_sum(e_sum);
     const int rec = blockIdx.x * (kGradBlockX / 64) + threadIdx.x / 64;
     double* out = partials + (size_t)rec * kPartials;
