@@ -179,6 +179,8 @@ struct ListState {
     DBuf<int> cell, cell_count, cell_start, cell_pos, cell_slot;  // cell_pos: a slot's place in its cell
     DBuf<int4> counts, offsets, counts_x, offsets_x;
     DBuf<int4> wpre, wpre_x;      // per (query, wavefront): prefix within the query
+    DBuf<int> cell_sums;          // per block of k_cell_sums
+    DBuf<ScanShare> shares;       // per block of k_scan_shares
     DBuf<int> list2, list3, evals[kFamilies];
     DBuf<double> gscratch;        // match storage when it does not fit in LDS
     // capacities in n-mers: cap = {list2, MB-pol 2B, list3, MB-pol 3B},
@@ -206,8 +208,10 @@ struct EvalState {
 // Largest match storage kept in LDS (80 bytes per match): 512 matches = 40 KB per block.
 constexpr int kMaxLdsMatches = 384;  // 160 bytes of LDS a match: at most 60 KB a block
 constexpr int kScratchBlocks = 2048;
-// slices per configuration in the per-configuration reductions (blocks = configurations x slices)
-constexpr int kConfSlices = 16;
+// slices per configuration in the per-configuration reductions (blocks = configurations x slices x
+// families): about kConfSlice n-mers each, so a few hundred configurations are not cut further (256 gas
+// clusters: 16 slices always, a launch per family, cost 24 + 5 us a family)
+constexpr int kConfSlices = 16, kConfSlice = 2048;
 
 }  // namespace
 
@@ -235,7 +239,6 @@ struct mbxg_ctx {
     std::vector<int> mon_off, pt_off;
     DBuf<int> d_pconf, d_pt_off;
     DBuf<double> d_conf_tot;  // per configuration: 2B record, then 3B record (kPartials each)
-    DBuf<double> d_conf_fam;  // per family and configuration (kPartials each)
     DBuf<double> d_conf_part; // per family, configuration and slice (kConfSlices per configuration)
     ListState L;
     EvalState fam[kFamilies];
@@ -281,6 +284,11 @@ struct mbxg_ctx {
     DBuf<int> t_counts, t_off, t_list, t_ovf;  // tetramers
     int64_t n4_listed = 0;
     bool x_last = false;                     // the last compute ran the further families / 4B
+    // pinned host memory: what each compute's last kernel publishes, and a stage for the per-atom arrays
+    Published* host = nullptr;
+    double* host_atoms = nullptr;
+    size_t host_atoms_n = 0;
+    bool recomputed = false;                 // the last finish() computed again (lists had outgrown)
 };
 
 int mbxg::report_error(int code, const char* msg) {
@@ -306,6 +314,11 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
         delete c;
         return fail(MBXG_EHIP, "mbxg_create: stream/event creation failed: %s", hipGetErrorString(e));
     }
+    if (hipHostMalloc((void**)&c->host, sizeof(Published), hipHostMallocDefault) != hipSuccess) {
+        delete c;
+        return fail(MBXG_ENOMEM, "mbxg_create: pinned host allocation failed");
+    }
+    std::memset(c->host, 0, sizeof(Published));
     int n1b = 0, n1b_co2 = 0;
     const double* fit1b = ch4_1b_fit(&n1b);
     const double* fit1b_co2 = co2_1b_fit(&n1b_co2);
@@ -375,12 +388,13 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
     L.offsets_x.release();
     L.wpre.release();
     L.wpre_x.release();
+    L.cell_sums.release();
+    L.shares.release();
     for (DBuf<int>& b : L.evals) b.release();
     L.gscratch.release();
     c->d_pconf.release();
     c->d_pt_off.release();
     c->d_conf_tot.release();
-    c->d_conf_fam.release();
     c->d_conf_part.release();
     c->d_fam_tot.release();
     for (DBuf<double>& b : c->d_coefn) b.release();
@@ -429,6 +443,8 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
     for (hipEvent_t& e : c->ev)
         if (e) (void)hipEventDestroy(e);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
+    if (c->host) (void)hipHostFree(c->host);
+    if (c->host_atoms) (void)hipHostFree(c->host_atoms);
     (void)hipEventDestroy(c->fork);
     (void)hipEventDestroy(c->join);
     (void)hipStreamDestroy(c->stream2);
@@ -476,7 +492,6 @@ int set_configs(mbxg_ctx* c, int nconf, const int* mon_off) {
     for (int q = 0; q < nconf; ++q) pt_off[q + 1] += pt_off[q];
     if (c->d_pconf.reserve(pconf.size()) || c->d_pt_off.reserve(nconf + 1) ||
         c->d_conf_tot.reserve((size_t)2 * kPartials * nconf) ||
-        c->d_conf_fam.reserve((size_t)kFamilies * kPartials * nconf) ||
         c->d_conf_part.reserve((size_t)kFamilies * kConfSlices * kPartials * nconf))
         return fail(MBXG_ENOMEM, "configurations: device allocation failed");
     HIPCHK(hipMemcpy(c->d_pconf.p, pconf.data(), sizeof(int) * pconf.size(), hipMemcpyHostToDevice));
@@ -888,7 +903,8 @@ int prepare_layout(mbxg_ctx* c, double cut) {
         total += bound[k];
     }
     if (L.d_grids.reserve(nconf) || L.d_cell_base.reserve(nconf) || L.d_cell_bound.reserve(nconf) ||
-        L.cell_count.reserve(total) || L.cell_start.reserve(total + 1))
+        L.cell_count.reserve(total) || L.cell_start.reserve(total + 1) ||
+        L.cell_sums.reserve((total + kCellChunk - 1) / kCellChunk))
         return fail(MBXG_ENOMEM, "cell layout: device allocation failed");
     hipStream_t st = c->stream;
     launch_zero_int(L.cell_count.p, total, st);  // every scan leaves the counts zero again
@@ -924,7 +940,8 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
         L.bz.reserve(ns) || L.cell.reserve(ns) || L.cell_pos.reserve(ns) || L.cell_slot.reserve(ns) || L.pinfo.reserve(np) ||
         L.counts.reserve(np) || L.wpre.reserve((size_t)np * kQueryWaves) || L.wpre_x.reserve((size_t)np * kQueryWaves) ||
         L.offsets.reserve(np + 1) || L.counts_x.reserve(np) || L.offsets_x.reserve(np + 1) ||
-        L.wmax.reserve(np) || L.wmax_x.reserve(np) || L.maxw.reserve(2))
+        L.wmax.reserve(np) || L.wmax_x.reserve(np) || L.maxw.reserve(2) ||
+        L.shares.reserve((np + kScanChunk - 1) / kScanChunk))
         return fail(MBXG_ENOMEM, "list buffers: device allocation failed");
     const int tb = 256, pb = (np + tb - 1) / tb, sb = (ns + tb - 1) / tb;
     // the gas-phase grids read the input coordinates (the working copy equals them there)
@@ -947,7 +964,14 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
                            L.cell.p, L.pinfo.p);
         hipLaunchKernelGGL(k_bin_count, dim3(sb), dim3(tb), 0, st, L.cell.p, ns, L.cell_count.p, L.cell_pos.p);
     }
-    hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(1024), 0, st, L.cell_count.p, L.ncell_total, L.cell_start.p);
+    if (L.ncell_total <= kCellsOneBlock) {
+        hipLaunchKernelGGL(k_scan_cells, dim3(1), dim3(1024), 0, st, L.cell_count.p, L.ncell_total, L.cell_start.p);
+    } else {
+        const int cb = (L.ncell_total + kCellChunk - 1) / kCellChunk;
+        hipLaunchKernelGGL(k_cell_sums, dim3(cb), dim3(1024), 0, st, L.cell_count.p, L.ncell_total, L.cell_sums.p);
+        hipLaunchKernelGGL(k_scan_cells_wide, dim3(cb), dim3(1024), 0, st, L.cell_count.p, L.ncell_total,
+                           L.cell_sums.p, L.cell_start.p);
+    }
     hipLaunchKernelGGL(k_bin_fill, dim3(sb), dim3(tb), 0, st, L.cell.p, ns, L.cell_start.p, L.cell_pos.p, L.cx.p,
                        L.cy.p, L.cz.p, L.cell_slot.p, L.bx.p, L.by.p, L.bz.p);
     HIPCHK(hipGetLastError());
@@ -994,8 +1018,16 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
         double* gs = scratch();
         if (L.match_cap > kMaxLdsMatches && !gs) return fail(MBXG_ENOMEM, "match scratch: device allocation failed");
         HIPCHK(launch_nmers(A, N, one_pass ? 2 : 0, none, none, L.match_cap, gs, kScratchBlocks, st));
-        hipLaunchKernelGGL(k_scan_all, dim3(1), dim3(1024), 0, st, L.wmax.p, L.wmax_x.p, L.maxw.p, L.counts.p,
-                           L.offsets.p, L.counts_x.p, L.offsets_x.p, np);
+        if (np <= kScanOneBlock) {
+            hipLaunchKernelGGL(k_scan_all, dim3(1), dim3(1024), 0, st, L.wmax.p, L.wmax_x.p, L.maxw.p, L.counts.p,
+                               L.offsets.p, L.counts_x.p, L.offsets_x.p, np);
+        } else {
+            const int qb = (np + kScanChunk - 1) / kScanChunk;
+            hipLaunchKernelGGL(k_scan_shares, dim3(qb), dim3(kScanChunk / 4), 0, st, L.wmax.p, L.wmax_x.p, L.counts.p,
+                               L.counts_x.p, np, L.shares.p);
+            hipLaunchKernelGGL(k_scan_wide, dim3(qb), dim3(kScanChunk / 4), 0, st, L.shares.p, L.counts.p, L.offsets.p,
+                               L.counts_x.p, L.offsets_x.p, L.maxw.p, np);
+        }
         HIPCHK(hipGetLastError());
         if (!sync) break;
         int4 tot, totx;
@@ -1057,6 +1089,12 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
     HIPCHK(launch_nmers(A, N, 1, L.cap, L.capx, L.match_cap,
                         L.match_cap > kMaxLdsMatches ? L.gscratch.p : nullptr, kScratchBlocks, st));
     return 0;
+}
+
+PublishJob publish_job(const mbxg_ctx* c) {
+    const ListState& L = c->L;
+    if (!L.built) return {c->host, nullptr, nullptr, nullptr};
+    return {c->host, L.offsets.p + c->np, L.offsets_x.p + c->np, L.maxw.p};
 }
 
 void drop_graph(mbxg_ctx* c) {
@@ -1144,7 +1182,7 @@ int run_xfam(mbxg_ctx* c, const NmerCtx& N, bool want2, bool want3, bool want4, 
             }
         }
     }
-    HIPCHK(launch_xcombine(c->d_xfam_tot.p, c->d_totals.p, st));
+    HIPCHK(launch_xcombine(c->d_xfam_tot.p, c->d_totals.p, publish_job(c), st));
     return MBXG_OK;
 }
 
@@ -1172,8 +1210,7 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                            c->d_first.p, c->d_nat.p, c->nmon, c->box);
         HIPCHK(hipGetLastError());
     }
-    // the gradient, the 1B record when no 1B term runs and (batches) the family records start at
-    // zero: zeroed by the list build's first kernel, or by one launch of their own
+    // the gradient and the 1B record when no 1B term runs start at zero: zeroed by the list build's first kernel, or by one launch of their own
     c->one_body_last = (terms & MBXG_1B) && !(terms & MBXG_LISTS_ONLY);
     const bool batch = c->nconf > 1;
     ZeroJobs Z{};
@@ -1184,12 +1221,6 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
     if (!c->one_body_last) {
         Z.p[1] = c->d_totals.p + 2 * kPartials;
         Z.n[1] = kPartials;
-    }
-    if (batch) {
-        Z.p[2] = c->d_fam_tot.p;
-        Z.n[2] = (size_t)kFamilies * kPartials;
-        Z.p[3] = c->d_conf_fam.p;
-        Z.n[3] = (size_t)kFamilies * kPartials * c->nconf;
     }
     if (!(L.built && c->fuse_prep)) {
         hipLaunchKernelGGL(k_zero_multi, dim3(64), dim3(256), 0, st, Z);
@@ -1222,6 +1253,8 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
     HIPCHK(hipGetLastError());
     c->evaluated = L.built && !(terms & MBXG_LISTS_ONLY);
     FinishJobs J{};  // single configuration: the families' records, reduced after the join
+    ConfigJobs CJ{};  // batches: the families' n-mers, reduced per configuration after the join
+    int slices = 1;
     if (c->evaluated) {
         // the 2B families run on stream2, concurrently with the 3B ones: their small blocks
         // fill the machine while the last 3B blocks drain
@@ -1245,26 +1278,20 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
             return !(o.e_nmer.reserve(cap) || o.partials.reserve((size_t)kPartials * partials_records(cap)) ||
                      o.ws.reserve(wsz) || (batch && o.vir_nmer.reserve((size_t)6 * ld)));
         };
-        auto reduce = [&](int f, hipStream_t sk) {
+        auto reduce = [&](int f) {
             const int cap = fam_cap(L, f);
-            const int ld = (cap + 63) / 64 * 64;
             EvalState& o = c->fam[f];
             const int* nd = fam_ndev(L, c->np, f);
-            if (!batch) {
-                J.partials[f] = o.partials.p;
-                J.n_dev[f] = nd;
-                J.cap[f] = cap;
-                return;
-            }
-            hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, sk, o.partials.p, nd, cap,
-                               c->d_fam_tot.p + kPartials * f);
+            J.partials[f] = o.partials.p;
+            J.n_dev[f] = nd;
+            J.cap[f] = cap;
             if (batch) {
-                double* part = c->d_conf_part.p + (size_t)f * kConfSlices * kPartials * c->nconf;
-                hipLaunchKernelGGL(k_reduce_configs, dim3(c->nconf, kConfSlices), dim3(256), 0, sk, o.e_nmer.p,
-                                   o.vir_nmer.p, ld, f == FAM_MBPOL_2B || f == FAM_MBPOL_3B ? L.offsets.p : L.offsets_x.p,
-                                   c->d_pt_off.p, fam_component(f), cap, part);
-                hipLaunchKernelGGL(k_reduce_slices, dim3((c->nconf * kPartials + 255) / 256), dim3(256), 0, sk, part,
-                                   c->nconf, kConfSlices, c->d_conf_fam.p + (size_t)f * kPartials * c->nconf);
+                CJ.e_out[f] = o.e_nmer.p;
+                CJ.vir_out[f] = o.vir_nmer.p;
+                CJ.offsets[f] = f == FAM_MBPOL_2B || f == FAM_MBPOL_3B ? L.offsets.p : L.offsets_x.p;
+                CJ.comp[f] = fam_component(f);
+                CJ.cap[f] = cap;
+                slices = std::max(slices, std::min(kConfSlices, (int)(cap / ((int64_t)c->nconf * kConfSlice)) + 1));
             }
         };
         for (int i = 0; i < kFamilies; ++i) {
@@ -1317,8 +1344,8 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                 HIPCHK(launch_mbpol2b_chain(L.evals[f2].p, nd2, cap2, N, 1, c->d_grad.p, o2.e_nmer.p,
                                             batch ? o2.vir_nmer.p : nullptr, o2.partials.p, o2.ws.p, st));
                 if (ev) HIPCHK(hipEventRecord(ev[7], st));
-                reduce(f, st);
-                reduce(f2, st);
+                reduce(f);
+                reduce(f2);
                 HIPCHK(hipGetLastError());
                 continue;
             }
@@ -1335,7 +1362,7 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                                          o.e_nmer.p, vir, o.partials.p, o.ws.p, c->split3n, sk, nullptr));
                 if (timed) HIPCHK(hipEventRecord(ev[14], st));
             }
-            reduce(f, sk);
+            reduce(f);
             HIPCHK(hipGetLastError());
         }
         HIPCHK(hipEventRecord(c->join, c->stream2));
@@ -1343,17 +1370,20 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
     }
     // per-order totals: 2B = MB-pol + CH4-H2O + CH4-CH4, 3B = MB-pol + CH4-H2O-H2O (fixed order)
     if (!batch) {
-        hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinishThreads), 0, st, J, c->d_fam_tot.p, c->d_totals.p);
+        hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinishThreads), 0, st, J, c->d_fam_tot.p, c->d_totals.p,
+                           publish_job(c));
     } else {
-        hipLaunchKernelGGL(k_combine_families, dim3(1), dim3(64), 0, st, c->d_fam_tot.p, 1, c->d_totals.p);
-        launch_zero(c->d_totals.p + 3 * kPartials, kPartials, st);
+        const int nc = c->nconf;
+        hipLaunchKernelGGL(k_reduce_configs, dim3(nc, slices, kFamilies), dim3(256), 0, st, CJ, c->d_pt_off.p,
+                           c->d_conf_part.p);
+        hipLaunchKernelGGL(k_reduce_slices, dim3((nc * kPartials + 63) / 64), dim3(64), 0, st, CJ, c->d_conf_part.p, nc,
+                           slices, c->d_conf_tot.p);
+        hipLaunchKernelGGL(k_sum_configs, dim3(1), dim3(64 * 2 * kPartials), 0, st, c->d_conf_tot.p, nc, c->d_totals.p,
+                           publish_job(c));
     }
     c->x_last = xrun;
     if (xrun)  // then the further families' totals on top, and the 4B record
         if (int r = run_xfam(c, N, want2, want3, want4, !(terms & MBXG_LISTS_ONLY), do_grads)) return r;
-    if (c->nconf > 1)
-        hipLaunchKernelGGL(k_combine_families, dim3((c->nconf * kPartials + 63) / 64), dim3(64), 0, st,
-                           c->d_conf_fam.p, c->nconf, c->d_conf_tot.p);
     HIPCHK(hipGetLastError());
     if (ev) HIPCHK(hipEventRecord(ev[12], st));
     c->have_results = true;
@@ -1370,16 +1400,12 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
 int finish(mbxg_ctx* c) {
     HIPCHK(hipSetDevice(c->device));
     HIPCHK(hipStreamSynchronize(c->stream));
+    c->recomputed = false;
     if (!c->have_results || c->checked) return MBXG_OK;
     ListState& L = c->L;
-    int4 tot, totx;
+    const int4 tot = c->host->tot, totx = c->host->totx;
     int ovf = 0, mw[kFamilies] = {0, 0, 0, 0, 0};
-    int4 m2[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
-    HIPCHK(hipMemcpyAsync(&tot, L.offsets.p + c->np, sizeof(int4), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(&totx, L.offsets_x.p + c->np, sizeof(int4), hipMemcpyDeviceToHost, c->stream));
-    if (L.staged) HIPCHK(hipMemcpyAsync(m2, L.maxw.p, sizeof(m2), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    wave_maxima(m2, mw);
+    if (L.staged) wave_maxima(c->host->maxw, mw);
     ovf = totx.w;  // the largest match count of any query
     bool staging_short = false;  // a one-pass build staged more n-mers per wavefront than it holds
     for (int f = 0; f < kFamilies; ++f) staging_short = staging_short || mw[f] > L.scap[f];
@@ -1393,11 +1419,38 @@ int finish(mbxg_ctx* c) {
         }
         if (int r = run(c, c->last_terms, c->last_grads, true)) return r;
         HIPCHK(hipStreamSynchronize(c->stream));
+        c->recomputed = true;
     } else {
         L.tot = tot;
         L.totx = totx;
     }
     c->checked = true;
+    return MBXG_OK;
+}
+
+// A per-atom device array (3 * natoms doubles) into host memory `out`: the copy goes to pinned memory and
+// is on the stream before the wait, so there is one wait and no staging by the runtime.  A result of the
+// last compute is checked (finish()) and read again if that computed again.
+int read_atoms(mbxg_ctx* c, const double* src, double* out, bool result) {
+    const size_t n = 3 * (size_t)c->natoms;
+    if (n > c->host_atoms_n) {
+        if (c->host_atoms) HIPCHK(hipHostFree(c->host_atoms));
+        c->host_atoms = nullptr;
+        c->host_atoms_n = 0;
+        if (hipHostMalloc((void**)&c->host_atoms, n * sizeof(double), hipHostMallocDefault) != hipSuccess)
+            return fail(MBXG_ENOMEM, "results: pinned host allocation failed");
+        c->host_atoms_n = n;
+    }
+    for (int turn = 0; turn < 2; ++turn) {
+        HIPCHK(hipMemcpyAsync(c->host_atoms, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        if (!result) {
+            HIPCHK(hipStreamSynchronize(c->stream));
+            break;
+        }
+        if (int r = finish(c)) return r;
+        if (!c->recomputed) break;
+    }
+    std::memcpy(out, c->host_atoms, n * sizeof(double));
     return MBXG_OK;
 }
 
@@ -1640,12 +1693,9 @@ extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
 extern "C" int mbxg_get_results(mbxg_ctx* c, double* e2b, double* e3b, double* grad, double* virial) {
     if (!c) return fail(MBXG_EINVAL, "mbxg_get_results: null context");
     if (!c->have_results) return fail(MBXG_ESTATE, "mbxg_get_results: nothing computed");
-    if (int r = finish(c)) return r;
-    double tot[4 * kPartials];
-    HIPCHK(hipMemcpyAsync(tot, c->d_totals.p, sizeof(tot), hipMemcpyDeviceToHost, c->stream));
-    if (grad && c->natoms > 0)
-        HIPCHK(hipMemcpyAsync(grad, c->d_grad.p, sizeof(double) * 3 * c->natoms, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipSetDevice(c->device));
+    if (int r = grad && c->natoms > 0 ? read_atoms(c, c->d_grad.p, grad, true) : finish(c)) return r;
+    const double* tot = c->host->totals;
     if (e2b) *e2b = tot[0];
     if (e3b) *e3b = tot[kPartials];
     if (virial) {
@@ -1671,8 +1721,7 @@ extern "C" int mbxg_get_batch_results(mbxg_ctx* c, double* e2b, double* e3b, dou
         HIPCHK(hipMemcpyAsync(tot.data(), c->d_conf_tot.p, sizeof(double) * tot.size(), hipMemcpyDeviceToHost,
                               c->stream));
     } else {
-        HIPCHK(hipMemcpyAsync(tot.data(), c->d_totals.p, sizeof(double) * 2 * kPartials, hipMemcpyDeviceToHost,
-                              c->stream));
+        std::copy(c->host->totals, c->host->totals + 2 * kPartials, tot.begin());
     }
     HIPCHK(hipStreamSynchronize(c->stream));
     const double* t2 = tot.data();
@@ -1755,8 +1804,7 @@ extern "C" int mbxg_get_nmer_energies(mbxg_ctx* c, int order, int32_t* nmers, do
 extern "C" int mbxg_get_coords(mbxg_ctx* c, double* xyz) {
     if (!c || !xyz) return fail(MBXG_EINVAL, "mbxg_get_coords: bad arguments");
     HIPCHK(hipSetDevice(c->device));
-    if (c->natoms > 0)
-        HIPCHK(hipMemcpyAsync(xyz, c->d_xyz.p, sizeof(double) * 3 * c->natoms, hipMemcpyDeviceToHost, c->stream));
+    if (c->natoms > 0) return read_atoms(c, c->d_xyz.p, xyz, false);
     HIPCHK(hipStreamSynchronize(c->stream));
     return MBXG_OK;
 }
@@ -1792,9 +1840,7 @@ extern "C" int mbxg_get_energies(mbxg_ctx* c, double* e1b, double* e2b, double* 
     if (!c) return fail(MBXG_EINVAL, "mbxg_get_energies: null context");
     if (!c->have_results) return fail(MBXG_ESTATE, "mbxg_get_energies: nothing computed");
     if (int r = finish(c)) return r;
-    double tot[3 * kPartials];
-    HIPCHK(hipMemcpyAsync(tot, c->d_totals.p, sizeof(tot), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    const double* tot = c->host->totals;
     if (e1b) *e1b = tot[2 * kPartials];
     if (e2b) *e2b = tot[0];
     if (e3b) *e3b = tot[kPartials];
@@ -1832,9 +1878,7 @@ extern "C" int mbxg_get_term_energies(mbxg_ctx* c, double* e) {
     if (!c || !e) return fail(MBXG_EINVAL, "mbxg_get_term_energies: bad arguments");
     if (!c->have_results) return fail(MBXG_ESTATE, "mbxg_get_term_energies: nothing computed");
     if (int r = finish(c)) return r;
-    double tot[4 * kPartials];
-    HIPCHK(hipMemcpyAsync(tot, c->d_totals.p, sizeof(tot), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    const double* tot = c->host->totals;
     e[0] = tot[2 * kPartials];
     e[1] = tot[0];
     e[2] = tot[kPartials];

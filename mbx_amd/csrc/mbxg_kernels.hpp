@@ -70,6 +70,10 @@ __global__ void k_cloud_fix(const double* in, double* xyz, const int* first_atom
                             const int* pconf, const int* cell_base, double* cx, double* cy, double* cz, int* cell,
                             PtInfo* pinfo, int* cell_count, int* cell_pos, ZeroJobs Z);
 __global__ void k_scan_cells(int* cell_count, int ncell, int* cell_start);
+// The same over more than kCellsOneBlock cells: blocks of kCellChunk cells, sums[blocks] between them.
+constexpr int kCellChunk = 4096, kCellsOneBlock = 8192;
+__global__ void k_cell_sums(const int* cell_count, int ncell, int* sums);
+__global__ void k_scan_cells_wide(int* cell_count, int ncell, const int* sums, int* cell_start);
 __global__ void k_bin_fill(const int* cell, int ns, const int* cell_start, const int* cell_pos, const double* cx,
                            const double* cy, const double* cz, int* cell_slot, double* bx, double* by, double* bz);
 __global__ void k_zero(double* p, size_t n);
@@ -131,6 +135,16 @@ struct NmersArgs {
 // the exclusive scans of counts and counts_x (.w maximised), totals at n, in one launch.
 __global__ void k_scan_all(const int4* wmax, const int4* wmax_x, int4* maxw, const int4* counts, int4* offsets,
                            const int4* counts_x, int4* offsets_x, int n);
+// The same over more than kScanOneBlock queries (the two launches take what one workgroup takes at 2048):
+// blocks of kScanChunk queries, their shares between the launches.
+constexpr int kScanChunk = 1024, kScanOneBlock = 2048;
+struct ScanShare {
+    int4 c, cx, m, mx;
+};
+__global__ void k_scan_shares(const int4* wmax, const int4* wmax_x, const int4* counts, const int4* counts_x, int n,
+                              ScanShare* shares);
+__global__ void k_scan_wide(const ScanShare* shares, const int4* counts, int4* offsets, const int4* counts_x,
+                            int4* offsets_x, int4* maxw, int n);
 
 // The staged n-mers of a one-pass build, moved to the evaluate lists: block q (striding),
 // wavefront w copies its family-f n-mers to evals[f] at the family's offset of query q plus the
@@ -143,9 +157,31 @@ struct FinishJobs {
 };
 // One workgroup of kFinishThreads: each family's partial records summed in a fixed order into fam
 // (kPartials per family, zeros for the families not evaluated), then the per-order records of
-// totals as k_combine_families does (2B, 3B) and the 4B record zeroed.
+// totals (2B = MB-pol + CH4-H2O + CH4-CH4, 3B = MB-pol + CH4-H2O-H2O) and the 4B record zeroed.  (The 1B
+// record is a launch of its own before.)
+// The last kernel of a compute also publishes what the host reads after every step (the totals and the
+// list builder's counts and maxima) into pinned host memory, so that waiting for the stream is all the
+// host does: three copies of a few bytes each cost 40 us a step.
+struct Published {
+    double totals[4 * kPartials];
+    int4 tot, totx, maxw[2];
+};
+struct PublishJob {
+    Published* host;
+    const int4 *tot, *totx, *maxw;  // tot null: no lists were built
+};
 constexpr int kFinishThreads = 512;
-__global__ void k_finish(FinishJobs J, double* fam, double* totals);
+__global__ void k_finish(FinishJobs J, double* fam, double* totals, PublishJob P);
+
+// By one workgroup, after its threads have written (and __syncthreads() has ordered) totals.
+__device__ __forceinline__ void publish(const PublishJob& P, const double* totals) {
+    const int t = threadIdx.x;
+    if (t < 4 * kPartials) P.host->totals[t] = totals[t];
+    const int4 zero = make_int4(0, 0, 0, 0);
+    if (t == 0) P.host->tot = P.tot ? *P.tot : zero;
+    if (t == 1) P.host->totx = P.tot ? *P.totx : zero;
+    if (t < 2) P.host->maxw[t] = P.tot ? P.maxw[t] : zero;
+}
 
 struct CompactArgs {
     const int* stage[kFamilies];
@@ -256,15 +292,21 @@ hipError_t launch_poly_ch4h2o2_3b(const double* xs, const int* n_dev, int cap, i
 // (deterministic totals).
 __global__ void k_reduce_partials(const double* partials, const int* n_dev, int n_cap, double* out);
 
-// Per-configuration totals in two fixed-order levels: block (c, s) of a (nconf, S) grid sums
-// slice s of configuration c's evaluated n-mers, [offsets[pt_off[c]].comp,
-// offsets[pt_off[c+1]].comp) clamped to cap, from e_out / vir_out (leading dimension ld) into
-// part[c][s][kPartials] (energy, 6 virial components; zeros when vir_out is null); comp selects
-// the int4 component (0..3) holding the family's count.  k_reduce_slices then adds the S
-// slices of each configuration in order.
-__global__ void k_reduce_configs(const double* e_out, const double* vir_out, int ld, const int4* offsets,
-                                 const int* pt_off, int comp, int cap, double* part);
-__global__ void k_reduce_slices(const double* part, int nconf, int nsl, double* out);
-__global__ void k_combine_families(const double* fam, int nconf, double* out);
+// Per-configuration totals in two fixed-order levels, all families in one launch each: block (c, s, f) of
+// a (nconf, S, kFamilies) grid sums slice s of configuration c's evaluated n-mers of family f (null e_out:
+// not evaluated), [offsets[pt_off[c]].comp, offsets[pt_off[c+1]].comp) clamped to cap, from e_out / vir_out
+// (leading dimension cap rounded up to 64; zeros when vir_out is null) into part[f][c][s][kPartials]; comp
+// selects the int4 component (0..3) holding the family's count.  k_reduce_slices adds the slices of the
+// families of each order: out[2][nconf][kPartials].  k_sum_configs adds the configurations into the 2B and
+// 3B records of totals, zeroes the 4B one and publishes.
+struct ConfigJobs {
+    const double* e_out[kFamilies];
+    const double* vir_out[kFamilies];
+    const int4* offsets[kFamilies];
+    int comp[kFamilies], cap[kFamilies];
+};
+__global__ void k_reduce_configs(ConfigJobs J, const int* pt_off, double* part);
+__global__ void k_reduce_slices(ConfigJobs J, const double* part, int nconf, int nsl, double* out);
+__global__ void k_sum_configs(const double* conf, int nconf, double* totals, PublishJob P);
 
 }  // namespace mbxg

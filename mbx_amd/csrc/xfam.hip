@@ -889,18 +889,21 @@ size_t xclass_blocks(int n) { return ((size_t)n + kXBlock - 1) / kXBlock; }
 
 // The further families' records onto the per-order totals: 2B record += the 2B families, 3B
 // record += the 3B families, 4B record = the 4B family (fixed order).
-__global__ void k_xcombine(const double* __restrict__ xt, double* __restrict__ totals) {
+__global__ void k_xcombine(const double* __restrict__ xt, double* totals, PublishJob P) {
     const int q = threadIdx.x;
-    if (q >= kPartials) return;
-    double a[3] = {totals[q], totals[kPartials + q], 0.0};
-    for (int f = 0; f < kXFam; ++f) a[xfam_order(f) - 2] += xt[(size_t)f * kPartials + q];
-    totals[q] = a[0];
-    totals[kPartials + q] = a[1];
-    totals[3 * kPartials + q] = a[2];
+    if (q < kPartials) {
+        double a[3] = {totals[q], totals[kPartials + q], 0.0};
+        for (int f = 0; f < kXFam; ++f) a[xfam_order(f) - 2] += xt[(size_t)f * kPartials + q];
+        totals[q] = a[0];
+        totals[kPartials + q] = a[1];
+        totals[3 * kPartials + q] = a[2];
+    }
+    __syncthreads();
+    publish(P, totals);
 }
 
-hipError_t launch_xcombine(const double* xfam_tot, double* totals, hipStream_t st) {
-    hipLaunchKernelGGL(k_xcombine, dim3(1), dim3(64), 0, st, xfam_tot, totals);
+hipError_t launch_xcombine(const double* xfam_tot, double* totals, const PublishJob& P, hipStream_t st) {
+    hipLaunchKernelGGL(k_xcombine, dim3(1), dim3(64), 0, st, xfam_tot, totals, P);
     return hipGetLastError();
 }
 

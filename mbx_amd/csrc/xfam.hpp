@@ -59,8 +59,8 @@ hipError_t launch_xemit(int order, const int* list, int n, const int* code, cons
 hipError_t launch_xfam(int f, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
                        double* grad, double* e_out, double* partials, double* ws, hipStream_t st);
 // The further families' energy records (kXFam x kPartials) added to the per-order totals
-// (records 2B, 3B, 1B, 4B).
-hipError_t launch_xcombine(const double* xfam_tot, double* totals, hipStream_t st);
+// (records 2B, 3B, 1B, 4B), and published.
+hipError_t launch_xcombine(const double* xfam_tot, double* totals, const PublishJob& P, hipStream_t st);
 // Tetramers of the cloud (pass 0: counts and offsets[np + 1]; pass 1: out, 4 ints each, at most
 // cap); *ovf receives the largest match count of a query that overflowed the match storage.
 hipError_t launch_tetra(const PtInfo* pinfo, const double* cx, const double* cy, const double* cz, int np, int ns,
