@@ -28,8 +28,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <map>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -130,17 +128,42 @@ const SymTable* sym_table(const std::string& structure) {
     return nullptr;
 }
 
-// The fitted coefficients' kernel form, computed once per process (some 0.3 ms for all the tables).
-const std::vector<double>& default_coefficients(const SymTable* t, const double* fit, int n) {
-    static std::mutex mu;
-    static std::map<const double*, std::vector<double>> done;
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = done.find(fit);
-    if (it == done.end()) it = done.emplace(fit, kernel_coefficients(t, fit, n)).first;
-    return it->second;
-}
+// Every table's fitted coefficients in their kernel form, in the order of coef_views, computed once per
+// process (some 0.3 ms); table k starts at at[k], on a 128-byte boundary.
+constexpr int kCoefTables = 7 + kXFam;
+struct DefaultCoefficients {
+    std::vector<double> data;
+    size_t at[kCoefTables];
+};
 
-int kernel_slots(const SymTable* t, int n) { return t ? t->nrow + t->nlow : n; }
+const DefaultCoefficients& default_coefficients() {
+    static const DefaultCoefficients D = [] {
+        DefaultCoefficients d;
+        int k = 0;
+        auto add = [&](const char* structure, const double* fit, int n) {
+            d.data.resize((d.data.size() + 15) / 16 * 16);
+            d.at[k++] = d.data.size();
+            const std::vector<double> b = kernel_coefficients(sym_table(structure), fit, n);
+            d.data.insert(d.data.end(), b.begin(), b.end());
+        };
+        add("mbpol_2b", kFit_mbpol_2b, kNCoef_mbpol_2b);
+        add("mbpol_3b", kFit_mbpol_3b, kNCoef_mbpol_3b);
+        add("ch4h2o_2b", kFit_ch4h2o_2b, kNCoef_ch4h2o_2b);
+        add("ch4ch4_2b", kFit_ch4ch4_2b, kNCoef_ch4ch4_2b);
+        add("ch4h2o2_3b", kFit_ch4h2o2_3b, kNCoef_ch4h2o2_3b);
+        int n = 0;
+        const double* fit = ch4_1b_fit(&n);
+        add("", fit, n);
+        fit = co2_1b_fit(&n);
+        add("", fit, n);
+        for (int f = 0; f < kXFam; ++f) {
+            fit = xfam_default_coef(f, &n);
+            add(xfam_structure(f), fit, n);
+        }
+        return d;
+    }();
+    return D;
+}
 
 template <class T>
 struct DBuf {
@@ -164,6 +187,11 @@ struct DBuf {
         p = nullptr;
         n = 0;
     }
+};
+
+// One coefficient table in the context's coefficient buffer.
+struct CoefView {
+    double* p = nullptr;
 };
 
 // Neighbour-search and list state (both orders share one gather).
@@ -229,8 +257,10 @@ struct mbxg_ctx {
     // state
     Box box{};
     double cut2 = 0.0, cut3 = 0.0;
-    DBuf<double> d_in, d_xyz, d_grad, d_totals, d_coef2, d_coef3;
-    DBuf<double> d_coefn[kFamilies];  // MB-nrg coefficient tables (families 1, 2, 4)
+    DBuf<double> d_in, d_xyz, d_grad, d_totals;
+    DBuf<double> d_coef;                // every coefficient table; the views below point into it
+    CoefView d_coef2, d_coef3;
+    CoefView d_coefn[kFamilies];      // MB-nrg coefficient tables (families 1, 2, 4)
     DBuf<double> d_fam_tot;           // per family: energy + 6 virial components
     DBuf<Box> d_box;
     // configurations (mbxg_set_batch): monomers [mon_off[c], mon_off[c+1]) form configuration c;
@@ -258,7 +288,8 @@ struct mbxg_ctx {
     // 1B term (MBXG_1B): the local waters, then the local CH4s; per monomer energy and virial rows
     std::vector<int> water_local, ch4_local, co2_local;
     DBuf<int> d_w1b;
-    DBuf<double> d_e1b, d_v1b, d_coef1b, d_coef1b_co2;
+    DBuf<double> d_e1b, d_v1b;
+    CoefView d_coef1b, d_coef1b_co2;
     bool one_body_last = false;  // the last compute evaluated the 1B term
     DBuf<double> d_wrap_in, d_wrap_out;  // mbxg_fix_coordinates
     int n_h2o = 0, n_ch4 = 0;             // monomers of each kind (mbxg_set_topology)
@@ -275,11 +306,11 @@ struct mbxg_ctx {
     // further MB-nrg families and the 4B term (xfam.hip); they run synchronously
     double cut4 = 0.0;
     bool has_xkind = false;                  // the topology holds co2 or ion monomers
-    DBuf<int> x_code, x_blk, x_off, x_tot;   // classification scratch; x_tot: [order 2, 3, 4][kXFam]
+    DBuf<int> x_code[3], x_blk[3], x_off[3], x_tot;  // classification scratch per order; x_tot: [3][kXFam]
     DBuf<int> x_list[kXFam];
     int x_count[kXFam] = {};
     EvalState xf[kXFam];
-    DBuf<double> d_xcoef[kXFam];
+    CoefView d_xcoef[kXFam];
     DBuf<double> d_xfam_tot;                 // per further family: energy + 6 virial components
     DBuf<int> t_counts, t_off, t_list, t_ovf;  // tetramers
     int64_t n4_listed = 0;
@@ -290,6 +321,18 @@ struct mbxg_ctx {
     size_t host_atoms_n = 0;
     bool recomputed = false;                 // the last finish() computed again (lists had outgrown)
 };
+
+// The context's coefficient tables in the order of default_coefficients().
+static void coef_views(mbxg_ctx* c, CoefView** v) {
+    *v++ = &c->d_coef2;
+    *v++ = &c->d_coef3;
+    *v++ = &c->d_coefn[FAM_CH4H2O_2B];
+    *v++ = &c->d_coefn[FAM_CH4CH4_2B];
+    *v++ = &c->d_coefn[FAM_CH4H2O2_3B];
+    *v++ = &c->d_coef1b;
+    *v++ = &c->d_coef1b_co2;
+    for (CoefView& x : c->d_xcoef) *v++ = &x;
+}
 
 int mbxg::report_error(int code, const char* msg) {
     g_err = msg;
@@ -319,42 +362,20 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
         return fail(MBXG_ENOMEM, "mbxg_create: pinned host allocation failed");
     }
     std::memset(c->host, 0, sizeof(Published));
-    int n1b = 0, n1b_co2 = 0;
-    const double* fit1b = ch4_1b_fit(&n1b);
-    const double* fit1b_co2 = co2_1b_fit(&n1b_co2);
+    // every coefficient table in its kernel form: one allocation, one copy
+    const DefaultCoefficients& D = default_coefficients();
     // totals: 2B record, 3B record, 1B record, 4B record (kPartials each)
-    bool xbad = false;
-    for (int f = 0; f < kXFam; ++f) {
-        int nx = 0;
-        xfam_default_coef(f, &nx);
-        xbad = xbad || c->d_xcoef[f].reserve(kernel_slots(sym_table(xfam_structure(f)), nx));
-    }
-    if (xbad || c->d_xfam_tot.reserve(kXFam * kPartials) || c->d_coef2.reserve(kNSlot_mbpol_2b) ||
-        c->d_coef3.reserve(kNSlot_mbpol_3b) || c->d_totals.reserve(4 * kPartials) || c->d_coef1b.reserve(n1b) ||
-        c->d_coef1b_co2.reserve(n1b_co2) ||
-        c->d_box.reserve(1) || c->d_fam_tot.reserve(kFamilies * kPartials) ||
-        c->d_coefn[FAM_CH4H2O_2B].reserve(kNSlot_ch4h2o_2b) || c->d_coefn[FAM_CH4CH4_2B].reserve(kNSlot_ch4ch4_2b) ||
-        c->d_coefn[FAM_CH4H2O2_3B].reserve(kNSlot_ch4h2o2_3b)) {
+    if (c->d_coef.reserve(D.data.size()) || c->d_xfam_tot.reserve(kXFam * kPartials) ||
+        c->d_totals.reserve(4 * kPartials) || c->d_box.reserve(1) || c->d_fam_tot.reserve(kFamilies * kPartials)) {
+        (void)hipHostFree(c->host);
         delete c;
         return fail(MBXG_ENOMEM, "mbxg_create: device allocation failed");
     }
-    auto upload = [](double* dst, const SymTable* t, const double* fit, int n) {
-        const std::vector<double>& b = default_coefficients(t, fit, n);
-        return hipMemcpy(dst, b.data(), sizeof(double) * b.size(), hipMemcpyHostToDevice);
-    };
-    HIPCHK(upload(c->d_coef2.p, sym_table("mbpol_2b"), kFit_mbpol_2b, kNCoef_mbpol_2b));
-    HIPCHK(hipMemcpy(c->d_coef1b.p, fit1b, sizeof(double) * n1b, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(c->d_coef1b_co2.p, fit1b_co2, sizeof(double) * n1b_co2, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->d_coef.p, D.data.data(), sizeof(double) * D.data.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->d_totals.p, 0, sizeof(double) * 4 * kPartials));
-    for (int f = 0; f < kXFam; ++f) {
-        int nx = 0;
-        const double* fit = xfam_default_coef(f, &nx);
-        HIPCHK(upload(c->d_xcoef[f].p, sym_table(xfam_structure(f)), fit, nx));
-    }
-    HIPCHK(upload(c->d_coef3.p, sym_table("mbpol_3b"), kFit_mbpol_3b, kNCoef_mbpol_3b));
-    HIPCHK(upload(c->d_coefn[FAM_CH4H2O_2B].p, sym_table("ch4h2o_2b"), kFit_ch4h2o_2b, kNCoef_ch4h2o_2b));
-    HIPCHK(upload(c->d_coefn[FAM_CH4CH4_2B].p, sym_table("ch4ch4_2b"), kFit_ch4ch4_2b, kNCoef_ch4ch4_2b));
-    HIPCHK(upload(c->d_coefn[FAM_CH4H2O2_3B].p, sym_table("ch4h2o2_3b"), kFit_ch4h2o2_3b, kNCoef_ch4h2o2_3b));
+    CoefView* views[kCoefTables];
+    coef_views(c, views);
+    for (int k = 0; k < kCoefTables; ++k) views[k]->p = c->d_coef.p + D.at[k];
     c->box.periodic = 0;
     *out = c;
     return MBXG_OK;
@@ -397,8 +418,6 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
     c->d_conf_tot.release();
     c->d_conf_part.release();
     c->d_fam_tot.release();
-    for (DBuf<double>& b : c->d_coefn) b.release();
-    for (DBuf<double>& b : c->d_xcoef) b.release();
     for (DBuf<int>& b : c->x_list) b.release();
     for (EvalState* o = c->xf; o != c->xf + kXFam; ++o) {
         o->e_nmer.release();
@@ -406,9 +425,11 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
         o->ws.release();
     }
     c->d_xfam_tot.release();
-    c->x_code.release();
-    c->x_blk.release();
-    c->x_off.release();
+    for (int k = 0; k < 3; ++k) {
+        c->x_code[k].release();
+        c->x_blk[k].release();
+        c->x_off[k].release();
+    }
     c->x_tot.release();
     c->t_counts.release();
     c->t_off.release();
@@ -433,12 +454,9 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
     c->d_w1b.release();
     c->d_e1b.release();
     c->d_v1b.release();
-    c->d_coef1b.release();
-    c->d_coef1b_co2.release();
     c->d_wrap_in.release();
     c->d_wrap_out.release();
-    c->d_coef2.release();
-    c->d_coef3.release();
+    c->d_coef.release();
     c->d_box.release();
     for (hipEvent_t& e : c->ev)
         if (e) (void)hipEventDestroy(e);
@@ -1105,8 +1123,8 @@ void drop_graph(mbxg_ctx* c) {
 }
 
 // One compute: lists, then the evaluation of the requested terms.
-// The further MB-nrg families and the 4B term, after the others (synchronous: each order's
-// family counts are read back to size its evaluate lists).  Tetramers are listed when the 4B term
+// The further MB-nrg families and the 4B term, after the others (synchronous: the families' counts are
+// read back to size their evaluate lists).  Tetramers are listed when the 4B term
 // is wanted; listed dimers / trimers are classified when the topology holds co2 or halides.
 int run_xfam(mbxg_ctx* c, const NmerCtx& N, bool want2, bool want3, bool want4, bool eval, int do_grads) {
     hipStream_t st = c->stream;
@@ -1114,7 +1132,6 @@ int run_xfam(mbxg_ctx* c, const NmerCtx& N, bool want2, bool want3, bool want4, 
     const int np = c->np;
     c->n4_listed = 0;
     for (int f = 0; f < kXFam; ++f) c->x_count[f] = 0;
-    launch_zero(c->d_xfam_tot.p, (size_t)kXFam * kPartials, st);
     if (c->x_tot.reserve(3 * kXFam)) return fail(MBXG_ENOMEM, "further families: device allocation failed");
     if (want4 && np >= 4) {
         const int ns = np * (c->box.periodic ? 8 : 1);
@@ -1135,6 +1152,7 @@ int run_xfam(mbxg_ctx* c, const NmerCtx& N, bool want2, bool want3, bool want4, 
         HIPCHK(launch_tetra(L.pinfo.p, L.cx.p, L.cy.p, L.cz.p, np, ns, N, c4sq, 1, c->t_counts.p, c->t_off.p,
                             c->t_list.p, h[0], c->t_ovf.p, st));
     }
+    XJobs J{};
     if (eval) {
         struct Ord {
             int order;
@@ -1144,44 +1162,42 @@ int run_xfam(mbxg_ctx* c, const NmerCtx& N, bool want2, bool want3, bool want4, 
         const Ord ords[3] = {{2, L.list2.p, want2 && c->has_xkind ? L.tot.x : 0},
                              {3, L.list3.p, want3 && c->has_xkind ? L.tot.z : 0},
                              {4, c->t_list.p, want4 ? (int)c->n4_listed : 0}};
-        double* grad = do_grads ? c->d_grad.p : nullptr;
+        bool any = false;
         for (const Ord& o : ords) {
             if (o.n <= 0) continue;
+            const int k = o.order - 2;
             const size_t nb = xclass_blocks(o.n);
-            if (c->x_code.reserve(o.n) || c->x_blk.reserve(nb * kXFam) || c->x_off.reserve(nb * kXFam))
+            if (c->x_code[k].reserve(o.n) || c->x_blk[k].reserve(nb * kXFam) || c->x_off[k].reserve(nb * kXFam))
                 return fail(MBXG_ENOMEM, "further families: device allocation failed");
-            int* tot = c->x_tot.p + (o.order - 2) * kXFam;
-            HIPCHK(launch_xclass(o.order, o.list, o.n, N, c->fam_mask >> kFamilies, c->x_code.p, c->x_blk.p,
-                                 c->x_off.p, tot, st));
-            int cnt[kXFam];
-            HIPCHK(hipMemcpyAsync(cnt, tot, sizeof(cnt), hipMemcpyDeviceToHost, st));
+            HIPCHK(launch_xclass(o.order, o.list, o.n, N, c->fam_mask >> kFamilies, c->x_code[k].p, c->x_blk[k].p,
+                                 c->x_off[k].p, c->x_tot.p + k * kXFam, st));
+            any = true;
+        }
+        int cnt[3 * kXFam] = {};
+        if (any) {  // the one wait: the families' counts size their lists and workspaces
+            HIPCHK(hipMemcpyAsync(cnt, c->x_tot.p, sizeof(cnt), hipMemcpyDeviceToHost, st));
             HIPCHK(hipStreamSynchronize(st));
-            XLists X;
+        }
+        for (const Ord& o : ords) {
+            if (o.n <= 0) continue;
+            const int k = o.order - 2;
+            XLists X{};
             for (int f = 0; f < kXFam; ++f) {
-                X.list[f] = nullptr;
-                X.cap[f] = 0;
-                if (xfam_order(f) != o.order || cnt[f] <= 0) continue;
-                c->x_count[f] = cnt[f];
+                const int n = cnt[k * kXFam + f];
+                if (xfam_order(f) != o.order || n <= 0) continue;
+                c->x_count[f] = n;
                 EvalState& e = c->xf[f];
-                if (c->x_list[f].reserve((size_t)(o.order + 1) * cnt[f]) || e.e_nmer.reserve(cnt[f]) ||
-                    e.partials.reserve((size_t)kPartials * partials_records(cnt[f])) ||
-                    e.ws.reserve(xfam_workspace(f, cnt[f])))
+                if (c->x_list[f].reserve((size_t)(o.order + 1) * n) || e.e_nmer.reserve(n) ||
+                    e.partials.reserve((size_t)kPartials * partials_records(n)) || e.ws.reserve(xfam_workspace(f, n)))
                     return fail(MBXG_ENOMEM, "further families: device allocation failed");
                 X.list[f] = c->x_list[f].p;
-                X.cap[f] = cnt[f];
+                X.cap[f] = n;
+                xfam_job(f, X.list[f], n, c->d_xcoef[f].p, e.e_nmer.p, e.partials.p, e.ws.p, J.job[f]);
             }
-            HIPCHK(launch_xemit(o.order, o.list, o.n, c->x_code.p, c->x_off.p, X, st));
-            for (int f = 0; f < kXFam; ++f) {
-                if (!X.cap[f]) continue;
-                EvalState& e = c->xf[f];
-                HIPCHK(launch_xfam(f, X.list[f], tot + f, cnt[f], N, c->d_xcoef[f].p, grad, e.e_nmer.p, e.partials.p,
-                                   e.ws.p, st));
-                hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(256), 0, st, e.partials.p, tot + f, cnt[f],
-                                   c->d_xfam_tot.p + (size_t)kPartials * f);
-                HIPCHK(hipGetLastError());
-            }
+            HIPCHK(launch_xemit(o.order, o.list, o.n, c->x_code[k].p, c->x_off[k].p, X, st));
         }
     }
+    HIPCHK(launch_xfams(J, N, do_grads ? c->d_grad.p : nullptr, c->d_xfam_tot.p, st));
     HIPCHK(launch_xcombine(c->d_xfam_tot.p, c->d_totals.p, publish_job(c), st));
     return MBXG_OK;
 }

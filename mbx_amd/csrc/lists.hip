@@ -1161,31 +1161,6 @@ __global__ void k_zero_int(int* __restrict__ p, size_t n) {
         p[i] = 0;
 }
 
-// Deterministic sum of per-wave partial records (kPartials doubles each) into out[kPartials]:
-// one workgroup, fixed strided accumulation and a fixed tree.  The record count comes from the
-// evaluated n-mer count on the device (ceil(n / 64), n clamped to the capacity).
-__global__ void __launch_bounds__(256) k_reduce_partials(const double* __restrict__ partials,
-                                                         const int* __restrict__ n_dev, int n_cap,
-                                                         double* __restrict__ out) {
-    __shared__ double sh[kPartials][256];
-    const int t = threadIdx.x;
-    int n = *n_dev;
-    n = n < n_cap ? n : n_cap;
-    const int nb = (n + 63) / 64;
-    double acc[kPartials];
-    for (int q = 0; q < kPartials; ++q) acc[q] = 0.0;
-    for (int b = t; b < nb; b += 256)
-        for (int q = 0; q < kPartials; ++q) acc[q] += partials[(size_t)b * kPartials + q];
-    for (int q = 0; q < kPartials; ++q) sh[q][t] = acc[q];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (t < s)
-            for (int q = 0; q < kPartials; ++q) sh[q][t] += sh[q][t + s];
-        __syncthreads();
-    }
-    if (t < kPartials) out[t] = sh[t][0];
-}
-
 __global__ void __launch_bounds__(256) k_reduce_configs(ConfigJobs J, const int* __restrict__ pt_off,
                                                         double* __restrict__ part) {
     __shared__ double sh[4][kPartials];

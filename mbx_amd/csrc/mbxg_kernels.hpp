@@ -288,10 +288,6 @@ hipError_t launch_poly_mbpol3b(const double* xs, const int* n_dev, int cap, int 
 hipError_t launch_poly_ch4h2o2_3b(const double* xs, const int* n_dev, int cap, int ld, const double* coef,
                                   int do_grads, double* gs, double* ps, int split, hipStream_t st);
 
-// Sum the partial records of min(*n_dev, n_cap) n-mers into out[kPartials] in a fixed order
-// (deterministic totals).
-__global__ void k_reduce_partials(const double* partials, const int* n_dev, int n_cap, double* out);
-
 // Per-configuration totals in two fixed-order levels, all families in one launch each: block (c, s, f) of
 // a (nconf, S, kFamilies) grid sums slice s of configuration c's evaluated n-mers of family f (null e_out:
 // not evaluated), [offsets[pt_off[c]].comp, offsets[pt_off[c+1]].comp) clamped to cap, from e_out / vir_out

@@ -44,13 +44,12 @@ constexpr size_t poly_lds_bytes(int P) { return (size_t)(P - 1) * (kRedChunk + 1
 
 // One block's work: 64 n-mers of group `grp`, P = blockDim.x / 64 wavefronts.
 template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM>
-__device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict__ xs, const int* __restrict__ n_dev,
-                                              int cap, int ld, uint64_t coef_addr, double* __restrict__ gs,
-                                              double* __restrict__ ps, double* red) {
+__device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict__ xs, int n, int ld,
+                                              uint64_t coef_addr, double* __restrict__ gs, double* __restrict__ ps,
+                                              double* red) {
     const int P = blockDim.x >> 6;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t = grp * 64 + lane;
-    const int n = min(*n_dev, cap);
     if (grp * 64 >= n) return;  // the whole block is past the end (uniform per block)
     const bool active = t < n;
     const mbxg_cptr C = (mbxg_cptr)coef_addr;
@@ -101,7 +100,7 @@ __global__ void __launch_bounds__(64 * poly_max_split(WPE)) __attribute__((amdgp
     k_poly_eg(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap, int ld, uint64_t coef_addr,
               double* __restrict__ gs, double* __restrict__ ps) {
     extern __shared__ double red[];  // [P-1][kRedChunk+1][64]
-    poly_eg_group<NV, Q, PART, SYM>(blockIdx.x, xs, n_dev, cap, ld, coef_addr, gs, ps, red);
+    poly_eg_group<NV, Q, PART, SYM>(blockIdx.x, xs, min(*n_dev, cap), ld, coef_addr, gs, ps, red);
 }
 
 // Two polynomials in one launch: blocks [0, nb_a) evaluate polynomial A (groups of 64 n-mers in
@@ -121,9 +120,44 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 3))
     k_poly_eg_pair(PolyJob A, PolyJob B, int nb_a) {
     extern __shared__ double red[];
     if ((int)blockIdx.x < nb_a)
-        poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
+        poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, min(*A.n_dev, A.cap), A.ld, A.coef_addr, A.gs, A.ps, red);
     else
-        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
+        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, min(*B.n_dev, B.cap), B.ld, B.coef_addr, B.gs, B.ps, red);
+}
+
+// One polynomial over several n-mer lists with their own coefficients, in one launch: the further
+// families that share a structure hold a few hundred n-mers each, so a launch a family is all latency.
+constexpr int kMaxPolyLists = 5;
+struct PolyList {
+    const double* xs;
+    uint64_t coef_addr;
+    double* gs;
+    double* ps;
+    int n, ld;
+};
+struct PolyLists {
+    PolyList list[kMaxPolyLists];
+    int count;
+};
+
+template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM, int WPE>
+__global__ void __launch_bounds__(64 * poly_max_split(WPE)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+    k_poly_eg_lists(PolyLists J) {
+    extern __shared__ double red[];
+    int grp = blockIdx.x, k = 0;
+    while (k < J.count - 1 && grp >= (J.list[k].n + 63) / 64) grp -= (J.list[k++].n + 63) / 64;
+    const PolyList& L = J.list[k];
+    poly_eg_group<NV, Q, PART, SYM>(grp, L.xs, L.n, L.ld, L.coef_addr, L.gs, L.ps, red);
+}
+
+template <int NV, int Q, poly_eg_part_fn PEG, poly_sym_fn SYM, int WPE>
+hipError_t launch_poly_eg_lists(const PolyLists& J, int P, hipStream_t st) {
+    int groups = 0;
+    for (int k = 0; k < J.count; ++k) groups += (J.list[k].n + 63) / 64;
+    if (groups == 0) return hipSuccess;
+    if (P > poly_max_split(WPE)) P = poly_max_split(WPE);
+    hipLaunchKernelGGL((k_poly_eg_lists<NV, Q, PEG, SYM, WPE>), dim3(groups), dim3(64 * P), poly_lds_bytes(P), st, J);
+    return hipGetLastError();
 }
 
 // Energy only.

@@ -57,11 +57,11 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 3))
     k_poly_eg_pair_chain3(PolyJob A, PolyJob B, int nb_a, NmerCtx N, Chain3Job C) {
     extern __shared__ double red[];
     if ((int)blockIdx.x >= nb_a) {
-        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, B.n_dev, B.cap, B.ld, B.coef_addr, B.gs, B.ps, red);
+        poly_eg_group<NVB, QB, PB, SB>(blockIdx.x - nb_a, B.xs, min(*B.n_dev, B.cap), B.ld, B.coef_addr, B.gs, B.ps, red);
         return;
     }
-    poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, A.n_dev, A.cap, A.ld, A.coef_addr, A.gs, A.ps, red);
     const int n = min(*A.n_dev, A.cap);
+    poly_eg_group<NVA, QA, PA, SA>(blockIdx.x, A.xs, n, A.ld, A.coef_addr, A.gs, A.ps, red);
     if ((threadIdx.x >> 6) != 0 || (int)blockIdx.x * 64 >= n) return;
     // this wavefront's gs / ps stores are complete before it loads them back
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");

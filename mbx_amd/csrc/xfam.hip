@@ -21,10 +21,12 @@
 //   k_xclass    family, holder order and skip rule of every listed n-mer; per-block counts
 //   k_xscan     block offsets and family totals (one workgroup, fixed order)
 //   k_xemit     each evaluated n-mer at its family's list, in listed order (deterministic)
-// then per family: k_xvars (sites, variables, switch) -> polynomial (gen/xpoly_*.hip)
-// -> k_xgrad (chain rule, switch derivatives, energy, virial, gradient scatter).
+// then over all families: k_xvars (sites, variables) -> each structure's polynomial (gen/xpoly_*.hip)
+// -> k_xgrad (chain rule, switch derivatives, energy, virial, gradient scatter) -> k_xreduce.
 // Tetramers (System::Get4B, AddClusters with nmax = 4, sys_tools.cpp:594-634): k_tetra counts
 // and writes, per query, every match triple the center-3-neighbour rule keeps.
+#include <string>
+
 #include "gen/xholder_br_h2o2_3b.inc"
 #include "gen/xholder_br_h2o_2b.inc"
 #include "gen/xholder_cl_h2o2_3b.inc"
@@ -70,6 +72,7 @@
 #include "mbxg_device.hpp"
 #include "mbxg_kernels.hpp"
 #include "nrg_kernel.hpp"
+#include "poly_kernel.hpp"
 #include "scatter.hpp"
 #include "xfam.hpp"
 
@@ -292,30 +295,33 @@ __global__ void __launch_bounds__(kXBlock) k_xclass(const int* __restrict__ list
     }
 }
 
-// Pass 2 (one workgroup): exclusive scan of the block counts per family; tot[f] = totals.
-__global__ void __launch_bounds__(1024) k_xscan(const int* __restrict__ blk, int nblk, int* __restrict__ off,
-                                                int* __restrict__ tot) {
-    __shared__ int sh[1024];
-    const int t = threadIdx.x;
-    for (int f = 0; f < kXFam; ++f) {
-        int base = 0;
-        for (int b0 = 0; b0 < nblk; b0 += 1024) {
-            const int b = b0 + t;
-            const int v = b < nblk ? blk[(size_t)b * kXFam + f] : 0;
-            sh[t] = v;
-            __syncthreads();
-            for (int s = 1; s < 1024; s <<= 1) {
-                const int a = t >= s ? sh[t - s] : 0;
-                __syncthreads();
-                sh[t] += a;
-                __syncthreads();
-            }
-            if (b < nblk) off[(size_t)b * kXFam + f] = base + sh[t] - v;
-            base += sh[1023];
-            __syncthreads();
+// Pass 2 (a workgroup per family): exclusive scan of the family's block counts; tot[f] = totals.
+constexpr int kXScan = 256;
+
+__global__ void __launch_bounds__(kXScan) k_xscan(const int* __restrict__ blk, int nblk, int* __restrict__ off,
+                                                  int* __restrict__ tot) {
+    __shared__ int ws[kXScan / 64];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, f = blockIdx.x;
+    int base = 0;
+    for (int b0 = 0; b0 < nblk; b0 += kXScan) {
+        const int b = b0 + t;
+        const int v = b < nblk ? blk[(size_t)b * kXFam + f] : 0;
+        int incl = v;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
         }
-        if (t == 0) tot[f] = base;
+        if (lane == 63) ws[wv] = incl;
+        __syncthreads();
+        int at = base + incl - v;
+        for (int w = 0; w < kXScan / 64; ++w) {
+            if (w < wv) at += ws[w];
+            base += ws[w];
+        }
+        if (b < nblk) off[(size_t)b * kXFam + f] = at;
+        __syncthreads();
     }
+    if (t == 0) tot[f] = base;
 }
 
 // Pass 3: every evaluated n-mer to its family's list at its offset: K monomer ids in the
@@ -471,14 +477,11 @@ __device__ __forceinline__ double xswitches(const double* x, double (*d)[3], dou
     return sw;
 }
 
-}  // namespace
-
-// Stage 1: variables and the switch combination.
+// Stage 1 of one n-mer: its variables.
 template <class H>
-__global__ void __launch_bounds__(64) k_xvars(const int* __restrict__ list, const int* __restrict__ n_dev, int cap,
-                                              NmerCtx N, double* __restrict__ xs, double* __restrict__ sw, int ld) {
-    const int t = blockIdx.x * 64 + threadIdx.x;
-    if (t >= min(*n_dev, cap)) return;
+__device__ __forceinline__ void xvars(int t, const int* __restrict__ list, int n, const NmerCtx& N,
+                                      double* __restrict__ xs, int ld) {
+    if (t >= n) return;
     double x[3 * H::kNSites], oh1[2][3], oh2[2][3];
     xsites<H>(N, list + (size_t)(H::kMon + 1) * t, x, oh1, oh2);
     static_for<H::kNVars>([&](auto J) {
@@ -486,8 +489,6 @@ __global__ void __launch_bounds__(64) k_xvars(const int* __restrict__ list, cons
         double dv[3], gg;
         xs[(size_t)j * ld + t] = xvalue<H, j>(x, dv, gg);
     });
-    double d[6][3], r[6], s[6], g[6];
-    sw[t] = xswitches<H>(x, d, r, s, g);
 }
 
 constexpr int kGradBlockX = 128;
@@ -497,14 +498,11 @@ constexpr int kGradBlockX = 128;
 // along every pair; virial -sum_atoms x (x) g; gradient scatter.  grad == nullptr: energies only
 // (the reference computes the virial with the gradients only).
 template <class H>
-__global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ list, const int* __restrict__ n_dev,
-                                                       int cap, NmerCtx N, const double* __restrict__ gs,
-                                                       const double* __restrict__ ps, int ld,
-                                                       double* __restrict__ grad, double* __restrict__ e_out,
-                                                       double* __restrict__ partials) {
-    __shared__ GradTable<H::kMon == 2 ? 256 : 128, 9> T;  // (as k_grad_nrg)
-    const int t = blockIdx.x * kGradBlockX + threadIdx.x;
-    const int n = min(*n_dev, cap);
+__device__ __forceinline__ void xgrad(int block, const int* __restrict__ list, int n, const NmerCtx& N,
+                                      const double* __restrict__ gs, const double* __restrict__ ps, int ld,
+                                      double* __restrict__ grad, double* __restrict__ e_out,
+                                      double* __restrict__ partials, GradTable<256, 9>& T) {
+    const int t = block * kGradBlockX + threadIdx.x;
     if (grad) {
         table_init(T);
         __syncthreads();
@@ -609,7 +607,7 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
         table_flush(T, grad);
     }
     e_sum = wave_sum(e_sum);
-    const int rec = blockIdx.x * (kGradBlockX / 64) + threadIdx.x / 64;
+    const int rec = block * (kGradBlockX / 64) + threadIdx.x / 64;
     double* out = partials + (size_t)rec * kPartials;
     const bool lead = (threadIdx.x & 63) == 0;
     if (lead) out[0] = e_sum;
@@ -618,6 +616,84 @@ __global__ void __launch_bounds__(kGradBlockX) k_xgrad(const int* __restrict__ l
         const double v = wave_sum(vir[q]);
         if (lead) out[1 + q] = v;
     }
+}
+
+}  // namespace
+
+// Both stages over every family that has n-mers, in one launch each: a solution holds a few hundred
+// n-mers of each of some twenty families, and a launch of its own a family and stage left the chip idle
+// (256 waters / ions / CO2: 80 launches of 5-30 us; see launch_xfams).  A block finds its family from its
+// index.  WIDE: the 4B family (its 66 variables take all registers of a SIMD); else the 2B and 3B ones.
+namespace {
+
+// Block `blockIdx.x` of blocks of `size` n-mers -> (family, block within it).
+template <bool WIDE>
+__device__ __forceinline__ int xblock(const XJobs& J, int size, int& block) {
+    block = blockIdx.x;
+    for (int f = 0; f < kXFam; ++f) {
+        if ((f == XF_H2OX4_4B) != WIDE) continue;
+        const int nb = (J.job[f].n + size - 1) / size;
+        if (block < nb) return f;
+        block -= nb;
+    }
+    return -1;
+}
+
+}  // namespace
+
+template <bool WIDE>
+__global__ void __launch_bounds__(64) k_xvars(XJobs J, NmerCtx N) {
+    int block;
+    const int f = xblock<WIDE>(J, 64, block);
+    if (f < 0) return;
+    const XJob& j = J.job[f];
+    const int t = block * 64 + threadIdx.x;
+    switch (f) {
+#define MBXG_XV(F, name, poly)                                                                         \
+    case F:                                                                                            \
+        if constexpr ((F == XF_H2OX4_4B) == WIDE) xvars<XHolder_##name>(t, j.list, j.n, N, j.xs, j.ld); \
+        break;
+        MBXG_XFAMILIES(MBXG_XV)
+#undef MBXG_XV
+    }
+}
+
+template <bool WIDE>
+__global__ void __launch_bounds__(kGradBlockX) k_xgrad(XJobs J, NmerCtx N, double* __restrict__ grad) {
+    __shared__ GradTable<256, 9> T;
+    int block;
+    const int f = xblock<WIDE>(J, kGradBlockX, block);
+    if (f < 0) return;
+    const XJob& j = J.job[f];
+    switch (f) {
+#define MBXG_XG(F, name, poly)                                                                              \
+    case F:                                                                                                 \
+        if constexpr ((F == XF_H2OX4_4B) == WIDE)                                                           \
+            xgrad<XHolder_##name>(block, j.list, j.n, N, j.gs, j.ps, j.ld, grad, j.e_out, j.partials, T);   \
+        break;
+        MBXG_XFAMILIES(MBXG_XG)
+#undef MBXG_XG
+    }
+}
+
+// Every family's partial records (one per 64 n-mers) into tot[f][kPartials], a workgroup per family, fixed
+// order; zeros for a family without n-mers.
+__global__ void __launch_bounds__(256) k_xreduce(XJobs J, double* __restrict__ tot) {
+    __shared__ double sh[4][kPartials];
+    const int f = blockIdx.x, t = threadIdx.x, nb = (J.job[f].n + 63) / 64;
+    double acc[kPartials];
+#pragma unroll
+    for (int q = 0; q < kPartials; ++q) acc[q] = 0.0;
+    for (int b = t; b < nb; b += 256)
+#pragma unroll
+        for (int q = 0; q < kPartials; ++q) acc[q] += J.job[f].partials[(size_t)b * kPartials + q];
+#pragma unroll
+    for (int q = 0; q < kPartials; ++q) {
+        const double v = wave_sum(acc[q]);
+        if ((t & 63) == 0) sh[t >> 6][q] = v;
+    }
+    __syncthreads();
+    if (t < kPartials) tot[f * kPartials + t] = sh[0][t] + sh[1][t] + sh[2][t] + sh[3][t];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -786,76 +862,85 @@ __global__ void __launch_bounds__(1024) k_scan_int(const int* __restrict__ cnt, 
 // Host launchers
 
 // The polynomial structures (gen/xpoly_<structure>.hip).
-#define MBXG_XPOLY(poly)                                                                                       \
-    hipError_t launch_xpoly_##poly(const double*, const int*, int, int, const double*, double*, double*, int, \
-                                   hipStream_t);
-MBXG_XPOLY(halide_h2o_2b)
-MBXG_XPOLY(co2co2_2b)
-MBXG_XPOLY(halide_h2o2_3b)
-MBXG_XPOLY(co2x3_3b)
-MBXG_XPOLY(h2ox4_4b)
-MBXG_XPOLY(alkali_h2o_2b)
-MBXG_XPOLY(alkali_h2o2_3b)
+#define MBXG_XPOLYS(X) \
+    X(halide_h2o_2b)   \
+    X(co2co2_2b)       \
+    X(alkali_h2o_2b)   \
+    X(halide_h2o2_3b)  \
+    X(co2x3_3b)        \
+    X(alkali_h2o2_3b)  \
+    X(h2ox4_4b)
+#define MBXG_XPOLY(poly) hipError_t launch_xpoly_##poly(const PolyLists&, int, hipStream_t);
+MBXG_XPOLYS(MBXG_XPOLY)
 #undef MBXG_XPOLY
-
-namespace {
-
-typedef hipError_t (*xpoly_launch)(const double*, const int*, int, int, const double*, double*, double*, int,
-                                   hipStream_t);
-
-template <class H>
-size_t xworkspace(int cap) {
-    const size_t ld = ((size_t)cap + 63) / 64 * 64;
-    return ((size_t)H::kNVars * 2 + 2) * ld;
-}
-
-template <class H>
-hipError_t xlaunch(xpoly_launch poly, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
-                   double* grad, double* e_out, double* partials, double* ws, hipStream_t st) {
-    if (cap <= 0) return hipSuccess;
-    const int nb = (cap + 63) / 64;
-    const int ld = nb * 64;
-    double* xs = ws;
-    double* gs = xs + (size_t)H::kNVars * ld;
-    double* ps = gs + (size_t)H::kNVars * ld;
-    double* sw = ps + ld;
-    hipLaunchKernelGGL(k_xvars<H>, dim3(nb), dim3(64), 0, st, list, n_dev, cap, N, xs, sw, ld);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = poly(xs, n_dev, cap, ld, coef, gs, ps, poly_split(cap, poly_wpe(H::kNVars)), st);
-    if (e != hipSuccess) return e;
-    const int ngb = (cap + kGradBlockX - 1) / kGradBlockX;
-    hipLaunchKernelGGL(k_xgrad<H>, dim3(ngb), dim3(kGradBlockX), 0, st, list, n_dev, cap, N, gs, ps, ld, grad, e_out,
-                       partials);
-    return hipGetLastError();
-}
-
-}  // namespace
 
 __host__ __device__ int xfam_order(int f) {
     if (f <= XF_CO2CO2_2B || (f >= XF_LI_H2O_2B && f <= XF_CS_H2O_2B)) return 2;
     return f == XF_H2OX4_4B ? 4 : 3;
 }
 
-size_t xfam_workspace(int f, int cap) {
+int xfam_variables(int f) {
     switch (f) {
 #define MBXG_XW(F, name, poly) \
-    case F: return xworkspace<XHolder_##name>(cap);
+    case F: return XHolder_##name::kNVars;
         MBXG_XFAMILIES(MBXG_XW)
 #undef MBXG_XW
         default: return 0;
     }
 }
 
-hipError_t launch_xfam(int f, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
-                       double* grad, double* e_out, double* partials, double* ws, hipStream_t st) {
-    switch (f) {
-#define MBXG_XL(F, name, poly) \
-    case F: return xlaunch<XHolder_##name>(launch_xpoly_##poly, list, n_dev, cap, N, coef, grad, e_out, partials, ws, st);
-        MBXG_XFAMILIES(MBXG_XL)
-#undef MBXG_XL
-        default: return hipErrorInvalidValue;
+// xs, gs (variables x ld each) and ps (ld).
+size_t xfam_workspace(int f, int cap) {
+    const size_t ld = ((size_t)cap + 63) / 64 * 64;
+    return ((size_t)xfam_variables(f) * 2 + 1) * ld;
+}
+
+void xfam_job(int f, const int* list, int n, const double* coef, double* e_out, double* partials, double* ws, XJob& j) {
+    j.n = n;
+    j.ld = (n + 63) / 64 * 64;
+    j.list = list;
+    j.coef = coef;
+    j.xs = ws;
+    j.gs = j.xs + (size_t)xfam_variables(f) * j.ld;
+    j.ps = j.gs + (size_t)xfam_variables(f) * j.ld;
+    j.e_out = e_out;
+    j.partials = partials;
+}
+
+hipError_t launch_xfams(const XJobs& J, const NmerCtx& N, double* grad, double* tot, hipStream_t st) {
+    int vb = 0, gb = 0;
+    for (int f = 0; f < kXFam; ++f)
+        if (f != XF_H2OX4_4B) {
+            vb += (J.job[f].n + 63) / 64;
+            gb += (J.job[f].n + kGradBlockX - 1) / kGradBlockX;
+        }
+    const int n4 = J.job[XF_H2OX4_4B].n;
+    if (vb) hipLaunchKernelGGL(k_xvars<false>, dim3(vb), dim3(64), 0, st, J, N);
+    if (n4) hipLaunchKernelGGL(k_xvars<true>, dim3((n4 + 63) / 64), dim3(64), 0, st, J, N);
+    // each structure's polynomial over the lists of its families
+#define MBXG_XP(poly_name)                                                                             \
+    {                                                                                                  \
+        PolyLists L{};                                                                                 \
+        int n = 0, nv = 0;                                                                             \
+        for (int f = 0; f < kXFam; ++f)                                                                \
+            if (J.job[f].n > 0 && std::string(xfam_structure(f)) == #poly_name) {                      \
+                const XJob& j = J.job[f];                                                              \
+                L.list[L.count++] = PolyList{j.xs, (uint64_t)(uintptr_t)j.coef, j.gs, j.ps, j.n, j.ld}; \
+                n += j.n;                                                                              \
+                nv = xfam_variables(f);                                                                \
+            }                                                                                          \
+        if (n > 0) {                                                                                   \
+            const hipError_t e = launch_xpoly_##poly_name(L, poly_split(n, poly_wpe(nv)), st);         \
+            if (e != hipSuccess) return e;                                                             \
+        }                                                                                              \
     }
+    MBXG_XPOLYS(MBXG_XP)
+#undef MBXG_XP
+    if (gb) hipLaunchKernelGGL(k_xgrad<false>, dim3(gb), dim3(kGradBlockX), 0, st, J, N, grad);
+    if (n4)
+        hipLaunchKernelGGL(k_xgrad<true>, dim3((n4 + kGradBlockX - 1) / kGradBlockX), dim3(kGradBlockX), 0, st, J, N, grad);
+    hipLaunchKernelGGL(k_xreduce, dim3(kXFam), dim3(256), 0, st, J, tot);
+    return hipGetLastError();
 }
 
 hipError_t launch_xclass(int order, const int* list, int n, const NmerCtx& N, int fam_mask, int* code, int* blk,
@@ -868,7 +953,7 @@ hipError_t launch_xclass(int order, const int* list, int n, const NmerCtx& N, in
         hipLaunchKernelGGL(k_xclass<3>, dim3(nb), dim3(kXBlock), 0, st, list, n, N, fam_mask, code, blk);
     else
         hipLaunchKernelGGL(k_xclass<4>, dim3(nb), dim3(kXBlock), 0, st, list, n, N, fam_mask, code, blk);
-    hipLaunchKernelGGL(k_xscan, dim3(1), dim3(1024), 0, st, blk, nb, blk_off, tot);
+    hipLaunchKernelGGL(k_xscan, dim3(kXFam), dim3(kXScan), 0, st, blk, nb, blk_off, tot);
     return hipGetLastError();
 }
 

@@ -54,10 +54,21 @@ hipError_t launch_xclass(int order, const int* list, int n, const NmerCtx& N, in
                          int* blk_off, int* tot, hipStream_t st);
 hipError_t launch_xemit(int order, const int* list, int n, const int* code, const int* blk_off, const XLists& X,
                         hipStream_t st);
-// One family over its evaluate list: energies e_out, one kPartials record per 64 n-mers
-// (partials_records(cap)), gradient added to grad; ws holds xfam_workspace(f, cap) doubles.
-hipError_t launch_xfam(int f, const int* list, const int* n_dev, int cap, const NmerCtx& N, const double* coef,
-                       double* grad, double* e_out, double* partials, double* ws, hipStream_t st);
+// The families' evaluate lists and buffers (n = 0: no n-mers): energies e_out, one kPartials record per 64
+// n-mers (partials_records(n)), a workspace of xfam_workspace(f, n) doubles.
+struct XJob {
+    const int* list;
+    const double* coef;
+    double *xs, *gs, *ps, *e_out, *partials;
+    int n, ld;
+};
+struct XJobs {
+    XJob job[kXFam];
+};
+void xfam_job(int f, const int* list, int n, const double* coef, double* e_out, double* partials, double* ws, XJob& j);
+// Evaluate all of them: gradient added to grad (null: energies only), the families' records to
+// tot[kXFam][kPartials].
+hipError_t launch_xfams(const XJobs& J, const NmerCtx& N, double* grad, double* tot, hipStream_t st);
 // The further families' energy records (kXFam x kPartials) added to the per-order totals
 // (records 2B, 3B, 1B, 4B), and published.
 hipError_t launch_xcombine(const double* xfam_tot, double* totals, const PublishJob& P, hipStream_t st);

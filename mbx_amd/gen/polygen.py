@@ -459,10 +459,8 @@ def generate_launcher(prefix, name, out_dir, energy_only):
                     nvars, NPARTS, fn, fn, fn, wpe),
                 "        P, st);", "}"]
     else:
-        out += ["hipError_t launch_%s(const double* xs, const int* n_dev, int cap, int ld, const double* coef, double* gs," % fn,
-                "    double* ps, int P, hipStream_t st) {",
-                "    return launch_poly_eg<%d, %d, %s_parts, %s_sym, %d>(xs, n_dev, cap, ld, coef, gs, ps, P, st);" % (
-                    nvars, NPARTS, fn, fn, wpe), "}"]
+        out += ["hipError_t launch_%s(const PolyLists& J, int P, hipStream_t st) {" % fn,
+                "    return launch_poly_eg_lists<%d, %d, %s_parts, %s_sym, %d>(J, P, st);" % (nvars, NPARTS, fn, fn, wpe), "}"]
     out += ["", "}  // namespace mbxg", ""]
     write_if_changed(os.path.join(out_dir, fn + ".hip"), "\n".join(out))
 
