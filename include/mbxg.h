@@ -220,19 +220,19 @@ int mbxg_set_graph(mbxg_ctx* ctx, int on);
 
 /* Schedule parameters.  "split_2b" / "split_3b": wavefronts (1, 2, 4 or 8) that share each
  * block of 64 dimers / trimers in the MB-pol polynomial stage, each evaluating 1/split of the
- * polynomial (defaults 4 and 2); "split_ch4h2o2_3b": the same for the CH4-H2O-H2O polynomial
- * (default 4); "fuse_poly" (0 or 1, default 1): the MB-pol 2B and 3B polynomials in one launch
- * when both run with gradients; "fuse_prep" (0 or 1, default 1): FixMonomerCoordinates, the
- * cloud and the cell counts in one launch; "fuse_chain" (0 or 1, default 1): with "fuse_poly", the
- * MB-pol 3B chain rule runs in the paired polynomial launch (each 3B block's tail) instead of a
- * kernel of its own; "fuse_vars" (0 or 1, default 1): with "fuse_poly", the 2B and 3B variables in
- * one launch.  mbxg_autotune times every split of both MB-pol orders
- * on the current inputs
+ * polynomial (until set: by the number of n-mers); "split_ch4h2o2_3b": the same for the
+ * CH4-H2O-H2O polynomial (default 4); "fuse_poly" (0 or 1, default 1): the MB-pol 2B and 3B
+ * polynomials in one launch when both run with gradients; "fuse_prep" (0 or 1, default 1):
+ * FixMonomerCoordinates, the cloud and the cell counts in one launch; "fuse_chain" (0 or 1,
+ * default 1): with "fuse_poly", the variables and chain rules of both orders run in that launch
+ * too, which is made for four wavefronts: a "split_3b" set to another number takes separate
+ * launches; "fuse_vars" (0 or 1, default 1): where those run, the 2B and 3B variables in one.
+ * mbxg_autotune times every split of both MB-pol orders on the current inputs
  * (the polynomial stage, `reps` timed repetitions after one warm-up) and, when CH4-H2O-H2O trimers
  * are evaluated, every split of that family (its whole evaluation), keeps the fastest of each,
- * then, on the paired path, every combination of "fuse_chain" and "fuse_vars" (the whole compute),
- * and recomputes once with them.  No counterpart in the reference (its kernels have no
- * launch shape). */
+ * then, on the paired path, the one launch against the separate ones with and without "fuse_vars"
+ * (the whole compute), and recomputes once with them.  No counterpart in the reference (its
+ * kernels have no launch shape). */
 int mbxg_set_tuning(mbxg_ctx* ctx, const char* key, int value);
 int mbxg_get_tuning(mbxg_ctx* ctx, const char* key, int* value);
 int mbxg_autotune(mbxg_ctx* ctx, int terms, int do_grads, int reps);

@@ -13,9 +13,7 @@
 //   k_compact_evals         evaluate lists (one-pass builds)
 //   1B, launch_mbpol2b/3b   variables, polynomials, chain rule over the evaluate lists; n-mer
 //   / MB-nrg families       counts read on the device.  With both MB-pol orders and gradients:
-//                           k_vars_mbpol_pair (both orders' variables), k_poly_eg_pair_chain3
-//                           (both polynomials, the 3B chain rule in the 3B blocks' tail),
-//                           k_grad_mbpol2b
+//                           k_mbpol_fused (variables, polynomials, chain rules of both orders)
 //   k_finish                deterministic energy / virial totals per family and per order
 //   run_xfam                (co2, ions, 4B) further families, synchronously
 // Capacities (list buffers, match storage) come from a synchronised first call and carry
@@ -293,12 +291,13 @@ struct mbxg_ctx {
     bool one_body_last = false;  // the last compute evaluated the 1B term
     DBuf<double> d_wrap_in, d_wrap_out;  // mbxg_fix_coordinates
     int n_h2o = 0, n_ch4 = 0;             // monomers of each kind (mbxg_set_topology)
-    // wavefronts per 64 n-mers in the polynomial stages (mbxg_set_tuning / mbxg_autotune)
-    int split2 = 4, split3 = 2, split3n = 4;
+    // wavefronts per 64 n-mers in the polynomial stages (mbxg_set_tuning / mbxg_autotune); 0: poly_split's
+    // rule.  CH4-H2O-H2O's is fixed, for a batch's gradients to be a lone configuration's to 1e-10.
+    int split2 = 0, split3 = 0, split3n = 4;
     int fuse_poly = 1;       // MB-pol 2B and 3B polynomials in one launch when both are evaluated
     int fuse_prep = 1;       // FixMonomerCoordinates, cloud and cell counts in one launch (k_cloud_fix)
-    int fuse_chain = 1;      // the 3B chain rule in the paired polynomial launch's 3B blocks
-    int fuse_vars = 1;       // the paired path's 2B and 3B variables in one launch
+    int fuse_chain = 1;      // variables and chain rules in the paired polynomial launch (k_mbpol_fused)
+    int fuse_vars = 1;       // without fuse_chain: the paired path's 2B and 3B variables in one launch
     bool fused_last = false;  // the last compute did so (its 2B polynomial time is in the 3B one)
     // stage timing (mbxg_set_timing): events bracketing each stage of the last compute
     bool timing = false;
@@ -1109,6 +1108,13 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
     return 0;
 }
 
+// The wavefronts per 64 n-mers of a polynomial of nv variables: as set, else by the rule.
+int split_of(int set, int cap, int nv) { return set ? set : poly_split(cap, poly_wpe(nv)); }
+
+// Whether MB-pol's paired path runs as one launch (mbpol_fused.hip: four wavefronts per 64 n-mers); another
+// split set by hand takes the separate launches, which have them all.
+bool one_launch(const mbxg_ctx* c) { return c->fuse_chain && (c->split3 == 0 || c->split3 == kFusedSplit); }
+
 PublishJob publish_job(const mbxg_ctx* c) {
     const ListState& L = c->L;
     if (!L.built) return {c->host, nullptr, nullptr, nullptr};
@@ -1288,7 +1294,10 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
             const int cap = fam_cap(L, f);
             EvalState& o = c->fam[f];
             const int ld = (cap + 63) / 64 * 64;
-            const size_t wsz = f == FAM_MBPOL_2B   ? workspace_mbpol2b(cap)
+            // the one-launch evaluation keeps its n-mers in LDS
+            const bool in_lds = fuse && one_launch(c) && (f == FAM_MBPOL_2B || f == FAM_MBPOL_3B);
+            const size_t wsz = in_lds              ? 0
+                               : f == FAM_MBPOL_2B ? workspace_mbpol2b(cap)
                                : f == FAM_MBPOL_3B ? workspace_mbpol3b(cap)
                                                    : workspace_nrg_family(f, cap);
             return !(o.e_nmer.reserve(cap) || o.partials.reserve((size_t)kPartials * partials_records(cap)) ||
@@ -1326,40 +1335,42 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                 const int f2 = FAM_MBPOL_2B, cap2 = fam_cap(L, f2);
                 EvalState& o2 = c->fam[f2];
                 const int* nd2 = fam_ndev(L, c->np, f2);
-                // all on the main stream (the 2B stages on stream2 beside the 3B ones measured
-                // slower: 0.641-0.646 against 0.636-0.637 ms a step at 2048 waters)
-                if (c->fuse_vars) {  // both orders' variables in one launch (timed as the 3B stage)
-                    if (ev) HIPCHK(hipEventRecord(ev[4], st));
-                    if (ev) HIPCHK(hipEventRecord(ev[5], st));
-                    if (ev) HIPCHK(hipEventRecord(ev[8], st));
-                    HIPCHK(launch_mbpol_vars_pair(L.evals[f].p, nd, cap, o.ws.p, L.evals[f2].p, nd2, cap2, o2.ws.p,
-                                                  N, st));
-                    if (ev) HIPCHK(hipEventRecord(ev[9], st));
+                // all on the main stream: the 2B work fills what the 3B blocks leave idle
+                double* vir2 = batch ? o2.vir_nmer.p : nullptr;
+                if (one_launch(c)) {  // everything in one launch (timed as the 3B polynomial)
+                    if (ev)
+                        for (int k = 4; k <= 9; ++k) HIPCHK(hipEventRecord(ev[k], st));
+                    const auto job = [&](const EvalState& e, const int* list, const int* n, int cp, const double* coef,
+                                         double* v) {
+                        return FusedJob{list, n, cp, (cp + 63) / 64 * 64, (uint64_t)(uintptr_t)coef, c->d_grad.p,
+                                        e.e_nmer.p, v, e.partials.p};
+                    };
+                    HIPCHK(launch_mbpol_fused(job(o, L.evals[f].p, nd, cap, c->d_coef3.p, vir),
+                                              job(o2, L.evals[f2].p, nd2, cap2, c->d_coef2.p, vir2), N, st));
+                    if (ev)
+                        for (int k = 10; k <= 11; ++k) HIPCHK(hipEventRecord(ev[k], st));
                 } else {
                     if (ev) HIPCHK(hipEventRecord(ev[4], st));
-                    HIPCHK(launch_mbpol2b_vars(L.evals[f2].p, nd2, cap2, N, o2.ws.p, st));
+                    if (!c->fuse_vars) HIPCHK(launch_mbpol2b_vars(L.evals[f2].p, nd2, cap2, N, o2.ws.p, st));
                     if (ev) HIPCHK(hipEventRecord(ev[5], st));
                     if (ev) HIPCHK(hipEventRecord(ev[8], st));
-                    HIPCHK(launch_mbpol3b_vars(L.evals[f].p, nd, cap, N, o.ws.p, st));
+                    if (c->fuse_vars)  // both orders' variables in one launch (timed as the 3B stage)
+                        HIPCHK(launch_mbpol_vars_pair(L.evals[f].p, nd, cap, o.ws.p, L.evals[f2].p, nd2, cap2, o2.ws.p,
+                                                      N, st));
+                    else
+                        HIPCHK(launch_mbpol3b_vars(L.evals[f].p, nd, cap, N, o.ws.p, st));
                     if (ev) HIPCHK(hipEventRecord(ev[9], st));
-                }
-                if (c->fuse_chain) {
-                    HIPCHK(launch_poly_mbpol_pair_chain3(o.ws.p, L.evals[f].p, nd, cap, c->d_coef3.p, o2.ws.p, nd2,
-                                                         cap2, c->d_coef2.p, c->split3, N, c->d_grad.p, o.e_nmer.p,
-                                                         vir, o.partials.p, st));
-                    if (ev) HIPCHK(hipEventRecord(ev[10], st));
-                } else {
                     HIPCHK(launch_poly_mbpol_pair(o.ws.p, nd, cap, c->d_coef3.p, o2.ws.p, nd2, cap2, c->d_coef2.p,
-                                                  c->split3, st));
+                                                  split_of(c->split3, cap, 36), st));
                     if (ev) HIPCHK(hipEventRecord(ev[10], st));
                     HIPCHK(launch_mbpol3b_chain(L.evals[f].p, nd, cap, N, 1, c->d_grad.p, o.e_nmer.p, vir,
                                                 o.partials.p, o.ws.p, st));
+                    if (ev) HIPCHK(hipEventRecord(ev[11], st));
+                    if (ev) HIPCHK(hipEventRecord(ev[6], st));
+                    HIPCHK(launch_mbpol2b_chain(L.evals[f2].p, nd2, cap2, N, 1, c->d_grad.p, o2.e_nmer.p, vir2,
+                                                o2.partials.p, o2.ws.p, st));
+                    if (ev) HIPCHK(hipEventRecord(ev[7], st));
                 }
-                if (ev) HIPCHK(hipEventRecord(ev[11], st));
-                if (ev) HIPCHK(hipEventRecord(ev[6], st));
-                HIPCHK(launch_mbpol2b_chain(L.evals[f2].p, nd2, cap2, N, 1, c->d_grad.p, o2.e_nmer.p,
-                                            batch ? o2.vir_nmer.p : nullptr, o2.partials.p, o2.ws.p, st));
-                if (ev) HIPCHK(hipEventRecord(ev[7], st));
                 reduce(f);
                 reduce(f2);
                 HIPCHK(hipGetLastError());
@@ -1367,15 +1378,16 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
             }
             if (f == FAM_MBPOL_2B)
                 HIPCHK(launch_mbpol2b(L.evals[f].p, nd, cap, N, c->d_coef2.p, do_grads, c->d_grad.p, o.e_nmer.p, vir,
-                                      o.partials.p, o.ws.p, c->split2, sk, ev ? ev + 4 : nullptr));
+                                      o.partials.p, o.ws.p, split_of(c->split2, cap, 31), sk, ev ? ev + 4 : nullptr));
             else if (f == FAM_MBPOL_3B)
                 HIPCHK(launch_mbpol3b(L.evals[f].p, nd, cap, N, c->d_coef3.p, do_grads, c->d_grad.p, o.e_nmer.p, vir,
-                                      o.partials.p, o.ws.p, c->split3, sk, ev ? ev + 8 : nullptr));
+                                      o.partials.p, o.ws.p, split_of(c->split3, cap, 36), sk, ev ? ev + 8 : nullptr));
             else {
                 const bool timed = ev && f == FAM_CH4H2O2_3B;
                 if (timed) HIPCHK(hipEventRecord(ev[13], st));
                 HIPCHK(launch_nrg_family(f, L.evals[f].p, nd, cap, N, c->d_coefn[f].p, do_grads, c->d_grad.p,
-                                         o.e_nmer.p, vir, o.partials.p, o.ws.p, c->split3n, sk, nullptr));
+                                         o.e_nmer.p, vir, o.partials.p, o.ws.p, split_of(c->split3n, cap, 55), sk,
+                                         nullptr));
                 if (timed) HIPCHK(hipEventRecord(ev[14], st));
             }
             reduce(f);
@@ -1597,9 +1609,7 @@ extern "C" int mbxg_set_tuning(mbxg_ctx* c, const char* key, int value) {
         c->fuse_vars = value;
     else
         return fail(MBXG_EINVAL, "mbxg_set_tuning: unknown key '%s'", key);
-    if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
-    c->gexec = nullptr;
-    c->g_terms = c->g_grads = -1;
+    drop_graph(c);  // another schedule may need other workspaces: an eager compute first
     return MBXG_OK;
 }
 
@@ -1607,11 +1617,11 @@ extern "C" int mbxg_get_tuning(mbxg_ctx* c, const char* key, int* value) {
     if (!c || !key || !value) return fail(MBXG_EINVAL, "mbxg_get_tuning: bad arguments");
     const std::string k(key);
     if (k == "split_2b")
-        *value = c->split2;
+        *value = split_of(c->split2, fam_cap(c->L, FAM_MBPOL_2B), 31);
     else if (k == "split_3b")
-        *value = c->split3;
+        *value = split_of(c->split3, fam_cap(c->L, FAM_MBPOL_3B), 36);
     else if (k == "split_ch4h2o2_3b")
-        *value = c->split3n;
+        *value = split_of(c->split3n, fam_cap(c->L, FAM_CH4H2O2_3B), 55);
     else if (k == "fuse_poly")
         *value = c->fuse_poly;
     else if (k == "fuse_prep")
@@ -1637,6 +1647,8 @@ extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
     const int cand[4] = {1, 2, 4, 8};
     double best[2] = {1e300, 1e300};
     int pick[2] = {c->split2, c->split3};
+    const int fuse_chain = c->fuse_chain;
+    c->fuse_chain = 0;  // the polynomial stage by itself
     for (int i = 0; i < 4; ++i) {
         c->split2 = c->split3 = cand[i];
         double t[2] = {1e300, 1e300};
@@ -1657,6 +1669,7 @@ extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
     }
     c->split2 = pick[0];
     c->split3 = pick[1];
+    c->fuse_chain = fuse_chain;
     if ((terms & MBXG_3B) && c->cut3 > 0.0 && family_launched(c, FAM_CH4H2O2_3B)) {
         double best3n = 1e300;
         int pick3n = c->split3n;
@@ -1676,16 +1689,17 @@ extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
         }
         c->split3n = pick3n;
     }
-    // The paired path's fusions (the 3B chain rule in the polynomial launch, both orders'
-    // variables in one launch): every combination, timed over the whole compute.
+    // The paired path as one launch, or separate ones with the split just found and the variables of both
+    // orders together or not: timed over the whole compute.
     if (c->fuse_poly && do_grads && (terms & MBXG_2B) && (terms & MBXG_3B) && family_launched(c, FAM_MBPOL_2B) &&
         family_launched(c, FAM_MBPOL_3B)) {
         double bestf = 1e300;
         int pickc = c->fuse_chain, pickv = c->fuse_vars;
         for (int fc = 0; fc < 2; ++fc)
-            for (int fv = 0; fv < 2; ++fv) {
+            for (int fv = 0; fv < 2 - fc; ++fv) {  // (one launch has no variables of its own)
                 c->fuse_chain = fc;
                 c->fuse_vars = fv;
+                c->split3 = fc ? kFusedSplit : pick[1];
                 double t = 1e300;
                 for (int r = 0; r < reps + 1; ++r) {
                     if (int e = mbxg_compute(c, terms, do_grads)) return e;
@@ -1701,6 +1715,7 @@ extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
             }
         c->fuse_chain = pickc;
         c->fuse_vars = pickv;
+        c->split3 = pickc ? kFusedSplit : pick[1];
     }
     if (int r = mbxg_set_timing(c, was_timing ? 1 : 0)) return r;
     return mbxg_compute(c, terms, do_grads);

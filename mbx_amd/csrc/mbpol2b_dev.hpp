@@ -84,10 +84,10 @@ __device__ __forceinline__ double switch2(double r, double& g) {
         g = 0.0;
         return 0.0;
     } else if (r > p2::r2i) {
-        const double t1 = M_PI / (p2::r2f - p2::r2i);
-        const double x = (r - p2::r2i) * t1;
-        g = -sin(x) * t1 / 2.0;
-        return (1.0 + cos(x)) / 2.0;
+        double sn, cs;  // (of pi x: no argument reduction by pi)
+        sincospi((r - p2::r2i) / (p2::r2f - p2::r2i), &sn, &cs);
+        g = -sn * (M_PI / (p2::r2f - p2::r2i)) / 2.0;
+        return (1.0 + cs) / 2.0;
     }
     g = 0.0;
     return 1.0;
@@ -124,11 +124,10 @@ __device__ __forceinline__ void load_dimer(const NmerCtx& N, int m1, int m2, dou
         s[9 + j] = b[j];
     }
     if (N.periodic) {
-        const Box& B = *N.box;
-        double dx, dy, dz;
-        image_shift(B, s[0], s[1], s[2], s[9], s[10], s[11], dx, dy, dz);
+        double v[3];
+        image_vector(*N.box, s[0], s[1], s[2], s[9], s[10], s[11], v);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) image_apply(B, dx, dy, dz, s[9 + 3 * j], s[10 + 3 * j], s[11 + 3 * j]);
+        for (int j = 0; j < 9; ++j) s[9 + j] -= v[j % 3];
     }
     msites(s, 0, 6, 7, oh1a, oh2a);
     msites(s, 3, 8, 9, oh1b, oh2b);

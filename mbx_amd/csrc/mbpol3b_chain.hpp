@@ -1,5 +1,5 @@
-// MB-pol 3B device code shared by the stage kernels (eval_mbpol3b.hip) and the paired polynomial
-// launch that runs the 3B chain rule in its tail (poly_mbpol_pair.hip): the variable table,
+// MB-pol 3B device code shared by the stage kernels (eval_mbpol3b.hip) and the one-launch evaluation
+// (mbpol_fused.hip): the variable table,
 // switches, trimer loading and the chain rule of 64 trimers (one lane each).
 //
 // Restates x2o::x3b_v2x::eval (potential/3b/x3b-v2x.cpp:1403-1806): variables
@@ -39,10 +39,10 @@ __device__ __forceinline__ double switch3(double r, double& g) {
         g = 0.0;
         return 0.0;
     } else if (r > p3::r3i) {
-        const double t1 = M_PI / (p3::r3f - p3::r3i);
-        const double x = (r - p3::r3i) * t1;
-        g = -sin(x) * t1 / 2.0;
-        return (1.0 + cos(x)) / 2.0;
+        double sn, cs;  // (of pi x: no argument reduction by pi)
+        sincospi((r - p3::r3i) / (p3::r3f - p3::r3i), &sn, &cs);
+        g = -sn * (M_PI / (p3::r3f - p3::r3i)) / 2.0;
+        return (1.0 + cs) / 2.0;
     }
     g = 0.0;
     return 1.0;
@@ -60,14 +60,14 @@ __device__ __forceinline__ void load_trimer(const NmerCtx& N, int m1, int m2, in
         w[18 + j] = c[j];
     }
     if (N.periodic) {
-        const Box& B = *N.box;
-        double dx, dy, dz;
-        image_shift(B, w[0], w[1], w[2], w[9], w[10], w[11], dx, dy, dz);
+        double v2[3], v3[3];
+        image_vector(*N.box, w[0], w[1], w[2], w[9], w[10], w[11], v2);
+        image_vector(*N.box, w[0], w[1], w[2], w[18], w[19], w[20], v3);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) image_apply(B, dx, dy, dz, w[9 + 3 * j], w[10 + 3 * j], w[11 + 3 * j]);
-        image_shift(B, w[0], w[1], w[2], w[18], w[19], w[20], dx, dy, dz);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) image_apply(B, dx, dy, dz, w[18 + 3 * j], w[19 + 3 * j], w[20 + 3 * j]);
+        for (int j = 0; j < 9; ++j) {
+            w[9 + j] -= v2[j % 3];
+            w[18 + j] -= v3[j % 3];
+        }
     }
 }
 
@@ -128,24 +128,15 @@ constexpr int kChainGroup3 = 4;
 
 // E = s*P for the trimer of lane t (t < n), and with GRAD the chain rule to its atoms, switch
 // derivatives, virial and gradient scatter through the LDS table T; the 64 lanes' energy and
-// virial sums go to partial record `rec`.  WAVE: T belongs to this wavefront alone (lane-strided
-// init and flush, no block barrier); otherwise every thread of the block calls this and T is the
-// block's.  READX: the variables are read back from xs instead of recomputed.
-template <bool GRAD, bool WAVE, int TB, bool READX = false>
+// virial sums go to partial record `rec`.  Every thread of the block calls this; T is the block's.
+template <bool GRAD, int TB>
 __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restrict__ list, const NmerCtx& N,
-                                       const double* __restrict__ xs, const double* __restrict__ gs, const double* __restrict__ ps,
+                                       const double* __restrict__ gs, const double* __restrict__ ps,
                                        const double* __restrict__ sw, int ld, double* __restrict__ grad,
                                        double* __restrict__ e_out, double* __restrict__ vir_out,
                                        double* __restrict__ partials, GradTable<TB, 9>& T) {
-    if (GRAD) {
-        if (WAVE) {
-            table_init_wave(T);
-            wave_lds_order();
-        } else {
-            table_init(T);
-        }
-    }
-    if (!WAVE) __syncthreads();
+    if (GRAD) table_init(T);
+    __syncthreads();
     double e_sum = 0.0;
     double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     int m1 = -1, m2 = -1, m3 = -1;
@@ -169,22 +160,16 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
             // hoists every load and square root and sinks every accumulation: ~500 registers.
             constexpr int G = kChainGroup3;
             size_t toff = (size_t)t;
-            double cg[G], ng[G], cx[G], nx[G];
+            double cg[G], ng[G];
 #pragma unroll
-            for (int k = 0; k < G; ++k) {
-                cg[k] = gs[(size_t)k * ld + toff];
-                if (READX) cx[k] = xs[(size_t)k * ld + toff];
-            }
+            for (int k = 0; k < G; ++k) cg[k] = gs[(size_t)k * ld + toff];
 #pragma unroll
             for (int g = 0; g < 36 / G; ++g) {
                 group_fence(toff, w);
                 group_fence(toff, gd);
                 if (g < 36 / G - 1) {
 #pragma unroll
-                    for (int k = 0; k < G; ++k) {
-                        ng[k] = gs[(size_t)(G * g + G + k) * ld + toff];
-                        if (READX) nx[k] = xs[(size_t)(G * g + G + k) * ld + toff];
-                    }
+                    for (int k = 0; k < G; ++k) ng[k] = gs[(size_t)(G * g + G + k) * ld + toff];
                 }
 #pragma unroll
                 for (int k = 0; k < G; ++k) {
@@ -195,9 +180,9 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
                     const double d2 = w[3 * a1 + 2] - w[3 * a2 + 2];
                     const double d = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
                     const double gj = cg[k] * s;
-                    // the variable itself: read back (READX) or recomputed as k_vars_mbpol3b computed
-                    // it (the same bits either way; alone, one exp is cheaper than the load)
-                    const double xv = READX ? cx[k] : exp(-kset(st) * (d - dset(st)));
+                    // the variable recomputed as k_vars_mbpol3b computed it (the same bits; one exp is
+                    // cheaper than the load)
+                    const double xv = exp(-kset(st) * (d - dset(st)));
                     const double gg = -kset(st) * gj * xv / d;
                     gd[3 * a1] += gg * d0;
                     gd[3 * a1 + 1] += gg * d1;
@@ -207,10 +192,7 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
                     gd[3 * a2 + 2] -= gg * d2;
                 }
 #pragma unroll
-                for (int k = 0; k < G; ++k) {
-                    cg[k] = ng[k];
-                    if (READX) cx[k] = nx[k];
-                }
+                for (int k = 0; k < G; ++k) cg[k] = ng[k];
             }
             group_fence(toff, gd);
             // switch derivatives (x3b-v2x.cpp:1676-1686)
@@ -247,13 +229,8 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
         table_add_runs<9>(T, act, m1, gd, grad, N.first_atom);
         if (act) table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
         if (act) table_add(T, m3, gd + 18, 9, grad, 3 * (size_t)N.first_atom[m3]);
-        if (WAVE) {
-            wave_lds_order();
-            table_flush_wave(T, grad);
-        } else {
-            __syncthreads();
-            table_flush(T, grad);
-        }
+        __syncthreads();
+        table_flush(T, grad);
     }
     // one partial record per wavefront
     e_sum = wave_sum(e_sum);

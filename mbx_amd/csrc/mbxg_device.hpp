@@ -79,6 +79,16 @@ __device__ __forceinline__ void image_apply(const Box& B, double dx, double dy, 
     to_cart(B, u, v, w, x, y, z);
 }
 
+// The same shift as a Cartesian vector, to be taken off every atom of the member: three operations an atom
+// instead of the 33 of the way to fractional coordinates and back, and no rounding on that way (the
+// list builder keeps image_apply, whose bits decide on which side of a cutoff an n-mer falls).
+__device__ __forceinline__ void image_vector(const Box& B, double x1, double y1, double z1, double x2, double y2,
+                                             double z2, double* s) {
+    double dx, dy, dz;
+    image_shift(B, x1, y1, z1, x2, y2, z2, dx, dy, dz);
+    to_cart(B, dx, dy, dz, s[0], s[1], s[2]);
+}
+
 // d0*d0 + d1*d1 + d2*d2 in the reference's order (kdtree_utils.h:63-69).
 __device__ __forceinline__ double dist2(double ax, double ay, double az, double bx, double by, double bz) {
     const double d0 = ax - bx;

@@ -250,12 +250,17 @@ hipError_t launch_poly_mbpol_pair(double* ws3, const int* n3_dev, int cap3, cons
 // launch_mbpol3b_vars and launch_mbpol2b_vars as one launch (workspaces as theirs).
 hipError_t launch_mbpol_vars_pair(const int* list3, const int* n3_dev, int cap3, double* ws3, const int* list2,
                                   const int* n2_dev, int cap2, double* ws2, const NmerCtx& N, hipStream_t st);
-// The same launch with the 3B chain rule (launch_mbpol3b_chain with gradients) in its tail:
-// energies e3_out, gradient added to grad, virials vir3_out (nullable), partial records partials3.
-hipError_t launch_poly_mbpol_pair_chain3(double* ws3, const int* list3, const int* n3_dev, int cap3,
-                                         const double* coef3, double* ws2, const int* n2_dev, int cap2,
-                                         const double* coef2, int split, const NmerCtx& N, double* grad,
-                                         double* e3_out, double* vir3_out, double* partials3, hipStream_t st);
+// Both orders' whole evaluation with gradients in one launch (mbpol_fused.hip): energies e_out, gradient added to grad, virials vir_out (nullable, leading dimension ld),
+// one partial record per 64 n-mers.  cap 0: that order is left out (n_dev is not read).
+constexpr int kFusedSplit = 4;  // wavefronts per 64 n-mers
+struct FusedJob {
+    const int* list;
+    const int* n_dev;
+    int cap, ld;
+    uint64_t coef_addr;
+    double *grad, *e_out, *vir_out, *partials;
+};
+hipError_t launch_mbpol_fused(const FusedJob& trimers, const FusedJob& dimers, const NmerCtx& N, hipStream_t st);
 // MB-nrg families (eval_nrg.hip): the same three stages for FAM_CH4H2O_2B, FAM_CH4CH4_2B and
 // FAM_CH4H2O2_3B; list entries in emission order (the kernels order each n-mer's monomers
 // for its holder).  `split` (1, 2, 4 or 8) is the wavefronts per 64 n-mers of the CH4-H2O-H2O

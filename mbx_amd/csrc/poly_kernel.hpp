@@ -3,9 +3,8 @@
 // It runs as its own kernel so the register allocator sees nothing but the generated
 // straight-line polynomial (x and g arrays plus a few trie temporaries); the variable and
 // chain-rule stages, whose exp/sqrt code the instruction selector freely interleaves, would
-// otherwise push the polynomial past the register file.  The one exception,
-// k_poly_eg_pair_chain3 (poly_mbpol_pair.hip), runs the 3B chain rule strictly after a block's
-// polynomial, behind a fence, so the two phases' registers are allocated one after the other.
+// otherwise push the polynomial past the register file.  (k_mbpol_fused, mbpol_fused.hip, runs them in one
+// kernel with barriers between.)
 //
 // The polynomial is evaluated in symmetry-adapted coordinates (mbx_amd/gen/symmetry.py): sums and
 // differences of the variables that exchanges of like sites permute.  In them a fraction of the
@@ -28,8 +27,8 @@
 
 namespace mbxg {
 
-typedef double (*poly_eg_part_fn)(int, int, mbxg_cptr, const double*, double*);
-typedef double (*poly_e_part_fn)(int, int, mbxg_cptr, const double*);
+typedef void (*poly_eg_part_fn)(int, int, mbxg_cptr, const double*, double*, double*);
+typedef void (*poly_e_part_fn)(int, int, mbxg_cptr, const double*, double*);
 typedef void (*poly_sym_fn)(double*);
 
 // The generated polynomial comes in Q pieces (linear: value and gradient are sums over the
@@ -38,9 +37,16 @@ typedef void (*poly_sym_fn)(double*);
 // summed through LDS in a fixed order by wavefront 0, kRedChunk gradient components at a time.
 // Splitting one n-mer's work over P wavefronts multiplies the number of wavefronts by P at 1/P
 // of the length each, so the last round of wavefronts on the machine is short (less idle
-// tail).  Dynamic LDS: poly_lds_bytes(P).
+// tail).  Dynamic LDS: poly_lds_bytes(P).  The pieces' values meet in LDS and are
+// added in one order for every P (poly_value), so energies do not depend on the split.
 constexpr int kRedChunk = 12;
-constexpr size_t poly_lds_bytes(int P) { return (size_t)(P - 1) * (kRedChunk + 1) * 64 * sizeof(double); }
+constexpr int kPolyParts = 8;
+constexpr size_t poly_lds_bytes(int P) { return ((size_t)(P - 1) * kRedChunk + kPolyParts) * 64 * sizeof(double); }
+
+// The value from the pieces' shares e[64 * piece].
+__device__ __forceinline__ double poly_value(const double* e) {
+    return ((e[0] + e[4 * 64]) + (e[2 * 64] + e[6 * 64])) + ((e[64] + e[5 * 64]) + (e[3 * 64] + e[7 * 64]));
+}
 
 // One block's work: 64 n-mers of group `grp`, P = blockDim.x / 64 wavefronts.
 template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM>
@@ -60,23 +66,22 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
         g[j] = 0.0;
     }
     SYM(x);
-    double E = PART(wv, P, C, x, g);
+    double* es = red + (size_t)(P - 1) * kRedChunk * 64 + lane;
+    PART(wv, P, C, x, g, es);
     if (P > 1) {
 #pragma unroll
         for (int c0 = 0; c0 < NV; c0 += kRedChunk) {
             if (wv > 0) {
-                double* r = red + (size_t)(wv - 1) * (kRedChunk + 1) * 64 + lane;
+                double* r = red + (size_t)(wv - 1) * kRedChunk * 64 + lane;
 #pragma unroll
                 for (int j = c0; j < c0 + kRedChunk && j < NV; ++j) r[(j - c0) * 64] = g[j];
-                if (c0 == 0) r[kRedChunk * 64] = E;
             }
             __syncthreads();
             if (wv == 0) {
                 for (int v = 1; v < P; ++v) {
-                    const double* r = red + (size_t)(v - 1) * (kRedChunk + 1) * 64 + lane;
+                    const double* r = red + (size_t)(v - 1) * kRedChunk * 64 + lane;
 #pragma unroll
                     for (int j = c0; j < c0 + kRedChunk && j < NV; ++j) g[j] += r[(j - c0) * 64];
-                    if (c0 == 0) E += r[kRedChunk * 64];
                 }
             }
             __syncthreads();
@@ -86,7 +91,7 @@ __device__ __forceinline__ void poly_eg_group(int grp, const double* __restrict_
         SYM(g);
 #pragma unroll
         for (int j = 0; j < NV; ++j) gs[(size_t)j * ld + t] = g[j];
-        ps[t] = E;
+        ps[t] = poly_value(es);
     }
 }
 
@@ -99,7 +104,7 @@ template <int NV, int Q, poly_eg_part_fn PART, poly_sym_fn SYM, int WPE>
 __global__ void __launch_bounds__(64 * poly_max_split(WPE)) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
     k_poly_eg(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap, int ld, uint64_t coef_addr,
               double* __restrict__ gs, double* __restrict__ ps) {
-    extern __shared__ double red[];  // [P-1][kRedChunk+1][64]
+    extern __shared__ double red[];  // poly_lds_bytes(P)
     poly_eg_group<NV, Q, PART, SYM>(blockIdx.x, xs, min(*n_dev, cap), ld, coef_addr, gs, ps, red);
 }
 
@@ -164,7 +169,7 @@ hipError_t launch_poly_eg_lists(const PolyLists& J, int P, hipStream_t st) {
 template <int NV, int Q, poly_e_part_fn PART, poly_sym_fn SYM>
 __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, const int* __restrict__ n_dev, int cap,
                                                 int ld, uint64_t coef_addr, double* __restrict__ ps) {
-    extern __shared__ double red[];  // [P-1][64]
+    extern __shared__ double red[];  // [kPolyParts][64]
     const int P = blockDim.x >> 6;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t = blockIdx.x * 64 + lane;
@@ -176,13 +181,9 @@ __global__ void __launch_bounds__(512) k_poly_e(const double* __restrict__ xs, c
 #pragma unroll
     for (int j = 0; j < NV; ++j) x[j] = active ? xs[(size_t)j * ld + t] : 0.0;
     SYM(x);
-    double E = PART(wv, P, C, x);
-    if (wv > 0) red[(wv - 1) * 64 + lane] = E;
+    PART(wv, P, C, x, red + lane);
     if (P > 1) __syncthreads();
-    if (wv == 0 && active) {
-        for (int v = 1; v < P; ++v) E += red[(v - 1) * 64 + lane];
-        ps[t] = E;
-    }
+    if (wv == 0 && active) ps[t] = poly_value(red + lane);
 }
 
 // Launch helpers: P wavefronts per 64 n-mers (P in {1, 2, 4, 8}, dividing Q; the widest polynomials
@@ -205,7 +206,7 @@ hipError_t launch_poly(const double* xs, const int* n_dev, int cap, int ld, cons
     if (do_grads) return launch_poly_eg<NV, Q, PEG, SYM, WPE>(xs, n_dev, cap, ld, coef, gs, ps, P, st);
     if (P != 1 && P != 2 && P != 4 && P != 8) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_poly_e<NV, Q, PE, SYM>), dim3((cap + 63) / 64), dim3(64 * P),
-                       (size_t)(P - 1) * 64 * sizeof(double), st, xs, n_dev, cap, ld, (uint64_t)(uintptr_t)coef, ps);
+                       kPolyParts * 64 * sizeof(double), st, xs, n_dev, cap, ld, (uint64_t)(uintptr_t)coef, ps);
     return hipGetLastError();
 }
 

@@ -376,11 +376,10 @@ __device__ __forceinline__ void xsites(const NmerCtx& N, const int* ent, double*
 #pragma unroll
         for (int j = 0; j < 3 * H::kNat[s]; ++j) dst[j] = a[j];
         if (N.periodic && s != anchor) {
-            const Box& B = *N.box;
-            double dx, dy, dz;
-            image_shift(B, x0, y0, z0, dst[0], dst[1], dst[2], dx, dy, dz);
+            double v[3];
+            image_vector(*N.box, x0, y0, z0, dst[0], dst[1], dst[2], v);
 #pragma unroll
-            for (int at = 0; at < H::kNat[s]; ++at) image_apply(B, dx, dy, dz, dst[3 * at], dst[3 * at + 1], dst[3 * at + 2]);
+            for (int j = 0; j < 3 * H::kNat[s]; ++j) dst[j] -= v[j % 3];
         }
     }
 #pragma unroll
@@ -441,10 +440,10 @@ __device__ __forceinline__ double xswitch(double r, double& g) {
         g = 0.0;
         return 0.0;
     } else if (r > H::kRIn) {
-        const double t1 = M_PI / (H::kROut - H::kRIn);
-        const double xx = (r - H::kRIn) * t1;
-        g = -sin(xx) * t1 / 2.0;
-        return (1.0 + cos(xx)) / 2.0;
+        double sn, cs;  // (of pi x: no argument reduction by pi)
+        sincospi((r - H::kRIn) / (H::kROut - H::kRIn), &sn, &cs);
+        g = -sn * (M_PI / (H::kROut - H::kRIn)) / 2.0;
+        return (1.0 + cs) / 2.0;
     }
     g = 0.0;
     return 1.0;

@@ -402,7 +402,7 @@ def blocked_source(name, fn, energy_only=True):
     hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
            "// Schedule: %s" % ", ".join("%s=%d" % kv for kv in c.items()),
            "// %d parts (op-count balance: %s); <fn>_parts(w, P, ...) evaluates parts w, w+P, ... "
-           "into g and returns their share of the value." % (NPARTS, ", ".join(str(v) for v in s.part_load)),
+           "into g and e[64 * part]." % (NPARTS, ", ".join(str(v) for v in s.part_load)),
            "// Symmetry-adapted coordinates: %s_sym transforms x before and g after; C holds %d slots "
            "(gen/sym_%s.inc)." % (fn, len(sym.rows) + len(sym.low), name),
            "#pragma once",
@@ -413,15 +413,16 @@ def blocked_source(name, fn, energy_only=True):
             continue
         for k in range(NPARTS):
             body.append(s.emit("%s%s_p%d" % (fn, suffix, k), grad=grad, part=k, assign=assign))
-        args, call = (("mbxg_cptr C, const double* x, double* g", "C, x, g, E") if grad
-                      else ("mbxg_cptr C, const double* x", "C, x, E"))
+        args, call = (("mbxg_cptr C, const double* x, double* g", "C, x, g, 0.0") if grad
+                      else ("mbxg_cptr C, const double* x", "C, x, 0.0"))
         # wavefront w of P evaluates pieces w, w + P, ...: a straight sequence of uniform
-        # branches (a switch over the pieces inside a loop costs the register allocator dearly)
-        d = ["__device__ __forceinline__ double %s%s_parts(int w, int P, %s) {" % (fn, suffix, args),
-             "    double E = 0.0;"]
+        # branches (a switch over the pieces inside a loop costs the register allocator dearly).
+        # Each piece's share of the value goes to its own place, so that the sum over the pieces
+        # (poly_value) is the same for every P.
+        d = ["__device__ __forceinline__ void %s%s_parts(int w, int P, %s, double* e) {" % (fn, suffix, args)]
         for k in range(NPARTS):
-            d.append("    if (%d %% P == w) E = %s%s_p%d(%s);" % (k, fn, suffix, k, call))
-        d += ["    return E;", "}", ""]
+            d.append("    if ((%d & (P - 1)) == w) e[%d] = %s%s_p%d(%s);" % (k, 64 * k, fn, suffix, k, call))
+        d += ["}", ""]
         body.append("\n".join(d))
     return "\n".join(hdr) + "\n".join(body), c
 
