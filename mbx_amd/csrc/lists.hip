@@ -458,6 +458,29 @@ __device__ __forceinline__ Lds carve(double* d, int cap) {
 
 }  // namespace
 
+namespace {
+
+// A monomer's share of an n-mer's composition: sums of three tell how many are of each kind.
+constexpr int kSpeciesH2O = 1, kSpeciesCH4 = 4;
+__device__ __forceinline__ int species(int kind) {
+    return kind == MON_H2O ? kSpeciesH2O : kind == MON_CH4 ? kSpeciesCH4 : 16;
+}
+
+// sqrt(rr) > f, exactly: the root is only taken where the squares are too close to tell.
+__device__ __forceinline__ bool sqrt_above(double rr, double f) {
+    const double f2 = f * f;
+    if (fabs(rr - f2) > 1e-14 * f2) return rr > f2;
+    return sqrt(rr) > f;
+}
+
+}  // namespace
+
+// Bound by instructions and by the waits between its short stages, in two rounds of blocks at 2048 waters
+// (cutoffs 9 and 7 A: some 100 matches and 1000 pairs a query).  Comparing squares instead of taking two
+// double precision roots a pair, kinds and tags packed beforehand, the query's own slot left out and
+// the candidates' rows without a walk took it from 2350 to 1760 vector instructions a wavefront: 53 -> 48 us;
+// 6859 waters 133 -> 115; 32 beads of 570 monomers 245 -> 216; 256 clusters of 16 to 512 waters 209 -> 201.
+//
 // One query, by the block's kQueryWaves wavefronts: gather, sort, per-match data, dimers,
 // trimers.  L is the block's match storage (LDS, or a global scratch slice when the matches do
 // not fit in LDS); sh_count and sh_w are block-shared.  The dimers and trimers of a query are
@@ -497,38 +520,24 @@ __device__ void nmers_query(int q, const PtInfo* __restrict__ pinfo, const doubl
     const double qx = cx[q], qy = cy[q], qz = cz[q];
     const int ci = cell[q] - base;
     const int ia = ci % G.n[0], ib = (ci / G.n[0]) % G.n[1], ic = ci / (G.n[0] * G.n[1]);
-    int rbeg[9], rlen[9];
-    int nrow = 0;
-    for (int cc = max(ic - 1, 0); cc <= min(ic + 1, G.n[2] - 1); ++cc) {
-        for (int cb = max(ib - 1, 0); cb <= min(ib + 1, G.n[1] - 1); ++cb) {
-            const int row = base + (cc * G.n[1] + cb) * G.n[0];
-            rbeg[nrow] = row + max(ia - 1, 0);
-            rlen[nrow] = row + min(ia + 1, G.n[0] - 1) + 1;
-            ++nrow;
-        }
-    }
+    // row r holds the candidates from first[r] on, candidate c at the slot-array position c + shift[r]
+    int first[9], shift[9];
     int ncand = 0;
-    for (int r = 0; r < 9; ++r) {
-        if (r < nrow) {
-            const int b0 = cell_start[rbeg[r]], e0 = cell_start[rlen[r]];
-            rbeg[r] = b0;
-            rlen[r] = e0 - b0;
-            ncand += e0 - b0;
-        }
-    }
-    // candidate c -> slot-array position (row by row, in order)
-    auto position = [&](int c) {
-        int at = -1;
 #pragma unroll
-        for (int r = 0; r < 9; ++r) {
-            if (r < nrow && at < 0) {
-                if (c < rlen[r])
-                    at = rbeg[r] + c;
-                else
-                    c -= rlen[r];
-            }
-        }
-        return at;
+    for (int r = 0; r < 9; ++r) {
+        const int cc = ic + r / 3 - 1, cb = ib + r % 3 - 1;
+        const bool in = cc >= 0 && cc < G.n[2] && cb >= 0 && cb < G.n[1];
+        const int* at = cell_start + base + (in ? (cc * G.n[1] + cb) * G.n[0] : 0);
+        const int b0 = at[max(ia - 1, 0)], e0 = at[min(ia + 1, G.n[0] - 1) + 1];
+        first[r] = ncand;
+        shift[r] = b0 - ncand;
+        ncand += in ? e0 - b0 : 0;
+    }
+    auto position = [&](int c) {
+        int by = shift[0];
+#pragma unroll
+        for (int r = 1; r < 9; ++r) by = c >= first[r] ? shift[r] : by;
+        return c + by;
     };
     if (tid == 0) *sh_count = 0;
     __syncthreads();
@@ -648,7 +657,8 @@ __device__ void nmers_query(int q, const PtInfo* __restrict__ pinfo, const doubl
         int n3w = 0;
         for (int b = 0; b < nm; b += 64) {
             const int a = b + lane;
-            const bool in3 = a < nm && (L.flags[a] & 2);
+            // (the query itself and its images are in no trimer of it)
+            const bool in3 = a < nm && (L.flags[a] & 2) && L.mon[a] != mi;
             const unsigned long long m = __ballot(in3);
             if (in3) L.m3[n3w + __popcll(m & ((1ull << lane) - 1ull))] = a;
             n3w += __popcll(m);
@@ -665,7 +675,7 @@ __device__ void nmers_query(int q, const PtInfo* __restrict__ pinfo, const doubl
         *(double2*)(e + 2) = make_double2(L.sz[a], L.ix[a]);
         *(double2*)(e + 4) = make_double2(L.iy[a], L.iz[a]);
         *(double2*)(e + 6) = make_double2(L.r[a], 0.0);
-        *(int4*)(e + 8) = make_int4(L.mon[a], L.tag[a], L.kind[a], 0);
+        *(int4*)(e + 8) = make_int4(L.mon[a], ti < L.tag[a], species(L.kind[a]), 0);
     }
     __syncthreads();
 
@@ -752,8 +762,10 @@ __device__ void nmers_query(int q, const PtInfo* __restrict__ pinfo, const doubl
     // other mixtures have no 3B term (energy3b.cpp:258-260).
     if (c3sq > 0.0) {
         // pairs u < v of the 3B matches in (u, v) order: pair t lies in row u, which starts at
-        // S(u) = u (2 n3 - u - 1) / 2 (a floating-point first guess, corrected exactly)
+        // S(u) = u (2 n3 - u - 1) / 2 (a single-precision first guess, corrected exactly)
         const int total = n3 * (n3 - 1) / 2;
+        const int w0 = 2 * n3 - 1, si = species(ki);
+        auto row = [&](int u) { return __mul24(u, w0 - u) / 2; };
         int b0, b1;
         range(total, b0, b1);
         for (int b = b0; b < b1; b += 64) {
@@ -761,42 +773,35 @@ __device__ void nmers_query(int q, const PtInfo* __restrict__ pinfo, const doubl
             bool listed = false;
             int mj = 0, mk = 0, fam = -1;
             if (t < b1) {
-                const double w = 2.0 * n3 - 1.0;
-                int u = (int)((w - sqrt(w * w - 8.0 * t)) * 0.5);
-                u = u < 0 ? 0 : (u > n3 - 2 ? n3 - 2 : u);
-                while (u > 0 && u * (2 * n3 - u - 1) / 2 > t) --u;
-                while (u < n3 - 2 && (u + 1) * (2 * n3 - u - 2) / 2 <= t) ++u;
-                const int v = t - u * (2 * n3 - u - 1) / 2 + u + 1;
-                {
-                    const double* ej = L.p3 + (size_t)kP3Doubles * u;
-                    const double* ek = L.p3 + (size_t)kP3Doubles * v;
-                    const int4 ij = *(const int4*)(ej + 8), ik = *(const int4*)(ek + 8);
-                    mj = ij.x;
-                    mk = ik.x;
-                    if (mj != mi && mk != mi && mj != mk) {
-                        const double2 j01 = *(const double2*)ej, k01 = *(const double2*)ek;
-                        const double2 j23 = *(const double2*)(ej + 2), k23 = *(const double2*)(ek + 2);
-                        const double djk = dist2(j01.x, j01.y, j23.x, k01.x, k01.y, k23.x);
-                        listed = djk > c3sq || (ti < ij.y && ti < ik.y);
-                        const int nch4 = (ki == MON_CH4) + (ij.z == MON_CH4) + (ik.z == MON_CH4);
-                        const int nh2o = (ki == MON_H2O) + (ij.z == MON_H2O) + (ik.z == MON_H2O);
-                        if (listed && (nh2o == 3 || (nh2o == 2 && nch4 == 1))) {
-                            const double2 j45 = *(const double2*)(ej + 4), k45 = *(const double2*)(ek + 4);
-                            const double e0 = j23.y - k23.y, e1 = j45.x - k45.x, e2 = j45.y - k45.y;
-                            double rr = 0.0;
-                            rr += e0 * e0;
-                            rr += e1 * e1;
-                            rr += e2 * e2;
-                            const double rab = ej[6], rac = ek[6], rbc = sqrt(rr);
-                            if (nh2o == 3) {
-                                const double f = p3::r3f;
-                                if (!((rab > f && rac > f) || (rab > f && rbc > f) || (rac > f && rbc > f)))
-                                    fam = FAM_MBPOL_3B;
-                            } else {
-                                const double f = Holder_ch4h2o2_3b::kROut;
-                                if (!(rab > f && rac > f && rbc > f)) fam = FAM_CH4H2O2_3B;
-                            }
-                        }
+                int u = (int)((w0 - __builtin_amdgcn_sqrtf((float)((double)w0 * w0 - 8.0 * t))) * 0.5f);
+                u = min(max(u, 0), n3 - 2);
+                while (u > 0 && row(u) > t) --u;
+                while (u < n3 - 2 && row(u + 1) <= t) ++u;
+                const int v = t - row(u) + u + 1;
+                const double* ej = L.p3 + (size_t)kP3Doubles * u;
+                const double* ek = L.p3 + (size_t)kP3Doubles * v;
+                const int4 ij = *(const int4*)(ej + 8), ik = *(const int4*)(ek + 8);
+                mj = ij.x;
+                mk = ik.x;
+                const double2 j01 = *(const double2*)ej, k01 = *(const double2*)ek;
+                const double2 j23 = *(const double2*)(ej + 2), k23 = *(const double2*)(ek + 2);
+                const double djk = dist2(j01.x, j01.y, j23.x, k01.x, k01.y, k23.x);
+                listed = mj != mk && (djk > c3sq || (ij.y && ik.y));
+                const int kinds = si + ij.z + ik.z;
+                if (listed && (kinds == 3 * kSpeciesH2O || kinds == 2 * kSpeciesH2O + kSpeciesCH4)) {
+                    const double2 j45 = *(const double2*)(ej + 4), k45 = *(const double2*)(ek + 4);
+                    const double e0 = j23.y - k23.y, e1 = j45.x - k45.x, e2 = j45.y - k45.y;
+                    double rr = 0.0;
+                    rr += e0 * e0;
+                    rr += e1 * e1;
+                    rr += e2 * e2;
+                    const double rab = ej[6], rac = ek[6];
+                    if (kinds == 3 * kSpeciesH2O) {
+                        const bool ab = rab > p3::r3f, ac = rac > p3::r3f, bc = sqrt_above(rr, p3::r3f);
+                        if (!((ab && ac) || (ab && bc) || (ac && bc))) fam = FAM_MBPOL_3B;
+                    } else {
+                        const double f = Holder_ch4h2o2_3b::kROut;
+                        if (!(rab > f && rac > f && sqrt_above(rr, f))) fam = FAM_CH4H2O2_3B;
                     }
                 }
             }
