@@ -142,29 +142,28 @@ __device__ __forceinline__ void holder_switches(const double* x, double d[3][3],
     }
 }
 
-// Variable J's value from its site pair (tools/variable.cpp:49-129); gg with
-// d(value)/d(site s1) = gg * (x[s1] - x[s2]).  Everything about the variable is a constant.
+// Variable J's value from its site pair (tools/variable.cpp:49-129).  Everything about the variable is a
+// constant.
 template <class H, int J>
-__device__ __forceinline__ double nrg_value(const double* x, double* dvec, double& gg) {
+__device__ __forceinline__ double nrg_value(const double* x) {
+    constexpr NrgVar V = H::kVars[J];
+    const double d0 = x[3 * V.s1] - x[3 * V.s2], d1 = x[3 * V.s1 + 1] - x[3 * V.s2 + 1],
+                 d2 = x[3 * V.s1 + 2] - x[3 * V.s2 + 2];
+    const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+    if (V.form == 0) return exp(V.k * (V.d - r));
+    if (V.form == 1) return exp(V.k * (V.d - r)) / r;
+    return exp(V.k * (-r));
+}
+
+// gg with d(value)/d(site s1) = gg * (x[s1] - x[s2]), from the value.
+template <class H, int J>
+__device__ __forceinline__ double nrg_slope(const double* x, double val, double* dvec) {
     constexpr NrgVar V = H::kVars[J];
     dvec[0] = x[3 * V.s1] - x[3 * V.s2];
     dvec[1] = x[3 * V.s1 + 1] - x[3 * V.s2 + 1];
     dvec[2] = x[3 * V.s1 + 2] - x[3 * V.s2 + 2];
-    const double r = sqrt(dvec[0] * dvec[0] + dvec[1] * dvec[1] + dvec[2] * dvec[2]);
-    double val;
-    if (V.form == 0) {
-        val = exp(V.k * (V.d - r));
-        gg = -V.k * val / r;
-    } else if (V.form == 1) {
-        const double e1 = exp(V.k * (V.d - r));
-        const double rinv = 1.0 / r;
-        val = e1 * rinv;
-        gg = -(V.k + rinv) * val * rinv;
-    } else {
-        val = exp(V.k * (-r));
-        gg = -V.k * val / r;
-    }
-    return val;
+    const double rinv = rsqrt(dvec[0] * dvec[0] + dvec[1] * dvec[1] + dvec[2] * dvec[2]);
+    return -(V.form == 1 ? V.k + rinv : V.k) * val * rinv;
 }
 
 }  // namespace
@@ -180,8 +179,7 @@ __global__ void __launch_bounds__(64) k_vars_nrg(const int* __restrict__ list, c
     holder_sites<H>(N, list + H::kMon * (size_t)t, x, mon, oh1, oh2);
     static_for<H::kNVars>([&](auto J) {
         constexpr int j = decltype(J)::value;
-        double dv[3], gg;
-        xs[(size_t)j * ld + t] = nrg_value<H, j>(x, dv, gg);
+        xs[(size_t)j * ld + t] = nrg_value<H, j>(x);
     });
     double d[3][3], r[3], s[3], gs[3];
     holder_switches<H>(x, d, r, s, gs);
@@ -191,7 +189,11 @@ __global__ void __launch_bounds__(64) k_vars_nrg(const int* __restrict__ list, c
 constexpr int kGradBlockNrg = 128;
 
 // Stage 3: energy; with GRAD the chain rule, virial and gradient scatter.  gs / ps hold the
-// polynomial's gradient ([var][ld]) and value.
+// polynomial's gradient ([var][ld]) and value.  CH4-H2O-H2O is bound by reading its 55 variables and 55
+// gradients (0.9 KB a trimer, a million trimers for 32 beads of 570 monomers: 190 us at the rate of a copy):
+// 279 us with the variables read back and one rsqrt each, 310 with root, exponential and division taken
+// again.  Variables, polynomial and chain rule in one launch, as for MB-pol, was no faster (940 us
+// against 128 + 560 + 279): 256 registers leave two wavefronts a SIMD, too few to hide its thirty barriers.
 template <class H, bool GRAD>
 __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restrict__ list, const int* __restrict__ n_dev,
                                                             int cap, NmerCtx N, const double* __restrict__ xs,
@@ -229,8 +231,8 @@ __global__ void __launch_bounds__(kGradBlockNrg) k_grad_nrg(const int* __restric
                 constexpr int j = decltype(J)::value;
                 double gj = gs[(size_t)j * ld + t];
                 if (H::kMon == 3) gj *= sw;  // the 3B holder scales the polynomial gradient first
-                double dv[3], gg;
-                nrg_value<H, j>(x, dv, gg);
+                double dv[3];
+                const double gg = nrg_slope<H, j>(x, xs[(size_t)j * ld + t], dv);
                 constexpr int a1 = H::kVars[j].s1, a2 = H::kVars[j].s2;
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
