@@ -9,15 +9,16 @@ into the engine's working buffer is part of each step); results stay on the devi
 Throughput is listed dimers + trimers per second (the n-mers the reference's Get2B / Get3B walk).
 
 The JSON line also carries
-  roofline:     the polynomial launch (the dominant kernel: the MB-pol 3B and 2B polynomials in
-                one launch with the 3B chain rule in its 3B blocks, k_poly_eg_pair_chain3; without
-                the chain rule when fuse_chain is off; the 3B one alone when the pairing is off)
-                against MI355X FP64 vector peak, with the reference's algorithmic FLOPs per
-                evaluated trimer (81,549, plus 1,094 for the chain rule) and dimer (27,208),
-                counted from the reference's code (mbx_amd/tables/flops.json), timed with HIP events
+  roofline:     the dominant launch (k_mbpol_fused: variables, polynomials and chain rules of MB-pol 3B
+                and 2B; the paired polynomials when fuse_chain is off; the 3B one alone when the
+                pairing is off) against the MI355X FP64 vector unit's operations (an FMA is one:
+                39.3 T/s).  Counted are the FP64 operations that the polynomials execute per
+                evaluated trimer (17,106) and dimer (6,541), from their generated sources: in
+                symmetry-adapted coordinates a quarter of the reference's multiplies and adds
+                (81,549 and 27,208), which would give more than the peak.  Timed with HIP events
                 on the engine stream in a stage-timing pass of the same workload; traffic from the
                 committed rocprofv3 PMC summary when present.  config.polynomial_alone times the
-                launch without the chain rule beside it;
+                polynomials without the stages around them beside it;
   cpu_baseline: the reference's own compiled 2B/3B leaves (oracle/_ref, OpenMP driver) on this
                 host's cores, on the same workload, in two dispatch modes: the reference's own
                 batch of 8 n-mers per polynomial call and a best-effort batch of 1024; the faster
@@ -30,6 +31,7 @@ C++ System, 1B + 2B + 3B, host arrays in and out).
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -37,7 +39,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 METRIC = "2B+3B dimers+trimers/sec (E+F, FP64) at 2048 H2O; batched vs plain speedup"
-FP64_VECTOR_PEAK = 78.6e12  # MI355X FP64 vector, FLOP/s
+FP64_VECTOR_PEAK = 78.6e12 / 2  # MI355X FP64 vector, operations/s (an FMA is one)
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_poly3b_water2048.txt")
 LIST_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic_lists_water2048.txt")
 HBM_PEAK = 8.0e12  # MI355X HBM3E, B/s
@@ -75,6 +77,12 @@ def host_cpu():
     except OSError:
         pass
     return model, len(cores) or logical, logical
+
+
+def executed_ops(name):
+    """FP64 operations (an FMA is one) of a polynomial's value and gradient, from its generated source."""
+    with open(os.path.join(ROOT, "mbx_amd", "csrc", "gen", "poly_%s.inc" % name)) as f:
+        return int(re.search(r"fp64_ops_eg=(\d+)", f.read(2000)).group(1))
 
 
 def read_traffic(path=TRAFFIC_FILE, key="traffic_bytes_per_launch:"):
@@ -406,8 +414,8 @@ def main():
         poly_ms.append(tm["poly_3b"])
         for k, v in tm.items():
             stage[k] = stage.get(k, 0.0) + v
-    # the polynomial launch without the 3B chain rule (fuse_chain 0: the chain rule as a kernel of
-    # its own), for the polynomial's own roofline figure
+    # the polynomials without the stages around them (fuse_chain 0: those are launches of their
+    # own), for the polynomials' own roofline figure
     unfused = None
     if eng.tuning("fuse_chain") == 1:
         eng.set_tuning("fuse_chain", 0)
@@ -438,17 +446,14 @@ def main():
     dt = (t1 - t0) / args.steps if not args.solo else stage["total"] / 1e3 / args.steps
     e2, e3, grad, vir = eng.results()
 
-    flops = json.load(open(os.path.join(ROOT, "mbx_amd", "tables", "flops.json")))
-    f3, f2 = flops["mbpol_3b_eg"]["flops"], flops["mbpol_2b_eg"]["flops"]
+    f3, f2 = executed_ops("mbpol_3b"), executed_ops("mbpol_2b")
     paired = eng.tuning("fuse_poly") == 1 and counts[1] > 0 and counts[3] > 0
     chained = paired and eng.tuning("fuse_chain") == 1
-    if chained:  # the launch also runs the 3B chain rule: its algorithmic work counts too
-        f3 += flops["mbpol_3b_chain"]["flops"]
     t_poly = float(np.mean(poly_ms)) * 1e-3
     achieved = (counts[3] * f3 + (counts[1] * f2 if paired else 0)) / t_poly
     traffic = read_traffic()
-    kernel = ("k_poly_eg_pair_chain3<36, 31> (MB-pol 3B and 2B polynomials E+G and the 3B chain rule, one launch)"
-              if chained else "k_poly_eg_pair<36, 31> (MB-pol 3B and 2B polynomials E+G, one launch)" if paired
+    kernel = ("k_mbpol_fused (MB-pol 3B and 2B variables, polynomials E+G and chain rules, one launch)" if chained
+              else "k_poly_eg_pair<36, 31> (MB-pol 3B and 2B polynomials E+G, one launch)" if paired
               else "k_poly_eg<36> (MB-pol 3B polynomial E+G)")
 
     out = {
@@ -470,20 +475,19 @@ def main():
                    "stage_ms": {k: v / args.steps for k, v in stage.items()}, "e2b": e2, "e3b": e3,
                    "schedule": schedule},
         "roofline": {"bound": "fp64-valu", "kernel": kernel,
-                     "achieved": achieved / 1e12, "peak": FP64_VECTOR_PEAK / 1e12, "unit": "TFLOP/s",
+                     "achieved": achieved / 1e12, "peak": FP64_VECTOR_PEAK / 1e12, "unit": "T FP64 operations/s (FMA = 1)",
                      "frac": achieved / FP64_VECTOR_PEAK, "traffic": traffic,
-                     "flops_per_unit": {"trimer": f3, "dimer": f2 if paired else 0},
+                     "operations_per_unit": {"trimer": f3, "dimer": f2 if paired else 0},
                      "units_per_launch": {"trimers": int(counts[3]), "dimers": int(counts[1]) if paired else 0},
                      "launch_ms": t_poly * 1e3},
         "cpu_baseline": None,
     }
     # list build (fix, cloud, binning, both n-mer passes): PMC bytes per step over its HIP-event time
     if chained and unfused:
-        f3p = flops["mbpol_3b_eg"]["flops"]
-        a_u = (counts[3] * f3p + counts[1] * f2) / (unfused[0] * 1e-3)
+        a_u = (counts[3] * f3 + counts[1] * f2) / (unfused[0] * 1e-3)
         out["config"]["polynomial_alone"] = {
-            "kernel": "k_poly_eg_pair<36, 31> (fuse_chain 0; the 3B chain rule then runs as k_grad_mbpol3b)",
-            "launch_ms": unfused[0], "achieved_TFLOPs": a_u / 1e12, "frac": a_u / FP64_VECTOR_PEAK,
+            "kernel": "k_poly_eg_pair<36, 31> (fuse_chain 0; variables and chain rules are then launches of their own)",
+            "launch_ms": unfused[0], "achieved_Tops": a_u / 1e12, "frac": a_u / FP64_VECTOR_PEAK,
             "chain_3b_ms": unfused[1]}
     out["config"]["with_grad_d2h"] = {
         "ms_per_step": t_d2h * 1e3, "nmers_per_s": n_listed / t_d2h,
