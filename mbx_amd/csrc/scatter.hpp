@@ -36,17 +36,11 @@ __device__ __forceinline__ void lds_add(double* p, double v) {
     __builtin_amdgcn_ds_atomic_fadd_f64((__attribute__((address_space(3))) double*)p, v);
 }
 
-// Clear the table with threads first, first + step, ...
-template <int TB, int NA>
-__device__ __forceinline__ void table_init_from(GradTable<TB, NA>& T, int first, int step) {
-    for (int i = first; i < TB; i += step) T.key[i] = -1;
-    for (int i = first; i < TB * NA; i += step) T.val[i] = 0.0;
-    if (first == 0) T.count = 0;
-}
-
 template <int TB, int NA>
 __device__ __forceinline__ void table_init(GradTable<TB, NA>& T) {
-    table_init_from(T, threadIdx.x, blockDim.x);
+    for (int i = threadIdx.x; i < TB; i += blockDim.x) T.key[i] = -1;
+    for (int i = threadIdx.x; i < TB * NA; i += blockDim.x) T.val[i] = 0.0;
+    if (threadIdx.x == 0) T.count = 0;
 }
 
 // The entry of monomer `mon`, whose cnt values start at grad + goff; -1: the table is full.
@@ -150,41 +144,16 @@ __device__ __forceinline__ void table_add_slot(GradTable<TB, NA>& T, bool act, b
         table_add(T, mon, g, CNT, grad, 3 * (size_t)first_atom[mon]);
 }
 
-// The occupied entries into the gradient, by threads first, first + step, ...: one device atomic per
-// value, consecutive threads on consecutive values, so a wavefront's atomics fall on some eight cache
-// lines instead of one line per lane, and nothing is loaded from memory on the way.
+// After a barrier: the occupied entries into the gradient, one device atomic per value, consecutive threads
+// on consecutive values, so a wavefront's atomics fall on some eight cache lines instead of one line per
+// lane, and nothing is loaded from memory on the way.
 template <int TB, int NA>
-__device__ __forceinline__ void table_flush_from(const GradTable<TB, NA>& T, int first, int step, double* grad) {
+__device__ __forceinline__ void table_flush(const GradTable<TB, NA>& T, double* grad) {
     const int n = T.count * NA;
-    for (int i = first; i < n; i += step) {
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int e = i / NA, c = i - e * NA, h = T.used[e], d = T.dest[h];
         if (c < (d & 31)) unsafeAtomicAdd(grad + (d >> 5) + c, T.val[h * NA + c]);
     }
-}
-
-// After a barrier: the whole block's threads.
-template <int TB, int NA>
-__device__ __forceinline__ void table_flush(const GradTable<TB, NA>& T, double* grad) {
-    table_flush_from(T, threadIdx.x, blockDim.x, grad);
-}
-
-// A table that one wavefront owns alone (the other wavefronts of its block never touch it):
-// lane-strided init and flush, no block barrier.  The LDS unit performs one wavefront's
-// operations in issue order, so between the phases only the compiler has to be kept from moving
-// them and the outstanding LDS operations have to be waited for: wave_lds_order.
-__device__ __forceinline__ void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-}
-
-template <int TB, int NA>
-__device__ __forceinline__ void table_init_wave(GradTable<TB, NA>& T) {
-    table_init_from(T, threadIdx.x & 63, 64);
-}
-
-template <int TB, int NA>
-__device__ __forceinline__ void table_flush_wave(const GradTable<TB, NA>& T, double* grad) {
-    table_flush_from(T, threadIdx.x & 63, 64, grad);
 }
 
 }  // namespace mbxg
