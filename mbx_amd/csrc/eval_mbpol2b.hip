@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(kGradBlock2) k_grad_mbpol2b(const int* __restr
     }
     if (GRAD) {
         table_add_runs<9>(T, t < n, m1, gd, grad, N.first_atom);
-        if (t < n) table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
+        if (t < n) table_add(T, m2, gd + 9, 9, grad, N.first_atom[m2]);
         __syncthreads();
         table_flush(T, grad);
     }

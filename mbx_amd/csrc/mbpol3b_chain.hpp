@@ -227,8 +227,8 @@ __device__ __forceinline__ void chain3(int t, int rec, int n, const int* __restr
     if (GRAD) {
         const bool act = t < n;  // inactive lanes hold zeros
         table_add_runs<9>(T, act, m1, gd, grad, N.first_atom);
-        if (act) table_add(T, m2, gd + 9, 9, grad, 3 * (size_t)N.first_atom[m2]);
-        if (act) table_add(T, m3, gd + 18, 9, grad, 3 * (size_t)N.first_atom[m3]);
+        if (act) table_add(T, m2, gd + 9, 9, grad, N.first_atom[m2]);
+        if (act) table_add(T, m3, gd + 18, 9, grad, N.first_atom[m3]);
         __syncthreads();
         table_flush(T, grad);
     }

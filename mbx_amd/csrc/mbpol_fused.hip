@@ -108,7 +108,7 @@ __device__ __forceinline__ void finish_nmers(const FusedJob& J, const NmerCtx& N
     if (wv == 0)
         table_add_runs<9>(T, act, mon, gd, J.grad, N.first_atom);  // the query monomer
     else if (wv < ORDER && act)
-        table_add(T, mon, gd, 9, J.grad, 3 * (size_t)N.first_atom[mon]);
+        table_add(T, mon, gd, 9, J.grad, N.first_atom[mon]);
     if (wv == kWaves - 1) {
         double vir[6];
 #pragma unroll

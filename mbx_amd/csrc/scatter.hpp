@@ -24,9 +24,9 @@ namespace mbxg {
 template <int TB, int NA>
 struct GradTable {
     double val[TB * NA];
-    int key[TB];   // monomer, -1: free
-    int dest[TB];  // its first value in the gradient * 32 + its number of values
-    int used[TB];  // the occupied entries, in the order they were taken
+    int key[TB];    // monomer, -1: free
+    int first[TB];  // its first atom (three values an atom: scaled by three it needs more than 32 bits)
+    int used[TB];   // the occupied entries * 32 + their numbers of values, in the order they were taken
     int count;
 };
 
@@ -43,17 +43,17 @@ __device__ __forceinline__ void table_init(GradTable<TB, NA>& T) {
     if (threadIdx.x == 0) T.count = 0;
 }
 
-// The entry of monomer `mon`, whose cnt values start at grad + goff; -1: the table is full.
+// The entry of monomer `mon`, whose cnt values start at atom `first`; -1: the table is full.
 template <int TB, int NA>
-__device__ __forceinline__ int table_entry(GradTable<TB, NA>& T, int mon, int cnt, size_t goff) {
+__device__ __forceinline__ int table_entry(GradTable<TB, NA>& T, int mon, int cnt, int first) {
     unsigned h = ((unsigned)mon * 2654435761u) % TB;
     for (int probe = 0; probe < TB; ++probe) {
         int k = __atomic_load_n(&T.key[h], __ATOMIC_RELAXED);
         if (k == -1) {
             k = atomicCAS(&T.key[h], -1, mon);
             if (k == -1) {  // taken here
-                T.dest[h] = (int)goff * 32 + cnt;
-                T.used[atomicAdd(&T.count, 1)] = h;
+                T.first[h] = first;
+                T.used[atomicAdd(&T.count, 1)] = (int)h * 32 + cnt;
                 return h;
             }
         }
@@ -63,18 +63,18 @@ __device__ __forceinline__ int table_entry(GradTable<TB, NA>& T, int mon, int cn
     return -1;
 }
 
-// Add cnt (<= NA) values for monomer `mon`; falls back to device atomics at grad + goff if full.
+// Add cnt (<= NA) values for monomer `mon`, whose first atom is `first`; device atomics if the table is full.
 template <int TB, int NA>
 __device__ __forceinline__ void table_add(GradTable<TB, NA>& T, int mon, const double* g, int cnt, double* grad,
-                                          size_t goff) {
-    const int h = table_entry(T, mon, cnt, goff);
+                                          int first) {
+    const int h = table_entry(T, mon, cnt, first);
 #pragma unroll
     for (int c = 0; c < NA; ++c)
         if (c < cnt) {
             if (h >= 0)
                 lds_add(&T.val[h * NA + c], g[c]);
             else
-                unsafeAtomicAdd(grad + goff + c, g[c]);
+                unsafeAtomicAdd(grad + 3 * (size_t)first + c, g[c]);
         }
 }
 
@@ -120,18 +120,18 @@ __device__ __forceinline__ void table_add_runs(GradTable<TB, NA>& T, bool act, i
     for (int run = 0; run < kRuns && left; ++run) {
         if (!next_run(act, mon, left, mq, in)) break;
         const double mine = run_sum<CNT>(in, g);
-        const size_t goff = 3 * (size_t)first_atom[mq];
+        const int first = first_atom[mq];
         int h = 0;
-        if (lane == 0) h = table_entry(T, mq, CNT, goff);
+        if (lane == 0) h = table_entry(T, mq, CNT, first);
         h = __builtin_amdgcn_readlane(h, 0);
         if (lane < CNT) {
             if (h >= 0)
                 lds_add(&T.val[h * NA + lane], mine);
             else
-                unsafeAtomicAdd(grad + goff + lane, mine);
+                unsafeAtomicAdd(grad + 3 * (size_t)first + lane, mine);
         }
     }
-    if (act && ((left >> lane) & 1)) table_add(T, mon, g, CNT, grad, 3 * (size_t)first_atom[mon]);
+    if (act && ((left >> lane) & 1)) table_add(T, mon, g, CNT, grad, first_atom[mon]);
 }
 
 // One slot of an n-mer whose query monomer may be in any slot (`query`: this lane's is in this one).
@@ -141,7 +141,7 @@ __device__ __forceinline__ void table_add_slot(GradTable<TB, NA>& T, bool act, b
     if (__ballot(act && query))
         table_add_runs<CNT>(T, act, mon, g, grad, first_atom);
     else if (act)
-        table_add(T, mon, g, CNT, grad, 3 * (size_t)first_atom[mon]);
+        table_add(T, mon, g, CNT, grad, first_atom[mon]);
 }
 
 // After a barrier: the occupied entries into the gradient, one device atomic per value, consecutive threads
@@ -151,8 +151,8 @@ template <int TB, int NA>
 __device__ __forceinline__ void table_flush(const GradTable<TB, NA>& T, double* grad) {
     const int n = T.count * NA;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int e = i / NA, c = i - e * NA, h = T.used[e], d = T.dest[h];
-        if (c < (d & 31)) unsafeAtomicAdd(grad + (d >> 5) + c, T.val[h * NA + c]);
+        const int e = i / NA, c = i - e * NA, u = T.used[e], h = u >> 5;
+        if (c < (u & 31)) unsafeAtomicAdd(grad + 3 * (size_t)T.first[h] + c, T.val[h * NA + c]);
     }
 }
 
