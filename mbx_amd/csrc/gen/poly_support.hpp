@@ -17,3 +17,11 @@ typedef const __attribute__((address_space(4))) double* mbxg_cptr;
         __builtin_amdgcn_sched_barrier(0);        \
         asm volatile("" : "+s"(C) : "v"(dep));    \
     } while (0)
+
+// The variables redefined opaquely: products of them computed before are computed again after, not kept
+// live in between.
+template <int N>
+__device__ __forceinline__ void mbxg_opaque(const double* x) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(((double*)x)[i]));
+}

@@ -9,7 +9,7 @@
 // fourth component of the gradient over the wavefronts, and runs the chain rule of its variables, for which
 // an exponential needs only y_j = x_j dP/dx_j; then each of the first
 // wavefronts gathers one monomer's gradient and scatters it while the last one has done the switch, energy
-// and virial.  With the polynomial down to 17.1k operations a trimer (poly_kernel.hpp) the stages around it
+// and virial.  With the polynomial down to 20.0k operations a trimer (poly_kernel.hpp) the stages around it
 // cost as much as it does as launches of their own: the variables 25 us at 2048 waters, the 2B chain rule
 // 18, the 3B chain rule on one wavefront of a block, reading variables and gradient back from memory in nine
 // dependent groups, 50.  Nothing of an n-mer but its energy goes through memory here.

@@ -8,8 +8,9 @@
 //
 // The polynomial is evaluated in symmetry-adapted coordinates (mbx_amd/gen/symmetry.py): sums and
 // differences of the variables that exchanges of like sites permute.  In them a fraction of the
-// monomials survives (MB-pol 3B 6,773 of 33,525: 17.1k FP64 operations a trimer for value and
-// gradient instead of 72.5k; 2B 6.5k instead of 27.5k; CH4-H2O-H2O 11.7k instead of 63.0k), which is
+// monomials survives (MB-pol 3B 6,773 of 33,525: 20.0k FP64 operations a trimer for value and
+// gradient instead of 72.5k; 2B 7.2k instead of 27.5k; CH4-H2O-H2O 14.3k instead of 63.0k; a sixth of them
+// carries what rounding the coefficients left, without which energies have an error that grows with the system), which is
 // what bounds these kernels: at full occupancy they run at 95-99% of the FP64 issue slots, alone on
 // the chip at one wavefront's serial length.  The transform (SYM, in place on the registers, its own
 // transpose) costs one to three additions a variable each way.  Whole steps, before and after: 2048

@@ -72,6 +72,7 @@ class Schedule:
 
     def __init__(self, nvars, terms):
         self.nvars = nvars
+        self.rest_vars = {}  # part: variables whose gradient holds second coefficients' terms already
         # coefficient slots are opaque ints indexing the derived table C
         by_deg = collections.defaultdict(list)
         for q, m in terms:
@@ -151,26 +152,51 @@ class Schedule:
                     deg2_const=len(self.const2), level1_nodes=len(self.nodes1), fp64_ops_eg=ops)
 
     # ---------------------------------------------------------------------------------------
-    def partition(self, nparts):
+    def item_of(self):
+        """{monomial: the item of partition() that evaluates it}."""
+        out = {}
+        for n, l in self.leaves3.items():
+            out.update((tuple(sorted(n + (v,))), ("n2", n[:2])) for _, v in l)
+        out.update((m, ("n2", m[:2])) for m in self.const3)
+        for n, l in self.leaves2.items():
+            out.update((tuple(sorted(n + (v,))), ("n2", n)) for _, v in l)
+        out.update((m, ("n2", m)) for m in self.const2)
+        for n, l in self.leaves1.items():
+            out.update((tuple(sorted(n + (v,))), ("x1", n)) for _, v in l)
+        out.update((m, ("x1", m)) for m in self.const1)
+        out.update(((v,), ("z",)) for _, v in self.leaves0)
+        out[()] = ("z",)
+        return out
+
+    def partition(self, nparts, rests=()):
         """Split the schedule into nparts pieces of near-equal op count.  Items are level-2
         subtrees, each level-1 node's own terms ('x1'), and the degree-0/1 terms ('z');
         everything is linear in the pieces, so value and gradient are sums over parts.
-        Longest-processing-time assignment; returns {item: part}."""
+        Longest-processing-time assignment; returns {item: part}.  rests: the monomials with a second
+        coefficient, evaluated by their piece too (some three operations each).  A level-1 node's constant goes with
+        one of its subtrees: alone it would be rounded the same way in every n-mer where it is
+        added to the gradient."""
         items = []
+        second = collections.Counter(self.item_of()[m] for m in rests)
+        lone = [n1 for n1 in self.nodes1 if n1 in self.const1 and not self.leaves1.get(n1)]
         for n1 in self.nodes1:
             for n2 in self.children1.get(n1, []):
                 c = 3 + 2 * len(self.leaves2.get(n2, [])) + (1 if n2 in self.const2 else 0)
                 for n3 in self.children2.get(n2, []):
                     c += 3 + 2 * len(self.leaves3[n3]) + (1 if n3 in self.const3 else 0)
                 items.append((c, ("n2", n2)))
-            items.append((2 + 2 * len(self.leaves1.get(n1, [])) + (1 if n1 in self.const1 else 0), ("x1", n1)))
+            if n1 not in lone:
+                items.append((2 + 2 * len(self.leaves1.get(n1, [])) + (1 if n1 in self.const1 else 0), ("x1", n1)))
         items.append((1 + 2 * len(self.leaves0), ("z",)))
         load = [0] * nparts
         assign = {}
+        items = [(c + 3 * second[it], it) for c, it in items]
         for c, it in sorted(items, key=lambda t: (-t[0], t[1])):
             k = min(range(nparts), key=lambda j: (load[j], j))
             assign[it] = k
             load[k] += c
+        for n1 in lone:
+            assign[("x1", n1)] = assign[("n2", self.children1[n1][0])]
         self.part_load = load
         return assign
 
@@ -194,6 +220,7 @@ class Schedule:
                 if grad:
                     w("g[%d] += {c};" % l, q)
         i1 = i2 = i3 = 0
+        fresh = set(self.rest_vars.get(part, ()))  # those without other terms yet
         for n1 in self.nodes1:
             p = n1[0]
             kids = [n2 for n2 in self.children1.get(n1, []) if mine(("n2", n2))]
@@ -206,6 +233,16 @@ class Schedule:
                 w("double %s = {c};" % R1, self.const1[n1])
             else:
                 w("double %s = 0.0;" % R1)
+            leaves1 = self.leaves1.get(n1, []) if own else []
+            for n2 in kids:
+                fresh.discard(n2[1])
+                for n3 in self.children2.get(n2, []):
+                    fresh -= {n3[2]} | set(l for _, l in self.leaves3[n3])
+                fresh -= set(l for _, l in self.leaves2.get(n2, []))
+            fresh -= set(l for _, l in leaves1)
+            # R1 is rounded already, and added to rests alone it would round them away: the first
+            # product that goes to it is added to them first
+            held = None
             for n2 in kids:
                 qv = n2[1]
                 P2, R2 = "P2_%d" % i2, "R2_%d" % i2
@@ -241,13 +278,21 @@ class Schedule:
                         w("g[%d] = __fma_rn({c}, %s, g[%d]);" % (l, P2, l), q)
                 if grad:
                     w("g[%d] = __fma_rn(x[%d], %s, g[%d]);" % (qv, p, R2, qv))
-                w("%s = __fma_rn(x[%d], %s, %s);" % (R1, qv, R2, R1))
-            for q, l in (self.leaves1.get(n1, []) if own else []):
+                if p in fresh:
+                    fresh.discard(p)
+                    if grad:
+                        w("g[%d] = __fma_rn(x[%d], %s, g[%d]);" % (p, qv, R2, p))
+                    held = (qv, R2)
+                else:
+                    w("%s = __fma_rn(x[%d], %s, %s);" % (R1, qv, R2, R1))
+            for q, l in leaves1:
                 w("%s = __fma_rn({c}, x[%d], %s);" % (R1, l, R1), q)
                 if grad:
                     w("g[%d] = __fma_rn({c}, x[%d], g[%d]);" % (l, p, l), q)
             if grad:
                 w("g[%d] += %s;" % (p, R1))
+            if held:
+                w("%s = __fma_rn(x[%d], %s, %s);" % (R1, held[0], held[1], R1))
             w("E = __fma_rn(x[%d], %s, E);" % (p, R1))
         return o
 
@@ -326,7 +371,31 @@ def adapted(name):
 # block of 64 n-mers (each wavefront evaluating NPARTS / P pieces).  A piece takes the running
 # value E0 and returns it with its own terms added; its first fence consumes E0, so no
 # arithmetic of the previous piece can sink into it.
+#
+# The second coefficients (symmetry.py) are a polynomial of their own, evaluated before the other: each
+# of its terms is less than half a unit in the last place of the first coefficient's, so added to a sum that
+# already holds that one it would be rounded away every time.  Sums that start from the rests are rounded
+# with them, up or down by where they fall, and the rests arrive on average over n-mers.  A rest is in the piece
+# of its monomial, where the sums it goes to are never left with rests alone.
 NPARTS = 8
+
+
+def schedules(nvars, sym, nparts):
+    """The polynomial's schedule, its partition, and per part the schedule of the second coefficients'
+    terms (None without any) with a partition that puts all of them there."""
+    nrow = len(sym.rows)
+    kind = TrieSchedule if max(len(m) for _, m in sym.terms) > 4 else Schedule
+    s = kind(nvars, [t for t in sym.terms if t[0] < nrow])
+    second = [(q, tuple(sorted(m))) for q, m in sym.terms if q >= nrow]
+    assign = s.partition(nparts, [m for _, m in second])
+    item = s.item_of()
+    rests = []
+    for k in range(nparts):
+        terms = [(q, m) for q, m in second if assign[item[m]] == k]
+        r = kind(nvars, terms) if terms else None
+        rests.append((r, {it: k for it in r.partition(1)} if r else None))
+        s.rest_vars[k] = set(v for _, m in terms for v in m)
+    return s, assign, rests
 
 
 WRITTEN = set()
@@ -395,14 +464,15 @@ def generate_holder(name, out_dir):
 def blocked_source(name, fn, energy_only=True):
     """The .inc of a polynomial in symmetry-adapted coordinates, cut into NPARTS parts."""
     nvars, coef, sym = adapted(name)
-    deep = max(len(m) for _, m in sym.terms) > 4
-    s = (TrieSchedule if deep else Schedule)(nvars, sym.terms)
-    assign = s.partition(NPARTS)
+    s, assign, rests = schedules(nvars, sym, NPARTS)
     c = s.counts()
+    c["fp64_ops_eg"] += sum(r.counts()["fp64_ops_eg"] for r, _ in rests if r)
+    c["second_coefficient_terms"] = len([q for q, _ in sym.terms if q >= len(sym.rows)])
     hdr = ["// GENERATED by mbx_amd/gen/polygen.py from mbx_amd/tables/%s.tbl -- do not edit." % name,
            "// Schedule: %s" % ", ".join("%s=%d" % kv for kv in c.items()),
            "// %d parts (op-count balance: %s); <fn>_parts(w, P, ...) evaluates parts w, w+P, ... "
-           "into g and e[64 * part]." % (NPARTS, ", ".join(str(v) for v in s.part_load)),
+           "into g and e[64 * part], the second coefficients' terms (_r<part>) first."
+           % (NPARTS, ", ".join(str(v) for v in s.part_load)),
            "// Symmetry-adapted coordinates: %s_sym transforms x before and g after; C holds %d slots "
            "(gen/sym_%s.inc)." % (fn, len(sym.rows) + len(sym.low), name),
            "#pragma once",
@@ -411,17 +481,25 @@ def blocked_source(name, fn, energy_only=True):
     for grad, suffix in ((True, ""), (False, "_e")):
         if not grad and not energy_only:
             continue
-        for k in range(NPARTS):
+        first = [k for k, (r, _) in enumerate(rests) if r]
+        for k, (r, where) in enumerate(rests):
+            if r:
+                body.append(r.emit("%s%s_r%d" % (fn, suffix, k), grad=grad, part=k, assign=where))
             body.append(s.emit("%s%s_p%d" % (fn, suffix, k), grad=grad, part=k, assign=assign))
-        args, call = (("mbxg_cptr C, const double* x, double* g", "C, x, g, 0.0") if grad
-                      else ("mbxg_cptr C, const double* x", "C, x, 0.0"))
+        args, call = (("mbxg_cptr C, const double* x, double* g", "C, x, g, %s") if grad
+                      else ("mbxg_cptr C, const double* x", "C, x, %s"))
         # wavefront w of P evaluates pieces w, w + P, ...: a straight sequence of uniform
         # branches (a switch over the pieces inside a loop costs the register allocator dearly).
         # Each piece's share of the value goes to its own place, so that the sum over the pieces
         # (poly_value) is the same for every P.
         d = ["__device__ __forceinline__ void %s%s_parts(int w, int P, %s, double* e) {" % (fn, suffix, args)]
+        d += ["    if ((%d & (P - 1)) == w) e[%d] = %s%s_r%d(%s);" % (k, 64 * k, fn, suffix, k, call % "0.0")
+              for k in first]
+        if first:  # (a piece and its rests share products, which would be live all the way)
+            d.append("    mbxg_opaque<%d>(x);" % nvars)
         for k in range(NPARTS):
-            d.append("    if ((%d & (P - 1)) == w) e[%d] = %s%s_p%d(%s);" % (k, 64 * k, fn, suffix, k, call))
+            d.append("    if ((%d & (P - 1)) == w) e[%d] = %s%s_p%d(%s);" % (
+                k, 64 * k, fn, suffix, k, call % ("e[%d]" % (64 * k) if k in first else "0.0")))
         d += ["}", ""]
         body.append("\n".join(d))
     return "\n".join(hdr) + "\n".join(body), c
@@ -671,8 +749,9 @@ def generate_ad(name, out_dir):
     """gen/ad_<name>_tan.{inc,hip} and gen/ad_<name>_basis.{inc,hip}: two translation units
     (compiled in parallel), each with its kernel's launcher."""
     nvars, coef, sym = adapted(name)
-    s = Schedule(nvars, sym.terms)
-    assign = s.partition(AD_PARTS)
+    s, assign, rests = schedules(nvars, sym, AD_PARTS)
+    pieces = [("r", k, r, where) for k, (r, where) in enumerate(rests) if r]  # before the part's others
+    pieces += [("p", k, s, assign) for k in range(AD_PARTS)]
     fn = "ad_%s" % name
     nrow = len(sym.rows)
     monos = [(q, m) for q, m in sym.terms if q < nrow]
@@ -681,11 +760,11 @@ def generate_ad(name, out_dir):
                          "// %s" % what, "#pragma once", "#include \"poly_support.hpp\"", "#include \"ad_kernel.hpp\"",
                          "", "namespace mbxg {", ""]
     # gradient tangent (Hessian-vector product), AD_PARTS parts
-    body = [emit_dual(s, "%s_tan_p%d" % (fn, k), k, assign, tangent_only=True) for k in range(AD_PARTS)]
+    body = [emit_dual(p, "%s_tan_%s%d" % (fn, w, k), k, where, tangent_only=True) for w, k, p, where in pieces]
     body.insert(0, symmetry.emit_transform("%s_tan_sym" % fn, sym.blocks))
     d = ["__device__ __forceinline__ void %s_tan(int part, mbxg_cptr C, const double* x, const double* xd, "
          "double* gd) {" % fn]
-    d += ["    if (part == %d) %s_tan_p%d(C, x, xd, gd);" % (k, fn, k) for k in range(AD_PARTS)]
+    d += ["    if (part == %d) %s_tan_%s%d(C, x, xd, gd);" % (k, fn, w, k) for w, k, _, _ in pieces]
     d += ["}", "", "}  // namespace mbxg", ""]
     write_if_changed(os.path.join(out_dir, "ad_%s_tan.inc" % name),
                      "\n".join(head("Gradient tangent of the polynomial (H xd) in %d parts." % AD_PARTS))
@@ -849,32 +928,34 @@ XKIND = {"h2o": "MON_H2O", "ch4": "MON_CH4", "co2": "MON_CO2", "f-": "MON_F", "c
 class TrieSchedule:
     """Terms of any degree in reverse mode over the full monomial trie (as emit_trie), with the parts
     interface of Schedule: a part is a set of level-2 subtrees, each level-1 node's own terms and the
-    terms of degree 0.  A second coefficient of a monomial (symmetry.py) is applied where its node meets
-    its parent, so it is not rounded away against the first."""
+    terms of degree 0."""
 
     def __init__(self, nvars, terms):
         self.nvars = nvars
-        self.coef = collections.defaultdict(list)
-        for q, m in terms:
-            self.coef[tuple(sorted(m))].append(q)
+        self.rest_vars = {}  # as in Schedule
+        self.coef = {tuple(sorted(m)): q for q, m in terms}
         self.children = collections.defaultdict(set)
         for m in self.coef:
             for d in range(1, len(m) + 1):
                 self.children[m[:d - 1]].add(m[d - 1])
 
     def _size(self, node):
-        return 2 * len(self.coef.get(node, [])) + sum(3 + self._size(node + (v,)) for v in self.children.get(node, ()))
+        return sum(3 + self._size(node + (v,)) for v in self.children.get(node, ()))
 
     def counts(self):
         n = sum(len(v) for v in self.children.values())
-        second = sum(len(q) - 1 for q in self.coef.values())
-        return dict(nodes=n, monomials=len(self.coef), second=second, fp64_ops_eg=3 * n + 2 * second)
+        return dict(nodes=n, monomials=len(self.coef), fp64_ops_eg=3 * n)
 
-    def partition(self, nparts):
+    def item_of(self):
+        return {m: m[:2] for m in self.coef}
+
+    def partition(self, nparts, rests=()):
+        second = collections.Counter(m[:2] for m in rests)
         items = [(1, ())]
         for v in self.children[()]:
             items.append((4, (v,)))
             items += [(4 + self._size((v, w)), (v, w)) for w in self.children.get((v,), ())]
+        items = [(c + 3 * second[it], it) for c, it in items]
         load, assign = [0] * nparts, {}
         for c, it in sorted(items, key=lambda t: (-t[0], t[1])):
             k = min(range(nparts), key=lambda j: (load[j], j))
@@ -898,12 +979,14 @@ class TrieSchedule:
 
         names = [0]
 
+        fresh = set(self.rest_vars.get(part, ()))
+
         def walk(node, product, own=True, kids=None):
-            """Statements of the subtree; returns the name of its adjoint R."""
+            """Statements of the subtree; returns the name of its adjoint R, and what is not in it yet (Schedule.ops)."""
+            first = None
             names[0] += 1
             r = "R%d" % names[0]
-            q = self.coef.get(node, []) if own else []
-            w("double %s = %s;" % (r, "C[%d]" % q[0] if q else "0.0"), r)
+            w("double %s = %s;" % (r, "C[%d]" % self.coef[node] if own and node in self.coef else "0.0"), r)
             for v in sorted(self.children.get(node, ()) if kids is None else kids):
                 child = node + (v,)
                 pc = None
@@ -911,29 +994,29 @@ class TrieSchedule:
                     names[0] += 1
                     pc = "P%d" % names[0]
                     w("const double %s = %s;" % (pc, "%s * x[%d]" % (product, v)))
-                meet(child, v, walk(child, pc), r, product)
-            return r
+                rc, _ = walk(child, pc)
+                w("g[%d] = __fma_rn(%s, %s, g[%d]);" % (v, product, rc, v))
+                fresh.discard(v)
+                if len(node) == 1 and node[0] in fresh:
+                    fresh.discard(node[0])
+                    w("g[%d] = __fma_rn(x[%d], %s, g[%d]);" % (node[0], v, rc, node[0]))
+                    first = (v, rc)
+                else:
+                    w("%s = __fma_rn(x[%d], %s, %s);" % (r, v, rc, r), r)
+            return r, first
 
-        def meet(child, v, rc, r, product):
-            """The child's adjoint, and its monomial's second coefficients, into g and the parent's r."""
-            for c in [rc] + ["C[%d]" % q for q in self.coef.get(child, [])[1:]]:
-                w("g[%d] = __fma_rn(%s, %s, g[%d]);" % (v, product, c, v))
-                w("%s = __fma_rn(x[%d], %s, %s);" % (r, v, c, r), r)
-
-        if assign[()] == part:
-            for q in self.coef.get((), []):
-                w("E += C[%d];" % q)
+        if assign[()] == part and () in self.coef:
+            w("E += C[%d];" % self.coef[()])
         for v in sorted(self.children[()]):
             kids = [u for u in self.children.get((v,), ()) if assign[(v, u)] == part]
             own = assign[(v,)] == part
             if not kids and not own:
                 continue
-            rc = walk((v,), "x[%d]" % v, own, kids)
+            rc, first = walk((v,), "x[%d]" % v, own, kids)
             w("g[%d] += %s;" % (v, rc))
+            if first:
+                w("%s = __fma_rn(x[%d], %s, %s);" % (rc, first[0], first[1], rc))
             w("E = __fma_rn(x[%d], %s, E);" % (v, rc))
-            for q in self.coef.get((v,), [])[1:] if own else []:
-                w("g[%d] += C[%d];" % (v, q))
-                w("E = __fma_rn(x[%d], C[%d], E);" % (v, q))
         w("return E;")
         out.append("}")
         return "\n".join(out) + "\n"

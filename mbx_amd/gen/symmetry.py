@@ -15,13 +15,13 @@ the 33,525 monomials of the MB-pol 3B polynomial become 6,773, the 201,250 of CH
 is the same polynomial with the same value; its gradient follows by the (symmetric) transform,
 dE/dx = H dE/du.
 
-The new coefficients are fixed linear combinations b = T a of the fitted ones, with weights that are
-multiples of powers of two (exact in binary).  Most tables have as many distinct combinations as
-coefficients.  A combination of several coefficients rounds once, the same way in every n-mer, so over
-many n-mers that error would add up where the others average out (MB-pol 3B: 1.4e-10 kcal/mol over 200
-close trimers against 2e-11 in the original coordinates).  It comes from few combinations: those that
-matter most carry a second coefficient with the rounded-off rest, on the same monomials (6% more
-operations; the sum above falls to 1e-11).
+The new coefficients are fixed linear combinations b = T a of the fitted ones, with dyadic weights.  Most
+tables have as many distinct combinations as coefficients.  A combination rounds once, the same way in
+every n-mer, so over many n-mers that error adds up where the others average out: 256 waters lose 2.5e-9
+(2B) and 3.3e-9 (3B) kcal/mol to it, where the original coordinates are off by 4e-10 and 1e-10 either way.  It
+comes from few combinations: those that matter most, for the monomials they cost, carry a second coefficient
+with the rounded-off rest on the same monomials.  With REST of the error left 256 waters are off by some 2e-11
+of that kind in each order, less than the random error of the largest boxes in use.
 """
 import collections
 import itertools
@@ -56,9 +56,10 @@ EXCHANGES = {
     "co2x3_3b": _WATERS[3],
     "h2ox4_4b": _WATERS[4],
 }
-# a holder with the structure's variables, where the structure serves several
-_HOLDER = {"halide_h2o_2b": "cl_h2o_2b", "alkali_h2o_2b": "na_h2o_2b", "halide_h2o2_3b": "cl_h2o2_3b",
-           "alkali_h2o2_3b": "na_h2o2_3b"}
+# the holders of the structures that serve several
+_HOLDERS = {s + t: [i + t for i in ions] for s, ions in (("halide", ("cl", "f", "br", "i")),
+                                                         ("alkali", ("na", "li", "k", "rb", "cs")))
+            for t in ("_h2o_2b", "_h2o2_3b")}
 
 # MB-pol: (rate, offset, Coulomb-like) of each variable class (2B x2b-v9x.cpp:1330-1345, 3B x3b-v2x.cpp:1256-1271)
 _MBPOL_CLASS = {
@@ -82,30 +83,73 @@ _MBPOL = {
 
 
 def _holder(name):
-    with open(os.path.join(TABLES, _HOLDER.get(name, name) + ".holder.json")) as f:
+    with open(os.path.join(TABLES, _HOLDERS.get(name, [name])[0] + ".holder.json")) as f:
         return json.load(f)
 
 
-def sample_variables(name, n):
-    """(nvars, n) variables of typical size: separations of 0.95-1.6 A inside a molecule, 2-5 A between."""
+# Sites of a molecule (Angstrom) and its centre's distance to a neighbour's, at least
+_SHAPE = {
+    "h2o": [(0.0, 0.0, 0.0), (0.757, 0.587, 0.0), (-0.757, 0.587, 0.0)],
+    "ch4": [(0.0, 0.0, 0.0), (0.629, 0.629, 0.629), (0.629, -0.629, -0.629), (-0.629, 0.629, -0.629),
+            (-0.629, -0.629, 0.629)],
+    "co2": [(0.0, 0.0, 0.0), (1.16, 0.0, 0.0), (-1.16, 0.0, 0.0)],
+}
+_CONTACT = {"h2o": 2.5, "ch4": 3.4, "co2": 3.4}
+_LONE_PAIR = (-0.0972, 0.0986)  # in the plane, out of it (x2b-v9x.cpp:1346-1347)
+
+
+def sample_nmers(name, n):
+    """(variables (nvars, n), switch (n)) of n-mers as a liquid has them: the molecules' centres anywhere
+    around the first one that the switch and the neighbours leave, random orientations, vibrating bonds."""
+    rng = np.random.default_rng(1)
     if name in _MBPOL:
-        cls = _MBPOL_CLASS[name]
-        vs = [cls[c] + (a, b) for c, a, b in _MBPOL[name]]
-        atoms, water = [3] * (3 if name == "mbpol_3b" else 2), [0, 0, 1, 1]
+        order = 3 if name == "mbpol_3b" else 2
+        mols = ["h2o"] * order
+        vs = [(k, d, f, a, b) for c, a, b in _MBPOL[name] for k, d, f in [_MBPOL_CLASS[name][c]]]
+        inner, outer = (4.5, 6.5) if order == 2 else (0.0, 4.5)
+        lone = [0, 3] if order == 2 else []
     else:
         h = _holder(name)
+        mols = h["monomers"]
         vs = [(k, d if f in ("exp0", "coul0") else 0.0, f in ("coul0", "coul"), a, b) for f, k, d, a, b in h["vars"]]
-        atoms = h["atoms"]
-        water = [m for m, kind in enumerate(h["monomers"]) if kind == "h2o" for _ in (0, 1)]
-    mol = [m for m, k in enumerate(atoms) for _ in range(k)]
-    mol += water  # lone-pair sites follow the atoms, two a water
-    rng = np.random.default_rng(1)
-    out = []
+        inner, outer = h["switch"]["inner"], h["switch"]["outer"]
+        lone = [v["oxygen_site"] for v in (h["vsites"] if "vsites" in h else [h["vsite"]] if h.get("vsite") else [])]
+    centres, count = [], 0
+    while count < n:
+        c = rng.uniform(-outer, outer, (8 * n, len(mols), 3))
+        c[:, 0] = 0.0
+        ok = np.ones(len(c), bool)
+        far = np.zeros(len(c), int)
+        for i in range(len(mols)):
+            for j in range(i):
+                r = np.linalg.norm(c[:, i] - c[:, j], axis=1)
+                ok &= r > (_CONTACT.get(mols[i], 2.5) + _CONTACT.get(mols[j], 2.5)) / 2
+                far += r > outer
+        centres.append(c[ok & (far <= (len(mols) == 3))])  # three-body switches: sums over two of the pairs
+        count += len(centres[-1])
+    c = np.concatenate(centres)[:n]
+    pairs = [(i, j) for i in range(len(mols)) for j in range(i)]
+    sw = []
+    for i, j in pairs:
+        t = np.clip((np.linalg.norm(c[:, i] - c[:, j], axis=1) - inner) / (outer - inner), 0.0, 1.0)
+        sw.append(0.5 * (1.0 + np.cos(np.pi * t)))
+    weight = sw[0] * sw[1] + sw[0] * sw[2] + sw[1] * sw[2] if len(mols) == 3 else np.prod(sw, axis=0)
+    sites = []
+    for m, kind in enumerate(mols):
+        body = np.array(_SHAPE.get(kind, [(0.0, 0.0, 0.0)]))
+        q = np.linalg.qr(rng.normal(size=(n, 3, 3)))[0]
+        at = (body + rng.normal(0.0, 0.03, (n,) + body.shape) * (np.abs(body).sum(1) > 0)[:, None]) @ q
+        sites += [c[:, m] + at[:, k] for k in range(len(body))]
+    for o in lone:
+        p, q = sites[o + 1] - sites[o], sites[o + 2] - sites[o]
+        mid, out = sites[o] + 0.5 * _LONE_PAIR[0] * (p + q), _LONE_PAIR[1] * np.cross(p, q)
+        sites += [mid + out, mid - out]
+    x = []
     for k, d, coulomb, a, b in vs:
-        r = rng.uniform(0.95, 1.6, n) if mol[a] == mol[b] else rng.uniform(2.0, 5.0, n)
+        r = np.linalg.norm(sites[a] - sites[b], axis=1)
         v = np.exp(k * (d - r))
-        out.append(v / r if coulomb else v)
-    return np.array(out)
+        x.append(v / r if coulomb else v)
+    return np.array(x), weight
 
 
 def variable_permutations(name):
@@ -137,7 +181,7 @@ def _parity(v):
 
 
 # Share of the combinations' rounding error that may stay without a second coefficient.
-REST = 1.0 / 10.0
+REST = 1.0 / 60.0
 
 
 class Adapted:
@@ -198,20 +242,25 @@ class Adapted:
 
     def _second_coefficients(self, name, coef):
         """Terms for the rests of the combinations that carry all but REST of the rounding error, judged
-        by |b| times the combination's monomials on sampled variables."""
-        u = self.transform(sample_variables(name, 256))
-        size = np.zeros((len(self.rows), u.shape[1]))
-        for q, m in self.terms:
-            size[q] += np.prod(u[list(m)], axis=0) if m else 1.0
-        weight = np.zeros(len(self.rows))
-        for q, r in enumerate(self.rows):
-            if len(r) > 1:
-                weight[q] = max(abs(coef[k] * w) for k, w in r) * math.sqrt((size[q] ** 2).mean())
-        order = np.argsort(-weight, kind="stable")
-        left = np.cumsum((weight ** 2)[order][::-1])[::-1]  # what stays if order[i:] have none
-        count = int((left > REST ** 2 * left[0]).sum())
-        self.low = sorted(order[:count].tolist())
-        at = {q: len(self.rows) + j for j, q in enumerate(self.low)}
+        on sampled n-mers (of every holder that the structure serves)."""
+        nrow = len(self.rows)
+        count = np.bincount([q for q, _ in self.terms], minlength=nrow)
+        rounded = np.array([len(r) > 1 or math.frexp(r[0][1])[0] not in (0.5, -0.5) for r in self.rows])
+        share = np.zeros(nrow)
+        for holder in _HOLDERS.get(name, [name]):
+            a = _holder(holder)["coef"] if name in _HOLDERS else coef
+            x, switch = sample_nmers(holder, 512)
+            u = self.transform(x)
+            size = np.zeros((nrow, u.shape[1]))
+            for q, m in self.terms:
+                size[q] += np.prod(u[list(m)], axis=0) if m else 1.0
+            b = np.array([sum(a[k] * w for k, w in r) for r in self.rows])
+            err = b ** 2 * ((size * switch) ** 2).mean(axis=1) * rounded  # a rounded b's, in units of 2^-53 / sqrt(3)
+            share = np.maximum(share, err / err.sum())
+        order = np.argsort(-share / count, kind="stable")
+        left = np.cumsum(share[order][::-1])[::-1]  # what stays if order[i:] have none
+        self.low = sorted(order[:int((left > REST ** 2).sum())].tolist())
+        at = {q: nrow + j for j, q in enumerate(self.low)}
         self.terms += [(at[q], m) for q, m in self.terms if q in at]
 
     def _expand(self, monos, elements, char, inv):
