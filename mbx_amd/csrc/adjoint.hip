@@ -36,6 +36,7 @@
 #include <mutex>
 
 #include "ad_kernel.hpp"
+#include "ad_slot.hpp"
 #include "gen/coef_mbpol_2b.inc"
 #include "gen/coef_mbpol_3b.inc"
 #define MBXG_SYM_SPACE static __device__
@@ -68,32 +69,6 @@ struct AdVar {
 };
 
 constexpr int kNTheta = 10;
-
-// Slot q of the symmetry-adapted polynomial's coefficients (gen/sym_<name>.inc): the products with
-// the weights are exact, the sum is carried with its rounding errors, so slots at or past nrow get
-// what rounding left of slot low[q - nrow].
-__device__ __forceinline__ double ad_slot(const int* row, const unsigned short* k, const double* w,
-                                          const unsigned short* low, int nrow, int q,
-                                          const double* __restrict__ coef) {
-    const int r = q < nrow ? q : low[q - nrow];
-    double s = 0.0, err = 0.0;
-    for (int i = row[r]; i < row[r + 1]; ++i) {
-        const double p = coef[k[i]] * w[i];
-        const double t = s + p, z = t - s;
-        err += (s - (t - z)) + (p - z);
-        s = t;
-    }
-    const double b = s + err;
-    return q < nrow ? b : err - (b - s);
-}
-
-// Entry k of the transposed map: the fitted coefficient's gradient from the slots' (row[q]).
-__device__ __forceinline__ double ad_coef_adjoint(const int* start, const unsigned short* slot, const double* w, int k,
-                                                  const double* __restrict__ row) {
-    double s = 0.0;
-    for (int i = start[k]; i < start[k + 1]; ++i) s = __fma_rn(row[slot[i]], w[i], s);
-    return s;
-}
 
 // Sites 0..5 = Oa Ha1 Ha2 Ob Hb1 Hb2, 6..9 = Xa1 Xa2 Xb1 Xb2 (x2b-v9x.cpp:1640-1675).
 struct Ad2b {
