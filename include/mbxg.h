@@ -231,8 +231,10 @@ int mbxg_set_graph(mbxg_ctx* ctx, int on);
  * (the polynomial stage, `reps` timed repetitions after one warm-up) and, when CH4-H2O-H2O trimers
  * are evaluated, every split of that family (its whole evaluation), keeps the fastest of each,
  * then, on the paired path, the one launch against the separate ones with and without "fuse_vars"
- * (the whole compute), and recomputes once with them.  No counterpart in the reference (its
- * kernels have no launch shape). */
+ * (the whole compute), and recomputes once with them.  The 2B split is left alone on the paired path,
+ * where that polynomial is part of the 3B launch; a 3B split found without the comparison with the one
+ * launch (energies, or one order alone) does not turn that off.  On an error the schedule stays as it
+ * was.  No counterpart in the reference (its kernels have no launch shape). */
 int mbxg_set_tuning(mbxg_ctx* ctx, const char* key, int value);
 int mbxg_get_tuning(mbxg_ctx* ctx, const char* key, int* value);
 int mbxg_autotune(mbxg_ctx* ctx, int terms, int do_grads, int reps);

@@ -291,13 +291,18 @@ struct mbxg_ctx {
     bool one_body_last = false;  // the last compute evaluated the 1B term
     DBuf<double> d_wrap_in, d_wrap_out;  // mbxg_fix_coordinates
     int n_h2o = 0, n_ch4 = 0;             // monomers of each kind (mbxg_set_topology)
-    // wavefronts per 64 n-mers in the polynomial stages (mbxg_set_tuning / mbxg_autotune); 0: poly_split's
-    // rule.  CH4-H2O-H2O's is fixed, for a batch's gradients to be a lone configuration's to 1e-10.
-    int split2 = 0, split3 = 0, split3n = 4;
-    int fuse_poly = 1;       // MB-pol 2B and 3B polynomials in one launch when both are evaluated
-    int fuse_prep = 1;       // FixMonomerCoordinates, cloud and cell counts in one launch (k_cloud_fix)
-    int fuse_chain = 1;      // variables and chain rules in the paired polynomial launch (k_mbpol_fused)
-    int fuse_vars = 1;       // without fuse_chain: the paired path's 2B and 3B variables in one launch
+    struct Schedule {
+        // wavefronts per 64 n-mers in the polynomial stages (mbxg_set_tuning / mbxg_autotune); 0: poly_split's
+        // rule.  CH4-H2O-H2O's is fixed, for a batch's gradients to be a lone configuration's to 1e-10.
+        int split2 = 0, split3 = 0, split3n = 4;
+        // the autotuner's split of the 3B polynomial as a launch of its own (0: none found): unlike a split3
+        // set by hand it says nothing against the one launch of both orders
+        int tuned3 = 0;
+        int fuse_poly = 1;   // MB-pol 2B and 3B polynomials in one launch when both are evaluated
+        int fuse_prep = 1;   // FixMonomerCoordinates, cloud and cell counts in one launch (k_cloud_fix)
+        int fuse_chain = 1;  // variables and chain rules in the paired polynomial launch (k_mbpol_fused)
+        int fuse_vars = 1;   // without fuse_chain: the paired path's 2B and 3B variables in one launch
+    } tune;
     bool fused_last = false;  // the last compute did so (its 2B polynomial time is in the 3B one)
     // stage timing (mbxg_set_timing): events bracketing each stage of the last compute
     bool timing = false;
@@ -965,7 +970,7 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
     if (!c->box.periodic)
         hipLaunchKernelGGL(k_grid_gas, dim3(c->nconf), dim3(256), 0, st, c->d_in.p, c->d_first.p, c->d_members.p,
                            c->d_pt_off.p, L.d_cell_bound.p, cut, L.d_grids.p);
-    if (c->fuse_prep) {  // fix, cloud, cell counts and the zero fills Z in one launch (64-thread
+    if (c->tune.fuse_prep) {  // fix, cloud, cell counts and the zero fills Z in one launch (64-thread
                          // blocks: the cell-count atomics spread over many CUs; eight lanes a point)
         const int nt = std::max(c->nmon, 8 * np);
         hipLaunchKernelGGL(k_cloud_fix, dim3((nt + 63) / 64), dim3(64), 0, st, c->d_in.p, c->d_xyz.p, c->d_first.p,
@@ -1111,9 +1116,12 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
 // The wavefronts per 64 n-mers of a polynomial of nv variables: as set, else by the rule.
 int split_of(int set, int cap, int nv) { return set ? set : poly_split(cap, poly_wpe(nv)); }
 
+// MB-pol 3B's where it is not in the one launch.
+int split_3b(const mbxg_ctx* c, int cap) { return split_of(c->tune.split3 ? c->tune.split3 : c->tune.tuned3, cap, 36); }
+
 // Whether MB-pol's paired path runs as one launch (mbpol_fused.hip: four wavefronts per 64 n-mers); another
 // split set by hand takes the separate launches, which have them all.
-bool one_launch(const mbxg_ctx* c) { return c->fuse_chain && (c->split3 == 0 || c->split3 == kFusedSplit); }
+bool one_launch(const mbxg_ctx* c) { return c->tune.fuse_chain && (c->tune.split3 == 0 || c->tune.split3 == kFusedSplit); }
 
 PublishJob publish_job(const mbxg_ctx* c) {
     const ListState& L = c->L;
@@ -1244,7 +1252,7 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
         Z.p[1] = c->d_totals.p + 2 * kPartials;
         Z.n[1] = kPartials;
     }
-    if (!(L.built && c->fuse_prep)) {
+    if (!(L.built && c->tune.fuse_prep)) {
         hipLaunchKernelGGL(k_zero_multi, dim3(64), dim3(256), 0, st, Z);
         HIPCHK(hipGetLastError());
     }
@@ -1288,7 +1296,7 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
         };
         // the MB-pol 2B and 3B polynomials share one launch (k_poly_eg_pair) when both run with
         // gradients; everything of both families then runs on the main stream
-        const bool fuse = c->fuse_poly && do_grads && active(FAM_MBPOL_2B) && active(FAM_MBPOL_3B);
+        const bool fuse = c->tune.fuse_poly && do_grads && active(FAM_MBPOL_2B) && active(FAM_MBPOL_3B);
         c->fused_last = fuse;
         auto buffers = [&](int f) -> bool {  // false: allocation failed
             const int cap = fam_cap(L, f);
@@ -1351,17 +1359,17 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                         for (int k = 10; k <= 11; ++k) HIPCHK(hipEventRecord(ev[k], st));
                 } else {
                     if (ev) HIPCHK(hipEventRecord(ev[4], st));
-                    if (!c->fuse_vars) HIPCHK(launch_mbpol2b_vars(L.evals[f2].p, nd2, cap2, N, o2.ws.p, st));
+                    if (!c->tune.fuse_vars) HIPCHK(launch_mbpol2b_vars(L.evals[f2].p, nd2, cap2, N, o2.ws.p, st));
                     if (ev) HIPCHK(hipEventRecord(ev[5], st));
                     if (ev) HIPCHK(hipEventRecord(ev[8], st));
-                    if (c->fuse_vars)  // both orders' variables in one launch (timed as the 3B stage)
+                    if (c->tune.fuse_vars)  // both orders' variables in one launch (timed as the 3B stage)
                         HIPCHK(launch_mbpol_vars_pair(L.evals[f].p, nd, cap, o.ws.p, L.evals[f2].p, nd2, cap2, o2.ws.p,
                                                       N, st));
                     else
                         HIPCHK(launch_mbpol3b_vars(L.evals[f].p, nd, cap, N, o.ws.p, st));
                     if (ev) HIPCHK(hipEventRecord(ev[9], st));
                     HIPCHK(launch_poly_mbpol_pair(o.ws.p, nd, cap, c->d_coef3.p, o2.ws.p, nd2, cap2, c->d_coef2.p,
-                                                  split_of(c->split3, cap, 36), st));
+                                                  split_3b(c, cap), st));
                     if (ev) HIPCHK(hipEventRecord(ev[10], st));
                     HIPCHK(launch_mbpol3b_chain(L.evals[f].p, nd, cap, N, 1, c->d_grad.p, o.e_nmer.p, vir,
                                                 o.partials.p, o.ws.p, st));
@@ -1378,15 +1386,15 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
             }
             if (f == FAM_MBPOL_2B)
                 HIPCHK(launch_mbpol2b(L.evals[f].p, nd, cap, N, c->d_coef2.p, do_grads, c->d_grad.p, o.e_nmer.p, vir,
-                                      o.partials.p, o.ws.p, split_of(c->split2, cap, 31), sk, ev ? ev + 4 : nullptr));
+                                      o.partials.p, o.ws.p, split_of(c->tune.split2, cap, 31), sk, ev ? ev + 4 : nullptr));
             else if (f == FAM_MBPOL_3B)
                 HIPCHK(launch_mbpol3b(L.evals[f].p, nd, cap, N, c->d_coef3.p, do_grads, c->d_grad.p, o.e_nmer.p, vir,
-                                      o.partials.p, o.ws.p, split_of(c->split3, cap, 36), sk, ev ? ev + 8 : nullptr));
+                                      o.partials.p, o.ws.p, split_3b(c, cap), sk, ev ? ev + 8 : nullptr));
             else {
                 const bool timed = ev && f == FAM_CH4H2O2_3B;
                 if (timed) HIPCHK(hipEventRecord(ev[13], st));
                 HIPCHK(launch_nrg_family(f, L.evals[f].p, nd, cap, N, c->d_coefn[f].p, do_grads, c->d_grad.p,
-                                         o.e_nmer.p, vir, o.partials.p, o.ws.p, split_of(c->split3n, cap, 55), sk,
+                                         o.e_nmer.p, vir, o.partials.p, o.ws.p, split_of(c->tune.split3n, cap, 55), sk,
                                          nullptr));
                 if (timed) HIPCHK(hipEventRecord(ev[14], st));
             }
@@ -1584,6 +1592,7 @@ namespace {
 
 bool valid_split(int v) { return v == 1 || v == 2 || v == 4 || v == 8; }
 
+
 }  // namespace
 
 extern "C" int mbxg_set_tuning(mbxg_ctx* c, const char* key, int value) {
@@ -1594,19 +1603,20 @@ extern "C" int mbxg_set_tuning(mbxg_ctx* c, const char* key, int value) {
     if ((k == "fuse_poly" || k == "fuse_prep" || k == "fuse_chain" || k == "fuse_vars") && value != 0 && value != 1)
         return fail(MBXG_EINVAL, "mbxg_set_tuning: %s is 0 or 1", key);
     if (k == "split_2b")
-        c->split2 = value;
-    else if (k == "split_3b")
-        c->split3 = value;
-    else if (k == "split_ch4h2o2_3b")
-        c->split3n = value;
+        c->tune.split2 = value;
+    else if (k == "split_3b") {
+        c->tune.split3 = value;
+        c->tune.tuned3 = 0;
+    } else if (k == "split_ch4h2o2_3b")
+        c->tune.split3n = value;
     else if (k == "fuse_poly")
-        c->fuse_poly = value;
+        c->tune.fuse_poly = value;
     else if (k == "fuse_prep")
-        c->fuse_prep = value;
+        c->tune.fuse_prep = value;
     else if (k == "fuse_chain")
-        c->fuse_chain = value;
+        c->tune.fuse_chain = value;
     else if (k == "fuse_vars")
-        c->fuse_vars = value;
+        c->tune.fuse_vars = value;
     else
         return fail(MBXG_EINVAL, "mbxg_set_tuning: unknown key '%s'", key);
     drop_graph(c);  // another schedule may need other workspaces: an eager compute first
@@ -1617,108 +1627,123 @@ extern "C" int mbxg_get_tuning(mbxg_ctx* c, const char* key, int* value) {
     if (!c || !key || !value) return fail(MBXG_EINVAL, "mbxg_get_tuning: bad arguments");
     const std::string k(key);
     if (k == "split_2b")
-        *value = split_of(c->split2, fam_cap(c->L, FAM_MBPOL_2B), 31);
+        *value = split_of(c->tune.split2, fam_cap(c->L, FAM_MBPOL_2B), 31);
     else if (k == "split_3b")
-        *value = split_of(c->split3, fam_cap(c->L, FAM_MBPOL_3B), 36);
+        *value = split_3b(c, fam_cap(c->L, FAM_MBPOL_3B));
     else if (k == "split_ch4h2o2_3b")
-        *value = split_of(c->split3n, fam_cap(c->L, FAM_CH4H2O2_3B), 55);
+        *value = split_of(c->tune.split3n, fam_cap(c->L, FAM_CH4H2O2_3B), 55);
     else if (k == "fuse_poly")
-        *value = c->fuse_poly;
+        *value = c->tune.fuse_poly;
     else if (k == "fuse_prep")
-        *value = c->fuse_prep;
+        *value = c->tune.fuse_prep;
     else if (k == "fuse_chain")
-        *value = c->fuse_chain;
+        *value = c->tune.fuse_chain;
     else if (k == "fuse_vars")
-        *value = c->fuse_vars;
+        *value = c->tune.fuse_vars;
     else
         return fail(MBXG_EINVAL, "mbxg_get_tuning: unknown key '%s'", key);
     return MBXG_OK;
 }
 
-// Autotuner: time the polynomial stage of each order for every split on the current inputs
-// (HIP events, stages run one at a time), keep the fastest, then recompute once so the results
-// are those of the chosen schedule.
-extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
-    if (!c) return fail(MBXG_EINVAL, "mbxg_autotune: null context");
-    if (!c->have_coords) return fail(MBXG_ESTATE, "mbxg_autotune: coordinates not set");
-    if (reps < 1) reps = 1;
-    const bool was_timing = c->timing;
-    if (int r = mbxg_set_timing(c, 1)) return r;
-    const int cand[4] = {1, 2, 4, 8};
-    double best[2] = {1e300, 1e300};
-    int pick[2] = {c->split2, c->split3};
-    const int fuse_chain = c->fuse_chain;
-    c->fuse_chain = 0;  // the polynomial stage by itself
-    for (int i = 0; i < 4; ++i) {
-        c->split2 = c->split3 = cand[i];
-        double t[2] = {1e300, 1e300};
-        for (int r = 0; r < reps + 1; ++r) {  // first repetition warms up
-            if (int e = mbxg_compute(c, terms, do_grads)) return e;
-            double ms[10];
-            if (int e = mbxg_get_timings(c, ms, 10)) return e;
-            if (r > 0) {
-                t[0] = std::min(t[0], ms[4]);
-                t[1] = std::min(t[1], ms[7]);
-            }
-        }
-        for (int k = 0; k < 2; ++k)
-            if (t[k] < best[k]) {
-                best[k] = t[k];
-                pick[k] = cand[i];
-            }
+namespace {
+
+// The shortest of `reps` timed computes (one more before them warms up) of each of n stages (mbxg_get_timings).
+int time_stages(mbxg_ctx* c, int terms, int do_grads, int reps, const int* stage, int n, double* best) {
+    std::fill(best, best + n, 1e300);
+    for (int r = 0; r < reps + 1; ++r) {
+        if (int e = mbxg_compute(c, terms, do_grads)) return e;
+        double ms[11];
+        if (int e = mbxg_get_timings(c, ms, 11)) return e;
+        for (int k = 0; k < n && r > 0; ++k) best[k] = std::min(best[k], ms[stage[k]]);
     }
-    c->split2 = pick[0];
-    c->split3 = pick[1];
-    c->fuse_chain = fuse_chain;
-    if ((terms & MBXG_3B) && c->cut3 > 0.0 && family_launched(c, FAM_CH4H2O2_3B)) {
-        double best3n = 1e300;
-        int pick3n = c->split3n;
+    return MBXG_OK;
+}
+
+// The fastest schedule into c->tune; what was not timed stays as it is.
+int tune_schedule(mbxg_ctx* c, int terms, int do_grads, int reps) {
+    const mbxg_ctx::Schedule was = c->tune;
+    const bool eval = !(terms & MBXG_LISTS_ONLY);
+    const bool two = eval && (terms & MBXG_2B) && c->cut2 > 0.0 && family_launched(c, FAM_MBPOL_2B);
+    const bool three = eval && (terms & MBXG_3B) && c->cut3 > 0.0 && family_launched(c, FAM_MBPOL_3B);
+    const bool paired = c->tune.fuse_poly && do_grads && two && three;
+    const int cand[4] = {1, 2, 4, 8};
+    int pick[2] = {was.split2, 0};
+    if (two || three) {
+        double best[2] = {1e300, 1e300};
+        c->tune.fuse_chain = 0;  // the polynomial stage by itself
         for (int i = 0; i < 4; ++i) {
-            c->split3n = cand[i];
-            double t = 1e300;
-            for (int r = 0; r < reps + 1; ++r) {
-                if (int e = mbxg_compute(c, terms, do_grads)) return e;
-                double ms[11];
-                if (int e = mbxg_get_timings(c, ms, 11)) return e;
-                if (r > 0) t = std::min(t, ms[10]);
-            }
-            if (t < best3n) {
-                best3n = t;
+            c->tune.split2 = c->tune.split3 = cand[i];
+            const int stage[2] = {4, 7};  // poly 2B, poly 3B
+            double t[2];
+            if (int e = time_stages(c, terms, do_grads, reps, stage, 2, t)) return e;
+            // paired, the 2B polynomial is in the 3B launch and has no time of its own
+            const bool timed[2] = {two && !paired, three};
+            for (int k = 0; k < 2; ++k)
+                if (timed[k] && t[k] < best[k]) {
+                    best[k] = t[k];
+                    pick[k] = cand[i];
+                }
+        }
+        c->tune.split2 = pick[0];
+        c->tune.split3 = three ? 0 : was.split3;
+        c->tune.tuned3 = three ? pick[1] : was.tuned3;
+        c->tune.fuse_chain = was.fuse_chain;
+    }
+    if (eval && (terms & MBXG_3B) && c->cut3 > 0.0 && family_launched(c, FAM_CH4H2O2_3B)) {
+        double best = 1e300;
+        int pick3n = c->tune.split3n;
+        for (int i = 0; i < 4; ++i) {
+            c->tune.split3n = cand[i];
+            const int stage = 10;
+            double t;
+            if (int e = time_stages(c, terms, do_grads, reps, &stage, 1, &t)) return e;
+            if (t < best) {
+                best = t;
                 pick3n = cand[i];
             }
         }
-        c->split3n = pick3n;
+        c->tune.split3n = pick3n;
     }
     // The paired path as one launch, or separate ones with the split just found and the variables of both
     // orders together or not: timed over the whole compute.
-    if (c->fuse_poly && do_grads && (terms & MBXG_2B) && (terms & MBXG_3B) && family_launched(c, FAM_MBPOL_2B) &&
-        family_launched(c, FAM_MBPOL_3B)) {
-        double bestf = 1e300;
-        int pickc = c->fuse_chain, pickv = c->fuse_vars;
+    if (paired) {
+        double best = 1e300;
+        mbxg_ctx::Schedule pick_one = c->tune;
         for (int fc = 0; fc < 2; ++fc)
             for (int fv = 0; fv < 2 - fc; ++fv) {  // (one launch has no variables of its own)
-                c->fuse_chain = fc;
-                c->fuse_vars = fv;
-                c->split3 = fc ? kFusedSplit : pick[1];
-                double t = 1e300;
-                for (int r = 0; r < reps + 1; ++r) {
-                    if (int e = mbxg_compute(c, terms, do_grads)) return e;
-                    double ms[10];
-                    if (int e = mbxg_get_timings(c, ms, 10)) return e;
-                    if (r > 0) t = std::min(t, ms[9]);
-                }
-                if (t < bestf) {
-                    bestf = t;
-                    pickc = fc;
-                    pickv = fv;
+                c->tune.fuse_chain = fc;
+                c->tune.fuse_vars = fv;
+                const int stage = 9;
+                double t;
+                if (int e = time_stages(c, terms, do_grads, reps, &stage, 1, &t)) return e;
+                if (t < best) {
+                    best = t;
+                    pick_one = c->tune;
                 }
             }
-        c->fuse_chain = pickc;
-        c->fuse_vars = pickv;
-        c->split3 = pickc ? kFusedSplit : pick[1];
+        c->tune = pick_one;
+        if (c->tune.fuse_chain) c->tune.tuned3 = 0;  // the pair's split is not in use then
     }
-    if (int r = mbxg_set_timing(c, was_timing ? 1 : 0)) return r;
-    return mbxg_compute(c, terms, do_grads);
+    return MBXG_OK;
+}
+
+}  // namespace
+
+// Autotuner: time the polynomial stage of each order for every split on the current inputs
+// (HIP events, stages run one at a time), keep the fastest, then recompute once so the results
+// are those of the chosen schedule.  After an error the schedule is what it was.
+extern "C" int mbxg_autotune(mbxg_ctx* c, int terms, int do_grads, int reps) {
+    if (!c) return fail(MBXG_EINVAL, "mbxg_autotune: null context");
+    if (!c->have_coords) return fail(MBXG_ESTATE, "mbxg_autotune: coordinates not set");
+    const bool was_timing = c->timing;
+    const mbxg_ctx::Schedule was = c->tune;
+    if (int r = mbxg_set_timing(c, 1)) return r;
+    const int r = tune_schedule(c, terms, do_grads, std::max(reps, 1));
+    if (r) c->tune = was;
+    c->timing = was_timing;
+    (void)hipStreamSynchronize(c->stream);
+    drop_graph(c);  // a captured step has the former schedule
+    return r ? r : mbxg_compute(c, terms, do_grads);
 }
 
 extern "C" int mbxg_get_results(mbxg_ctx* c, double* e2b, double* e3b, double* grad, double* virial) {
