@@ -220,7 +220,8 @@ int mbxg_set_graph(mbxg_ctx* ctx, int on);
 
 /* Schedule parameters.  "split_2b" / "split_3b": wavefronts (1, 2, 4 or 8) that share each
  * block of 64 dimers / trimers in the MB-pol polynomial stage, each evaluating 1/split of the
- * polynomial (until set: by the number of n-mers); "split_ch4h2o2_3b": the same for the
+ * polynomial (0, the default: by the number of n-mers; mbxg_get_tuning then returns the number in use,
+ * for "split_3b" the one launch's four while "fuse_chain" is on); "split_ch4h2o2_3b": the same for the
  * CH4-H2O-H2O polynomial (default 4); "fuse_poly" (0 or 1, default 1): the MB-pol 2B and 3B
  * polynomials in one launch when both run with gradients; "fuse_prep" (0 or 1, default 1):
  * FixMonomerCoordinates, the cloud and the cell counts in one launch; "fuse_chain" (0 or 1,

@@ -1592,14 +1592,15 @@ namespace {
 
 bool valid_split(int v) { return v == 1 || v == 2 || v == 4 || v == 8; }
 
+bool by_rule(const std::string& key) { return key == "split_2b" || key == "split_3b"; }
 
 }  // namespace
 
 extern "C" int mbxg_set_tuning(mbxg_ctx* c, const char* key, int value) {
     if (!c || !key) return fail(MBXG_EINVAL, "mbxg_set_tuning: bad arguments");
     const std::string k(key);
-    if ((k == "split_2b" || k == "split_3b" || k == "split_ch4h2o2_3b") && !valid_split(value))
-        return fail(MBXG_EINVAL, "mbxg_set_tuning: %s must be 1, 2, 4 or 8", key);
+    if ((by_rule(k) || k == "split_ch4h2o2_3b") && !valid_split(value) && !(by_rule(k) && value == 0))
+        return fail(MBXG_EINVAL, "mbxg_set_tuning: %s must be %s1, 2, 4 or 8", key, by_rule(k) ? "0, " : "");
     if ((k == "fuse_poly" || k == "fuse_prep" || k == "fuse_chain" || k == "fuse_vars") && value != 0 && value != 1)
         return fail(MBXG_EINVAL, "mbxg_set_tuning: %s is 0 or 1", key);
     if (k == "split_2b")
@@ -1628,8 +1629,10 @@ extern "C" int mbxg_get_tuning(mbxg_ctx* c, const char* key, int* value) {
     const std::string k(key);
     if (k == "split_2b")
         *value = split_of(c->tune.split2, fam_cap(c->L, FAM_MBPOL_2B), 31);
-    else if (k == "split_3b")
-        *value = split_3b(c, fam_cap(c->L, FAM_MBPOL_3B));
+    else if (k == "split_3b")  // unless set or tuned, the one launch's, which most computes take
+        *value = !c->tune.split3 && !c->tune.tuned3 && c->tune.fuse_poly && c->tune.fuse_chain
+                     ? kFusedSplit
+                     : split_3b(c, fam_cap(c->L, FAM_MBPOL_3B));
     else if (k == "split_ch4h2o2_3b")
         *value = split_of(c->tune.split3n, fam_cap(c->L, FAM_CH4H2O2_3B), 55);
     else if (k == "fuse_poly")

@@ -77,6 +77,25 @@ def test_autotune_error_restores(systems):
         e.timings()
 
 
+def test_back_to_the_rule(systems):
+    """0 gives a split back to the rule; what tuning() returns by default can be set without a change of route."""
+    e = _water(systems)
+    e.compute()
+    default = {k: e.tuning(k) for k in ("split_2b", "split_3b")}
+    for k in default:
+        e.set_tuning(k, 1)
+        assert e.tuning(k) == 1
+        e.set_tuning(k, 0)
+        assert e.tuning(k) == default[k]
+    e.set_tuning("fuse_chain", 0)
+    separate = _separate_ms(e)
+    e.set_tuning("fuse_chain", 1)
+    e.set_tuning("split_3b", default["split_3b"])
+    assert _separate_ms(e) < 0.5 * separate
+    with pytest.raises(engine.MbxgError):
+        e.set_tuning("split_ch4h2o2_3b", 0)
+
+
 def test_autotuned_schedule_is_replayed(systems):
     """A step captured before the autotuner ran is captured again: same results as an eager compute of the
     schedule found."""
