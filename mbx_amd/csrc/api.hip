@@ -926,7 +926,7 @@ int prepare_layout(mbxg_ctx* c, double cut) {
     }
     if (L.d_grids.reserve(nconf) || L.d_cell_base.reserve(nconf) || L.d_cell_bound.reserve(nconf) ||
         L.cell_count.reserve(total) || L.cell_start.reserve(total + 1) ||
-        L.cell_sums.reserve((total + kCellChunk - 1) / kCellChunk))
+        (total > kCellsOneBlock && L.cell_sums.reserve((total + kCellChunk - 1) / kCellChunk)))
         return fail(MBXG_ENOMEM, "cell layout: device allocation failed");
     hipStream_t st = c->stream;
     launch_zero_int(L.cell_count.p, total, st);  // every scan leaves the counts zero again
@@ -963,7 +963,7 @@ int build_lists(mbxg_ctx* c, const NmerCtx& N, double c2sq, double c3sq, double 
         L.counts.reserve(np) || L.wpre.reserve((size_t)np * kQueryWaves) || L.wpre_x.reserve((size_t)np * kQueryWaves) ||
         L.offsets.reserve(np + 1) || L.counts_x.reserve(np) || L.offsets_x.reserve(np + 1) ||
         L.wmax.reserve(np) || L.wmax_x.reserve(np) || L.maxw.reserve(2) ||
-        L.shares.reserve((np + kScanChunk - 1) / kScanChunk))
+        (np > kScanOneBlock && L.shares.reserve((np + kScanChunk - 1) / kScanChunk)))
         return fail(MBXG_ENOMEM, "list buffers: device allocation failed");
     const int tb = 256, pb = (np + tb - 1) / tb, sb = (ns + tb - 1) / tb;
     // the gas-phase grids read the input coordinates (the working copy equals them there)
