@@ -1466,16 +1466,25 @@ int finish(mbxg_ctx* c) {
 
 // A per-atom device array (3 * natoms doubles) into host memory `out`: the copy goes to pinned memory and
 // is on the stream before the wait, so there is one wait and no staging by the runtime.  A result of the
-// last compute is checked (finish()) and read again if that computed again.
+// last compute is checked (finish()) and read again if that computed again.  Where the host has no pinned
+// memory left for the array the runtime stages it.
 int read_atoms(mbxg_ctx* c, const double* src, double* out, bool result) {
     const size_t n = 3 * (size_t)c->natoms;
     if (n > c->host_atoms_n) {
         if (c->host_atoms) HIPCHK(hipHostFree(c->host_atoms));
         c->host_atoms = nullptr;
         c->host_atoms_n = 0;
-        if (hipHostMalloc((void**)&c->host_atoms, n * sizeof(double), hipHostMallocDefault) != hipSuccess)
-            return fail(MBXG_ENOMEM, "results: pinned host allocation failed");
-        c->host_atoms_n = n;
+        if (hipHostMalloc((void**)&c->host_atoms, n * sizeof(double), hipHostMallocDefault) == hipSuccess) {
+            c->host_atoms_n = n;
+        } else {
+            (void)hipGetLastError();
+            c->host_atoms = nullptr;
+            if (result)
+                if (int r = finish(c)) return r;
+            HIPCHK(hipMemcpyAsync(out, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(hipStreamSynchronize(c->stream));
+            return MBXG_OK;
+        }
     }
     for (int turn = 0; turn < 2; ++turn) {
         HIPCHK(hipMemcpyAsync(c->host_atoms, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
