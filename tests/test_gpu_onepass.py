@@ -65,10 +65,10 @@ def test_one_pass_equals_two_pass(graph):
 
 
 def test_paired_polynomials_match_separate_launches():
-    """The MB-pol 3B and 2B polynomials in one launch (fuse_poly = 1, the default) against
-    separate launches: the same per-n-mer schedules, so energies and gradients agree to rounding
-    (the 2B parts are summed over split_3b wavefronts instead of split_2b: gradients of
-    cancelling terms differ by a few 1e-10); both meet the oracle's bar."""
+    """MB-pol's 3B and 2B polynomials in one launch (fuse_poly = 1, the default: the whole evaluation
+    of both) against launches of their own per order: the same per-n-mer schedules, so energies and
+    gradients agree to rounding (the pieces are summed over four wavefronts instead of the size rule's:
+    gradients of cancelling terms differ by a few 1e-10); both meet the oracle's bar."""
     xyz, box, c2, c3 = configs.build(configs.C1)
     out = {}
     for fuse in (1, 0):
@@ -130,34 +130,43 @@ def test_fused_prep_matches_separate_launches(systems, case):
 
 @pytest.mark.parametrize("split", [1, 2, 4, 8])
 def test_fused_chain_matches_separate_kernel(systems, split):
-    """The MB-pol 3B chain rule in the paired polynomial launch's 3B blocks (fuse_chain = 1, the
-    default) against its own kernel (fuse_chain = 0), for every split of the 64-trimer blocks:
-    bit-identical energies (the same per-trimer arithmetic and the same records of 64 trimers),
-    gradients and virial to the rounding of the atomics' order.  Eager and graph replays; and the
-    oracle's energies and gradients."""
+    """MB-pol's variables, polynomials and chain rules of both orders in one launch (fuse_chain = 1 and
+    the split by default, four wavefronts per 64 n-mers) against launches of their own (fuse_chain = 0) at
+    every split of theirs: bit-identical energies (the same arithmetic, the pieces' values added in one
+    order for every split, the same records of 64 n-mers), gradients and virial to the rounding of the
+    atomics' order, and at the other splits of the pieces' order too (the tolerance of
+    test_paired_polynomials_match_separate_launches); and each schedule against the oracle's energies and
+    gradients.  Eager and graph replays."""
     from conftest import water_case
 
     xyz, box, c2, c3, _ = water_case(systems, "h2o_2048_cubic")
     kinds = [engine.H2O] * (len(xyz) // 9)
     out = {}
     for fuse in (1, 0):
-        print("fuse_chain", fuse, "split", split, flush=True)
+        print("fuse_chain", fuse, "separate launches' split", split, flush=True)
         e = engine.Engine()
         e.set_topology(kinds)
         e.set_box(box)
         e.set_cutoffs(c2, c3)
-        e.set_tuning("split_2b", split)
-        e.set_tuning("split_3b", split)
         e.set_tuning("fuse_chain", fuse)
         assert e.tuning("fuse_chain") == fuse
+        if not fuse:
+            e.set_tuning("split_2b", split)
+            e.set_tuning("split_3b", split)
         e.set_graph(True)
         e.set_coords(xyz)
         for _ in range(3):  # sizing compute, eager, graph replay
             e.compute()
         out[fuse] = _state(e)
-    _same(out[1], out[0])
     if split == 4:
-        r = oracle.water_system(xyz, box, c2, c3)
-        e2, e3, g, _ = out[1][:4]
+        _same(out[1], out[0])
+    else:
+        assert out[1][:2] == out[0][:2]
+        np.testing.assert_allclose(out[1][2], out[0][2], rtol=0, atol=5e-9)
+        np.testing.assert_allclose(out[1][3], out[0][3], rtol=1e-10, atol=1e-8)
+        assert np.array_equal(out[1][4], out[0][4]) and np.array_equal(out[1][5], out[0][5])
+    r = oracle.water_system(xyz, box, c2, c3)
+    for fuse in (1, 0):
+        e2, e3, g, _ = out[fuse][:4]
         assert e2 == pytest.approx(r["e2b"], rel=1e-10) and e3 == pytest.approx(r["e3b"], rel=1e-10)
         assert np.abs(g - r["grad"]).max() <= 1e-8
