@@ -259,7 +259,6 @@ struct mbxg_ctx {
     DBuf<double> d_coef;                // every coefficient table; the views below point into it
     CoefView d_coef2, d_coef3;
     CoefView d_coefn[kFamilies];      // MB-nrg coefficient tables (families 1, 2, 4)
-    DBuf<double> d_fam_tot;           // per family: energy + 6 virial components
     DBuf<Box> d_box;
     // configurations (mbxg_set_batch): monomers [mon_off[c], mon_off[c+1]) form configuration c;
     // its cloud points are [pt_off[c], pt_off[c+1])
@@ -370,7 +369,7 @@ extern "C" int mbxg_create(mbxg_ctx** out, int device) {
     const DefaultCoefficients& D = default_coefficients();
     // totals: 2B record, 3B record, 1B record, 4B record (kPartials each)
     if (c->d_coef.reserve(D.data.size()) || c->d_xfam_tot.reserve(kXFam * kPartials) ||
-        c->d_totals.reserve(4 * kPartials) || c->d_box.reserve(1) || c->d_fam_tot.reserve(kFamilies * kPartials)) {
+        c->d_totals.reserve(4 * kPartials) || c->d_box.reserve(1)) {
         (void)hipHostFree(c->host);
         delete c;
         return fail(MBXG_ENOMEM, "mbxg_create: device allocation failed");
@@ -421,7 +420,6 @@ extern "C" int mbxg_destroy(mbxg_ctx* c) {
     c->d_pt_off.release();
     c->d_conf_tot.release();
     c->d_conf_part.release();
-    c->d_fam_tot.release();
     for (DBuf<int>& b : c->x_list) b.release();
     for (EvalState* o = c->xf; o != c->xf + kXFam; ++o) {
         o->e_nmer.release();
@@ -825,11 +823,6 @@ int with_headroom(int n) { return n + n / 4 + 64; }
 void launch_zero_int(int* p, size_t n, hipStream_t st) {
     const int nb = (int)std::min<size_t>((n + 255) / 256, 1024);
     hipLaunchKernelGGL(k_zero_int, dim3(nb > 0 ? nb : 1), dim3(256), 0, st, p, n);
-}
-
-void launch_zero(double* p, size_t n, hipStream_t st) {
-    const int nb = (int)std::min<size_t>((n + 255) / 256, 1024);
-    hipLaunchKernelGGL(k_zero, dim3(nb > 0 ? nb : 1), dim3(256), 0, st, p, n);
 }
 
 // Dimer and trimer lists at the larger cutoff (one gather for both orders).  With sync the
@@ -1240,7 +1233,8 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
                            c->d_first.p, c->d_nat.p, c->nmon, c->box);
         HIPCHK(hipGetLastError());
     }
-    // the gradient and the 1B record when no 1B term runs start at zero: zeroed by the list build's first kernel, or by one launch of their own
+    // the gradient and the 1B record when no 1B term runs start at zero: zeroed by the list build's first
+    // kernel, or by one launch of their own
     c->one_body_last = (terms & MBXG_1B) && !(terms & MBXG_LISTS_ONLY);
     const bool batch = c->nconf > 1;
     ZeroJobs Z{};
@@ -1406,8 +1400,7 @@ int run(mbxg_ctx* c, int terms, int do_grads, bool sync) {
     }
     // per-order totals: 2B = MB-pol + CH4-H2O + CH4-CH4, 3B = MB-pol + CH4-H2O-H2O (fixed order)
     if (!batch) {
-        hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinishThreads), 0, st, J, c->d_fam_tot.p, c->d_totals.p,
-                           publish_job(c));
+        hipLaunchKernelGGL(k_finish, dim3(1), dim3(kFinishThreads), 0, st, J, c->d_totals.p, publish_job(c));
     } else {
         const int nc = c->nconf;
         hipLaunchKernelGGL(k_reduce_configs, dim3(nc, slices, kFamilies), dim3(256), 0, st, CJ, c->d_pt_off.p,

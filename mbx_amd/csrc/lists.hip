@@ -429,7 +429,8 @@ struct Lds {
     double* iz;
     double* r;  // |query first atom - imaged partner first atom|
     double* p3;  // the matches inside the 3B cutoff packed in m3 order, kP3Doubles each: sx sy sz
-                 // ix iy iz r, then int4 {mon, tag, kind, 0} at double 8 (five 16-byte reads)
+                 // ix iy iz r 0, then int4 {mon, query's tag < its tag, species, 0} at double 8 (five
+                 // 16-byte reads)
 };
 
 // 7 doubles + 6 ints per match, and one packed 3B entry of 10 doubles.
@@ -1229,7 +1230,7 @@ __global__ void __launch_bounds__(64 * 2 * kPartials) k_sum_configs(const double
     publish(P, totals);
 }
 
-__global__ void __launch_bounds__(kFinishThreads) k_finish(FinishJobs J, double* __restrict__ fam, double* totals, PublishJob P) {
+__global__ void __launch_bounds__(kFinishThreads) k_finish(FinishJobs J, double* totals, PublishJob P) {
     __shared__ double sh[kPartials][kFinishThreads];
     __shared__ double res[kFamilies][kPartials];
     const int t = threadIdx.x;
@@ -1257,7 +1258,6 @@ __global__ void __launch_bounds__(kFinishThreads) k_finish(FinishJobs J, double*
     }
     __syncthreads();
     if (t < kPartials) {
-        for (int f = 0; f < kFamilies; ++f) fam[f * kPartials + t] = res[f][t];
         totals[t] = res[FAM_MBPOL_2B][t] + res[FAM_CH4H2O_2B][t] + res[FAM_CH4CH4_2B][t];
         totals[kPartials + t] = res[FAM_MBPOL_3B][t] + res[FAM_CH4H2O2_3B][t];
         totals[3 * kPartials + t] = 0.0;

@@ -130,8 +130,7 @@ struct NmersArgs {
     int4* wmax_x;
 };
 
-// out[0] / out[1] = componentwise maxima of wmax[0..n) / wmax_x[0..n) (one workgroup).
-// The per-(query, wavefront) maxima of wmax / wmax_x into maxw[0..1] (skipped with wmax null) and
+// One workgroup: the per-(query, wavefront) maxima of wmax / wmax_x into maxw[0..1] (skipped with wmax null) and
 // the exclusive scans of counts and counts_x (.w maximised), totals at n, in one launch.
 __global__ void k_scan_all(const int4* wmax, const int4* wmax_x, int4* maxw, const int4* counts, int4* offsets,
                            const int4* counts_x, int4* offsets_x, int n);
@@ -155,10 +154,9 @@ struct FinishJobs {
     const int* n_dev[kFamilies];
     int cap[kFamilies];
 };
-// One workgroup of kFinishThreads: each family's partial records summed in a fixed order into fam
-// (kPartials per family, zeros for the families not evaluated), then the per-order records of
-// totals (2B = MB-pol + CH4-H2O + CH4-CH4, 3B = MB-pol + CH4-H2O-H2O) and the 4B record zeroed.  (The 1B
-// record is a launch of its own before.)
+// One workgroup of kFinishThreads: each family's partial records summed in a fixed order (zeros for the
+// families not evaluated), then the per-order records of totals (2B = MB-pol + CH4-H2O + CH4-CH4, 3B =
+// MB-pol + CH4-H2O-H2O) and the 4B record zeroed.  (The 1B record is a launch of its own before.)
 // The last kernel of a compute also publishes what the host reads after every step (the totals and the
 // list builder's counts and maxima) into pinned host memory, so that waiting for the stream is all the
 // host does: three copies of a few bytes each cost 40 us a step.
@@ -171,7 +169,7 @@ struct PublishJob {
     const int4 *tot, *totx, *maxw;  // tot null: no lists were built
 };
 constexpr int kFinishThreads = 512;
-__global__ void k_finish(FinishJobs J, double* fam, double* totals, PublishJob P);
+__global__ void k_finish(FinishJobs J, double* totals, PublishJob P);
 
 // By one workgroup, after its threads have written (and __syncthreads() has ordered) totals.
 __device__ __forceinline__ void publish(const PublishJob& P, const double* totals) {
@@ -250,8 +248,9 @@ hipError_t launch_poly_mbpol_pair(double* ws3, const int* n3_dev, int cap3, cons
 // launch_mbpol3b_vars and launch_mbpol2b_vars as one launch (workspaces as theirs).
 hipError_t launch_mbpol_vars_pair(const int* list3, const int* n3_dev, int cap3, double* ws3, const int* list2,
                                   const int* n2_dev, int cap2, double* ws2, const NmerCtx& N, hipStream_t st);
-// Both orders' whole evaluation with gradients in one launch (mbpol_fused.hip): energies e_out, gradient added to grad, virials vir_out (nullable, leading dimension ld),
-// one partial record per 64 n-mers.  cap 0: that order is left out (n_dev is not read).
+// Both orders' whole evaluation with gradients in one launch (mbpol_fused.hip): energies e_out, gradient
+// added to grad, virials vir_out (nullable, leading dimension ld), one partial record per 64 n-mers.  cap 0:
+// that order is left out (n_dev is not read).
 constexpr int kFusedSplit = 4;  // wavefronts per 64 n-mers
 struct FusedJob {
     const int* list;
