@@ -272,14 +272,16 @@ hipError_t launch_nrg_family(int family, const int* list, const int* n_dev, int 
 // Wavefronts per 64 n-mers for a polynomial kernel of `wpe` wavefronts per SIMD, from the n-mers'
 // capacity.  Few groups of 64 leave the chip idle, so each is cut into more and shorter wavefronts; the
 // cut costs a reduction and variables loaded again, so it stops once the chip is full.  Measured on
-// the MB-pol pair with its 3B chain rule (wpe 3; us at split 2 / 4 / 8): 1 group 51 / 37 / 35, 24
-// groups 53 / 39 / 37, 260 61 / 55 / 59, 705 82 / 72 / 88, 1055 95 / 94 / 124, 1742 124 / 123 / 174,
-// 3465 198 / 212 / 322, 10562 539 / 606 / 994 (split 1: 67-80% slower below 1000, 545 at 10562).
+// MB-pol's polynomials as launches of their own (wpe 3; us at split 1 / 2 / 4 / 8).  3B, value and gradient: 72
+// groups 66 / 41 / 26 / 25, 261 70 / 44 / 35 / 46, 1065 102 / 79 / 69 / 104, 2352 144 / 118 / 119 / 194, 3987
+// 196 / 178 / 183 / 306, 11269 490 / 477 / 494 / 872; values alone: 72 46 / 28 / 18 / 14, 1065 65 / 44 / 40 / 39,
+// 2352 84 / 75 / 65 / 69, 7286 181 / 162 / 162 / 180.  2B, value and gradient: 78 27 / 19 / 14 / 13, 518
+// 37 / 28 / 24 / 34, 1711 49 / 46 / 43 / 68, 2657 63 / 61 / 60 / 102.
 // poly_wpe: wavefronts per SIMD of a value + gradient kernel of nv variables (the generator's rule).
 constexpr int poly_wpe(int nv) { return 512 / (4 * nv + 24) > 4 ? 4 : 512 / (4 * nv + 24) > 1 ? 512 / (4 * nv + 24) : 1; }
 inline int poly_split(int cap, int wpe) {
     const int groups = (cap + 63) / 64;
-    return groups <= 128 ? 8 : groups <= 400 * wpe ? 4 : 2;
+    return groups <= 128 ? 8 : groups <= 800 * wpe ? 4 : 2;
 }
 
 // Polynomial stage alone: xs/gs variable-major with leading dimension ld (= cap rounded up
