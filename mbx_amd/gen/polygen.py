@@ -764,7 +764,10 @@ def generate_ad(name, out_dir):
     body.insert(0, symmetry.emit_transform("%s_tan_sym" % fn, sym.blocks))
     d = ["__device__ __forceinline__ void %s_tan(int part, mbxg_cptr C, const double* x, const double* xd, "
          "double* gd) {" % fn]
-    d += ["    if (part == %d) %s_tan_%s%d(C, x, xd, gd);" % (k, fn, w, k) for w, k, _, _ in pieces]
+    for phase in "rp":
+        if phase == "p" and pieces[0][0] == "r":  # as in blocked_source
+            d += ["    mbxg_opaque<%d>(x);" % nvars, "    mbxg_opaque<%d>(xd);" % nvars]
+        d += ["    if (part == %d) %s_tan_%s%d(C, x, xd, gd);" % (k, fn, w, k) for w, k, _, _ in pieces if w == phase]
     d += ["}", "", "}  // namespace mbxg", ""]
     write_if_changed(os.path.join(out_dir, "ad_%s_tan.inc" % name),
                      "\n".join(head("Gradient tangent of the polynomial (H xd) in %d parts." % AD_PARTS))
