@@ -13,7 +13,7 @@ The JSON line also carries
                 and 2B; the paired polynomials when fuse_chain is off; the 3B one alone when the
                 pairing is off) against the MI355X FP64 vector unit's operations (an FMA is one:
                 39.3 T/s).  Counted are the FP64 operations that the polynomials execute per
-                evaluated trimer (17,106) and dimer (6,541), from their generated sources: in
+                evaluated trimer (19,955) and dimer (7,231), from their generated sources: in
                 symmetry-adapted coordinates a quarter of the reference's multiplies and adds
                 (81,549 and 27,208), which would give more than the peak.  Timed with HIP events
                 on the engine stream in a stage-timing pass of the same workload; traffic from the

@@ -10,13 +10,15 @@
 // an exponential needs only y_j = x_j dP/dx_j; then each of the first
 // wavefronts gathers one monomer's gradient and scatters it while the last one has done the switch, energy
 // and virial.  With the polynomial down to 20.0k operations a trimer (poly_kernel.hpp) the stages around it
-// cost as much as it does as launches of their own: the variables 25 us at 2048 waters, the 2B chain rule
-// 18, the 3B chain rule on one wavefront of a block, reading variables and gradient back from memory in nine
-// dependent groups, 50.  Nothing of an n-mer but its energy goes through memory here.
+// count: as launches of their own the variables take 27 us at 2048 waters, the 2B chain rule 20, the 3B chain
+// rule 35, the polynomials 132.  Nothing of an n-mer but its energy goes through memory here.  This launch
+// against those four, us: 6 waters 32 / 62, 256 waters 48 / 84, 617 waters 77 / 112, 2048 waters 192 / 214, 6859
+// waters 548 / 521 (the registers of all stages in one kernel spill some 340 B a lane).
 //
 // Four is fixed, for every size: the gradient's order of summation and with it the results do not depend on
-// how many n-mers there are, and it is the best or close to it over the range (a first form at split
-// 1 / 2 / 4 / 8, us: 6 waters 82 / 56 / 40 / 39, 256 waters 95 / 76 / 57 / 77, 617 105 / 85 / 87 / 135).
+// how many n-mers there are, and it is the best or close to it over the range (a first form, with fewer second
+// coefficients, at split 1 / 2 / 4 / 8, us: 6 waters 82 / 56 / 40 / 39, 256 waters 95 / 76 / 57 / 77, 617
+// 105 / 85 / 87 / 135).
 //
 // Each variable is its own uniform branch, which also keeps the compiler from computing all square roots
 // and exponentials at once (some 500 registers).

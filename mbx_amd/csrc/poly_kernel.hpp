@@ -9,13 +9,13 @@
 // The polynomial is evaluated in symmetry-adapted coordinates (mbx_amd/gen/symmetry.py): sums and
 // differences of the variables that exchanges of like sites permute.  In them a fraction of the
 // monomials survives (MB-pol 3B 6,773 of 33,525: 20.0k FP64 operations a trimer for value and
-// gradient instead of 72.5k; 2B 7.2k instead of 27.5k; CH4-H2O-H2O 14.3k instead of 63.0k; a sixth of them
-// carries what rounding the coefficients left, without which energies have an error that grows with the system), which is
-// what bounds these kernels: at full occupancy they run at 95-99% of the FP64 issue slots, alone on
+// gradient instead of 72.5k; 2B 7.2k instead of 27.5k; CH4-H2O-H2O 14.3k instead of 63.0k; a fifth of them
+// carries what rounding the coefficients left, without which energies have an error that grows with the
+// system), which is what bounds these kernels: at full occupancy they run at 95-99% of the FP64 issue slots, alone on
 // the chip at one wavefront's serial length.  The transform (SYM, in place on the registers, its own
-// transpose) costs one to three additions a variable each way.  Whole steps, before and after: 2048
-// waters 632 -> 354 us, 6859 waters 1592 -> 762 us, 32 beads of 57 CH4 + 513 H2O 4.24 -> 2.81 ms,
-// six waters 284 -> 206 us.
+// transpose) costs one to three additions a variable each way.  Whole steps, before and after with this
+// change alone (and a third of the present second coefficients): 2048 waters 632 -> 354 us, 6859 waters
+// 1592 -> 762 us, 32 beads of 57 CH4 + 513 H2O 4.24 -> 2.81 ms, six waters 284 -> 206 us.
 //
 // Layout: xs and gs are variable-major ("SoA"), entry (j, t) at j*ld + t, so a wavefront's 64
 // lanes read and write 64 consecutive doubles per variable.
