@@ -24,7 +24,8 @@ N = 16384
 
 
 @pytest.mark.parametrize("name, prefix", [("mbpol_2b", "poly_"), ("mbpol_3b", "poly_"), ("ch4h2o_2b", "poly_"),
-                                          ("alkali_h2o2_3b", "xpoly_")])
+                                          ("alkali_h2o2_3b", "xpoly_"), ("alkali_h2o_2b", "xpoly_"),
+                                          ("co2co2_2b", "xpoly_")])
 def test_no_error_that_adds_up(name, prefix, tmp_path):
     if not os.path.exists(os.path.join(GEN, "%s%s.inc" % (prefix, name))):
         pytest.skip("the untracked polynomials are generated by the build")
