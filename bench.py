@@ -47,7 +47,7 @@ HBM_PEAK = 8.0e12  # MI355X HBM3E, B/s
 
 def host_cores():
     """Threads for the CPU baseline: the cores this process may run on, capped by OMP_NUM_THREADS
-    where the environment sets it (the GPU box gives one GPU's process a 16-thread share and sets
+    where the environment sets it (a host of several GPUs gives one GPU's process a share and sets
     OMP_NUM_THREADS=16; without either, 16)."""
     try:
         n = len(os.sched_getaffinity(0))
